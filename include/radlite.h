@@ -254,8 +254,8 @@ enum {
                              (static, or persistent over a work counter) once per
                              batch shape and keep the fastest; 0: defaults */
     RL_OPT_TILE = 3,      /* fix the tile mapping (turns the autotuner off):
-                             0 = ray-major (ray, channel) pairs, 16/32/64 =
-                             channels per ray in a wave */
+                             16/32/64 = channels per ray in a wave, 0 = the
+                             default, 16 */
     RL_OPT_PERSISTENT = 4,/* with a fixed mapping: 1 (default) persistent grid
                              over the work counter, 0 static grid */
     RL_OPT_CKPT = 5       /* adjoint checkpoint interval: 0 (default) chosen

@@ -127,7 +127,7 @@ struct rl_ctx {
     // rays
     std::vector<RaySet> incl;
     // per-item work buffers
-    DevBuf d_cells, d_rec, d_rinfo, d_image, d_chan, d_partial, d_flux, d_err, d_ovs,
+    DevBuf d_cells, d_rec, d_blk, d_rinfo, d_image, d_chan, d_partial, d_flux, d_err, d_ovs,
         d_maser;
     // crossing-pass scratch, one slot per ray set of a launch: its
     // per-ray cone roots and its crossing slots; x_owner = the ray set
@@ -142,9 +142,10 @@ struct rl_ctx {
     std::vector<DevBuf> spare;
     std::vector<DevBuf> x_cnt;               // k_cross node counts per slot
     // batching
-    DevBuf d_items, d_tile0, d_counter, d_cmask;
+    DevBuf d_items, d_sel, d_tile0, d_counter, d_cmask;
     std::vector<rl::ItemDev> h_items;
     std::vector<long long> h_tile0;
+    std::vector<int> h_sel;
     size_t mem_budget = 0;            // 0: a share of the free device memory
     size_t auto_budget = 0;
     unsigned long long tick = 0;      // use counter of the ray sets
@@ -736,6 +737,7 @@ static void release_forward_work(rl_ctx *c) {
     if ((c->d_rec.n + c->d_cmask.n) * 10 > ctx_budget(c)) {
         (void)hipStreamSynchronize(c->stream);
         c->d_rec = DevBuf();
+        c->d_blk = DevBuf();
         c->d_cmask = DevBuf();
     }
 }
@@ -1125,16 +1127,21 @@ static int item_consts(rl_ctx *c, const rl_item &it, const RaySet &rs, rl::LineC
     return 0;
 }
 
-// Device bytes one item needs in a batch (node records, image, ring
+// bytes of an item's block records (rl_blocks.h)
+static size_t blk_bytes(const RaySet &rs) {
+    return (size_t)rl::blk_count(rs.nnodes, rs.nrays) * sizeof(rl::BlkRec);
+}
+
+// Device bytes one item needs in a batch (node and block records, image, ring
 // partial sums, channel tables, flux, ray info).
 static size_t item_bytes(const rl_ctx *c, const rl_item &it, const RaySet &rs) {
     const size_t rsz = c->precision == RL_FP64 ? sizeof(rl::NodeRec<double>) : sizeof(rl::NodeLine);
-    return (size_t)rs.nnodes * rsz + (size_t)rs.nrays * it.nfr * 8 +
+    return (size_t)rs.nnodes * rsz + blk_bytes(rs) + (size_t)rs.nrays * it.nfr * 8 +
            (size_t)rs.nrings * it.nfr * 8 + (size_t)it.nfr * 32 + (size_t)rs.nrays * 16 + 64;
 }
 
 static long long tiles_of(int cw, int nrays, int nfr) {
-    if (cw == 0) return ((long long)nrays * nfr + 63) / 64;
+    if (cw == 0) cw = 16;
     const int rows = 64 / cw;
     return (long long)((nrays + rows - 1) / rows) * ((nfr + cw - 1) / cw);
 }
@@ -1184,7 +1191,7 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
     size_t nchan = 0;
     for (int k = 0; k < nb; k++) nchan += 4 * (size_t)items[i0 + k].nfr;
     chan.assign(nchan, 0.0);
-    long long rec0 = 0, img0 = 0, chan0 = 0, part0 = 0, flux0 = 0;
+    long long rec0 = 0, blk0 = 0, img0 = 0, chan0 = 0, part0 = 0, flux0 = 0;
     int rinfo0 = 0, max_rays = 0, max_nfr = 0, max_rings = 0, any_skip = 0;
     for (int k = 0; k < nb; k++) {
         const rl_item &it = items[i0 + k];
@@ -1202,12 +1209,13 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
         d.geo = rs.d_nodes.as<GeoNode>();
         d.hot_off = (long long)(uintptr_t)rs.d_hot.p;     // made relative below
         d.aux_off = (long long)(uintptr_t)rs.d_aux.p;
-        d.rec0 = rec0; d.img0 = img0; d.chan0 = chan0; d.part0 = part0; d.flux0 = flux0;
+        d.rec0 = rec0; d.blk0 = blk0; d.img0 = img0; d.chan0 = chan0; d.part0 = part0; d.flux0 = flux0;
         d.rinfo0 = rinfo0;
         d.aks2 = 2.0 * (c->aksmax / 2.99792458e5);
         d.ring_w = rs.d_ringw.as<double>();
         d.center_w = rs.center_w;
-        rec0 += rs.nnodes; img0 += (long long)rs.nrays * it.nfr; chan0 += 4 * it.nfr;
+        rec0 += rs.nnodes; blk0 += rl::blk_count(rs.nnodes, rs.nrays);
+        img0 += (long long)rs.nrays * it.nfr; chan0 += 4 * it.nfr;
         part0 += (long long)rs.nrings * it.nfr; flux0 += it.nfr; rinfo0 += rs.nrays;
         max_rays = std::max(max_rays, rs.nrays);
         max_nfr = std::max(max_nfr, it.nfr);
@@ -1219,6 +1227,7 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
     }
     // device buffers
     HIPCHK(c, c->d_rec.ensure((size_t)rec0 * rsz));
+    HIPCHK(c, c->d_blk.ensure((size_t)blk0 * sizeof(rl::BlkRec)));
     HIPCHK(c, c->d_image.ensure((size_t)img0 * 8));
     HIPCHK(c, c->d_partial.ensure((size_t)part0 * 8));
     HIPCHK(c, c->d_flux.ensure((size_t)flux0 * 8));
@@ -1229,6 +1238,10 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
     HIPCHK(c, c->d_counter.ensure(8));
     HIPCHK(c, c->d_items.ensure((size_t)nb * sizeof(rl::ItemDev)));
     HIPCHK(c, c->d_tile0.ensure((size_t)(nb + 1) * 8));
+    HIPCHK(c, c->d_sel.ensure((size_t)nb * 4));
+    c->h_sel.resize(nb);
+    for (int k = 0; k < nb; k++) c->h_sel[k] = k;
+    if (int e = upload(c, c->d_sel, c->h_sel.data(), (size_t)nb * 4)) return e;
     if (cmask) HIPCHK(c, c->d_cmask.ensure((size_t)img0));
     if (int e = upload(c, c->d_chan, chan.data(), nchan * 8)) return e;
     c->cells_line = -1;       // d_cells is rewritten below for this batch's lines
@@ -1244,12 +1257,14 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
     L.items = c->d_items.as<rl::ItemDev>();
     L.cells = c->d_cells.as<CellRec>();
     L.rec = c->d_rec.p;
+    L.blk = c->d_blk.p;
     L.rinfo = c->d_rinfo.as<RayInfo>();
     L.chan = c->d_chan.as<double>();
     L.image = c->d_image.as<double>();
     L.partial = c->d_partial.as<double>();
     L.flux = c->d_flux.as<double>();
     L.d2 = (1.0 * 3.08572e18) * (1.0 * 3.08572e18);
+    L.sel = c->d_sel.as<int>();
     L.tile0 = c->d_tile0.as<long long>();
     L.ovs = c->d_ovs.as<unsigned long long>();
     L.counter = c->d_counter.as<unsigned long long>();
@@ -1309,7 +1324,7 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
             for (int gi = 0; gi < 2; gi++) {
                 zero_counters();
                 HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
-                rl::launch_batch_formal(c->stream, fp64, L, cws[ci], grids[gi], ntr);
+                rl::launch_batch_formal(c->stream, fp64, L, cws[ci] ? cws[ci] : 16, grids[gi], ntr);
                 HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
                 HIPCHK(c, hipEventSynchronize(c->ev[3]));
                 float t = 0;
@@ -1333,7 +1348,7 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
         cells();
         rl::launch_batch_nodes(c->stream, fp64, L);
         if (timed) HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
-        rl::launch_batch_formal(c->stream, fp64, L, cw, nblk, L.ntiles);
+        rl::launch_batch_formal(c->stream, fp64, L, cw ? cw : 16, nblk, L.ntiles);
         rl::launch_batch_finish(c->stream, fp64, L);
         if (timed) HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
         rl::launch_batch_flux(c->stream, L);
@@ -1345,9 +1360,9 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
     {
         char buf[64];
         auto add = [&](const void *p) { snprintf(buf, sizeof buf, ":%p", p); gkey += buf; };
-        for (const void *p : {c->d_rec.p, c->d_image.p, c->d_partial.p, c->d_flux.p,
+        for (const void *p : {c->d_rec.p, c->d_blk.p, c->d_image.p, c->d_partial.p, c->d_flux.p,
                               c->d_rinfo.p, c->d_cells.p, c->d_ovs.p, c->d_maser.p,
-                              c->d_counter.p, c->d_items.p, c->d_tile0.p, c->d_chan.p,
+                              c->d_counter.p, c->d_items.p, c->d_sel.p, c->d_tile0.p, c->d_chan.p,
                               (void *)L.cmask,
                               c->d_rho.p, c->d_abund.p, c->d_lw.p, c->d_pops.p, c->d_jd.p,
                               c->d_ad.p})
@@ -1572,7 +1587,7 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
         nchan += 4 * (size_t)it.nfr;
     }
     std::vector<double> chan(nchan, 0.0);
-    long long rec0 = 0, img0 = 0, chan0 = 0, part0 = 0, flux0 = 0;
+    long long rec0 = 0, blk0 = 0, img0 = 0, chan0 = 0, part0 = 0, flux0 = 0;
     int rinfo0 = 0, max_rays = 0, max_nfr = 0, max_rings = 0, any_skip = 0;
     for (int k = 0; k < nb; k++) {
         const rl_item &it = items[k];
@@ -1589,12 +1604,13 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
         d.geo = rs.d_nodes.as<GeoNode>();
         d.hot_off = (long long)(uintptr_t)rs.d_hot.p;     // made relative below
         d.aux_off = (long long)(uintptr_t)rs.d_aux.p;
-        d.rec0 = rec0; d.img0 = img0; d.chan0 = chan0; d.part0 = part0; d.flux0 = flux0;
+        d.rec0 = rec0; d.blk0 = blk0; d.img0 = img0; d.chan0 = chan0; d.part0 = part0; d.flux0 = flux0;
         d.rinfo0 = rinfo0;
         d.aks2 = 2.0 * (c->aksmax / 2.99792458e5);
         d.ring_w = rs.d_ringw.as<double>();
         d.center_w = rs.center_w;
-        rec0 += rs.nnodes; img0 += (long long)rs.nrays * it.nfr; chan0 += 4 * it.nfr;
+        rec0 += rs.nnodes; blk0 += rl::blk_count(rs.nnodes, rs.nrays);
+        img0 += (long long)rs.nrays * it.nfr; chan0 += 4 * it.nfr;
         part0 += (long long)rs.nrings * it.nfr; flux0 += it.nfr; rinfo0 += rs.nrays;
         max_rays = std::max(max_rays, rs.nrays);
         max_nfr = std::max(max_nfr, it.nfr);
@@ -1638,6 +1654,12 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
     const size_t o_counter = carve(8);
     const size_t o_items = carve((size_t)nb * sizeof(rl::ItemDev));
     const size_t o_tile0 = carve((size_t)(nb + 1) * 8);
+    const size_t o_sel = carve((size_t)nb * 4);
+    // the block records where they still fit; without them every segment is
+    // integrated
+    const size_t bbytes = (size_t)blk0 * sizeof(rl::BlkRec);
+    const bool with_blk = used + bbytes <= rl::SCRATCH_BYTES;
+    const size_t o_blk = with_blk ? carve(bbytes) : 0;
     if (used > rl::SCRATCH_BYTES)
         return fail(c, 13,
                     "rl_trace_lines_forward_noalloc: the items need %zu bytes of workspace, "
@@ -1654,6 +1676,7 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
     L.items = reinterpret_cast<const rl::ItemDev *>(ws + o_items);
     L.cells = reinterpret_cast<const CellRec *>(ws + o_cells);
     L.rec = ws + o_rec;
+    L.blk = with_blk ? ws + o_blk : nullptr;
     L.rinfo = reinterpret_cast<RayInfo *>(ws + o_rinfo);
     L.chan = reinterpret_cast<const double *>(ws + o_chan);
     L.image = image_dev ? image_dev : reinterpret_cast<double *>(ws + o_img);
@@ -1662,6 +1685,7 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
     L.cmask = nullptr;
     L.d2 = (1.0 * 3.08572e18) * (1.0 * 3.08572e18);
     L.tile0 = reinterpret_cast<const long long *>(ws + o_tile0);
+    L.sel = reinterpret_cast<const int *>(ws + o_sel);
     L.ntiles = t0[nb];
     L.ovs = reinterpret_cast<unsigned long long *>(ws + o_ovs);
     L.maser = reinterpret_cast<int *>(ws + o_maser);
@@ -1674,6 +1698,10 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
                              hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(ws + o_tile0, t0.data(), (size_t)(nb + 1) * 8,
                              hipMemcpyHostToDevice, c->stream));
+    std::vector<int> sel(nb);
+    for (int k = 0; k < nb; k++) sel[k] = k;
+    HIPCHK(c, hipMemcpyAsync(ws + o_sel, sel.data(), (size_t)nb * 4, hipMemcpyHostToDevice,
+                             c->stream));
     rl::launch_zero_u64(c->stream, L.ovs, nb);
     rl::launch_zero_u64(c->stream, reinterpret_cast<unsigned long long *>(L.maser), (nb + 1) / 2);
     for (size_t q = 0; q < slot_line.size(); q++) {
@@ -1688,7 +1716,7 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
     HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
     rl::launch_batch_nodes(c->stream, fp64, L);
     HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
-    rl::launch_batch_formal(c->stream, fp64, L, cw, nblk, L.ntiles);
+    rl::launch_batch_formal(c->stream, fp64, L, cw ? cw : 16, nblk, L.ntiles);
     rl::launch_batch_finish(c->stream, fp64, L);
     HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
     rl::launch_batch_flux(c->stream, L);

@@ -116,13 +116,13 @@ __device__ inline T voigt(const LineK<T> &L, T aks, T dnu) {
     return norm * dexp<T>(-(u * u));
 }
 
-// qdr_src_2, transfer.F:1498-1571 -- I <- I*xp + min(Q, theomax)
+// qdr_src_2, transfer.F:1498-1571 -- the map I <- I*xp + q, q = min(Q, theomax)
 template <typename T>
-__device__ inline T qdr(T I, T js1, T alp1, T js2, T alp2, T ds, int &ovs, T &S0,
-                        bool have_s0) {
+__device__ inline void qdr_map(T js1, T alp1, T js2, T alp2, T ds, int &ovs, T &S0, bool have_s0,
+                               T &xp, T &q) {
     T dtau1 = T(0.5) * (alp1 + alp2) * ds;
     T theomax = T(0.5) * (js1 + js2) * ds;
-    T a, b, xp;
+    T a, b;
     if (dtau1 > T(1.0e-6)) {
         xp = dexp<T>(-dtau1);
         T e0 = T(1) - xp;
@@ -141,17 +141,24 @@ __device__ inline T qdr(T I, T js1, T alp1, T js2, T alp2, T ds, int &ovs, T &S0
     T src1 = alp1 > T(0) ? q1 : (alp2 > T(0) ? q2 : T(0));
     T src2 = alp2 > T(0) ? q2 : (alp1 > T(0) ? q1 : T(0));
     S0 = q2;
-    T q;
     if (dtau1 > T((double)1e-9f)) q = a * src1 + b * src2;   // 1e-9 is REAL*4
     else q = T(0.5) * (js1 + js2) * ds;
     if (q > T(2) * theomax) ovs++;
     q = q < theomax ? q : theomax;
-    return I * xp + q;
 }
+// What a lane carries along its ray: the intensity, or (AFF) the map I -> P I
+// + I' of the part of the ray it has passed.
+template <typename T, bool AFF> struct Acc {
+    T I, P;
+    __device__ void map(T xp, T q) {
+        I = I * xp + q;
+        if (AFF) P = P * xp;
+    }
+};
 
 // integrate_element_linedust, line.F:4515-4624
-template <typename T>
-__device__ inline void integ_elem(const LineK<T> &L, T &I, T ds,
+template <typename T, bool AFF>
+__device__ inline void integ_elem(const LineK<T> &L, Acc<T, AFF> &x, T ds,
                                   const Pt<T> &p0, const Pt<T> &p1,
                                   T lw0, T lw1, Carry<T> &c, int &ovs) {
     T lwav = T(0.5) * (lw0 + lw1);
@@ -168,7 +175,9 @@ __device__ inline void integ_elem(const LineK<T> &L, T &I, T ds,
     T src0 = p0.srcd + c.srcl0, src1 = p1.srcd + srcl1;
     T alp0 = p0.alpd + c.alpl0, alp1 = p1.alpd + alpl1;
     const bool have = c.init == 0;
-    I = qdr<T>(I, src0, alp0, src1, alp1, ds, ovs, c.S0, have);
+    T xp, q;
+    qdr_map<T>(src0, alp0, src1, alp1, ds, ovs, c.S0, have, xp, q);
+    x.map(xp, q);
     c.tau = c.tau + T(0.5) * (alp0 + alp1) * ds;               // line.F:4598
     c.phi0 = phi1;
     c.srcl0 = srcl1;
@@ -178,8 +187,8 @@ __device__ inline void integ_elem(const LineK<T> &L, T &I, T ds,
 
 // clever_integrate_element_linedust, line.F:4636-4848 (SUBGRID on):
 // sub-points are generated on the fly instead of stored.
-template <typename T>
-__device__ inline void clever_elem(const LineK<T> &L, T &I, T ds,
+template <typename T, bool AFF>
+__device__ inline void clever_elem(const LineK<T> &L, Acc<T, AFF> &acc, T ds,
                                    const Pt<T> &p0, const Pt<T> &p1,
                                    T lw0, T lw1, Carry<T> &c, int &ovs) {
     const T crit = T(3.0);
@@ -215,14 +224,14 @@ __device__ inline void clever_elem(const LineK<T> &L, T &I, T ds,
                     b.u = ep * p0.u + e * p1.u;
                     b.srcd = ep * p0.srcd + e * p1.srcd;
                     b.alpd = ep * p0.alpd + e * p1.alpd;
-                    integ_elem<T>(L, I, s - sa, a, b, lw, lw, c, ovs);
+                    integ_elem<T>(L, acc, s - sa, a, b, lw, lw, c, ovs);
                     a = b;
                     sa = s;
                 }
             }
         }
     }
-    integ_elem<T>(L, I, ds - sa, a, p1, lwa, lwb, c, ovs);
+    integ_elem<T>(L, acc, ds - sa, a, p1, lwa, lwb, c, ovs);
 }
 
 // ---------------------------------------------------------------------
@@ -289,9 +298,16 @@ template <> struct FOps<double> {
 };
 
 // qdr_src_2 weights: I_out = I*xp + a*S1 + b*S2.  ra = a/x (needed by the
-// adjoint: db/dx = a/x, da/dx = xp - a/x).
+// adjoint: db/dx = a/x, da/dx = xp - a/x).  e0 = 1 - xp.
+template <typename T>
+__device__ inline void qdr_weights_f(T x, T &a, T &b, T &xp, T &ra, T &e0);
 template <typename T>
 __device__ inline void qdr_weights_f(T x, T &a, T &b, T &xp, T &ra) {
+    T e0;
+    qdr_weights_f<T>(x, a, b, xp, ra, e0);
+}
+template <typename T>
+__device__ inline void qdr_weights_f(T x, T &a, T &b, T &xp, T &ra, T &e0) {
     // single precision: the series also covers dtau <= 1e-6, where it and
     // the thin-element weights (a = b = dtau/2, xp = 1 - dtau) agree to
     // O(dtau^2), below float resolution; one branch fewer per element
@@ -318,13 +334,13 @@ __device__ inline void qdr_weights_f(T x, T &a, T &b, T &xp, T &ra) {
                     x * (T(1) / 479001600 - x * (T(1) / 6227020800.0 -
                     x * (T(1) / 87178291200.0 - x * (T(1) / 1307674368000.0)))))))))))));
             b = x * p;
-            T e0 = x * (T(1) - b);
+            e0 = x * (T(1) - b);
             xp = T(1) - e0;
             a = e0 - b;
             ra = T(1) - b - p;
         } else {
             xp = FOps<T>::ex(-x);
-            T e0 = T(1) - xp;
+            e0 = T(1) - xp;
             b = FOps<T>::fdiv(x - e0, x);
             a = e0 - b;
             ra = FOps<T>::fdiv(a, x);
@@ -333,6 +349,7 @@ __device__ inline void qdr_weights_f(T x, T &a, T &b, T &xp, T &ra) {
         a = T(0.5) * x;
         b = T(0.5) * x;
         xp = T(1) - x;
+        e0 = x;
         ra = T(0.5);
     }
 }
@@ -540,5 +557,43 @@ template <typename T>
 struct alignas(sizeof(T) * 8) NodeRec {
     T ds, u, jd, ad, lw, nu, nl, flag;
 };
+
+template <typename T> __device__ inline Pt<T> pt_of(const NodeRec<T> &a) {
+    return Pt<T>{a.jd, a.ad, a.u, a.nu, a.nl};
+}
+
+// the carry of a node a as the end of the segment before it (p: that
+// segment's start node, whose width the profile takes)
+template <typename T>
+__device__ inline void carry_of(const LineK<T> &L, const NodeRec<T> &p, const NodeRec<T> &a,
+                                Carry<T> &c) {
+    c.phi0 = voigt<T>(L, T(0.5) * (p.lw + a.lw), L.dnu - L.nu0 * a.u);
+    c.srcl0 = L.hknu * a.nu * L.A * c.phi0;
+    c.alpl0 = L.hknu * c.phi0 * (a.nl * L.Bdu - a.nu * L.Bud);
+    const T al = a.ad + c.alpl0;
+    c.S0 = al > T(0) ? ddiv<T>(a.jd + c.srcl0, al) : T(0);
+    c.init = 0;
+}
+
+// segment (a -> b) of charintline: node flags, the element or its sub-grid,
+// the maser flag
+template <typename T, bool AFF>
+__device__ inline void segment_exact(const LineK<T> &L, Acc<T, AFF> &x, const NodeRec<T> &a,
+                                     const NodeRec<T> &b, T istar, T starfract, Carry<T> &c,
+                                     int &ovs, int &maser) {
+    T ds = b.ds;
+    const int fl = (int)b.flag;
+    if (fl & NF_RESET) { ds = T(0); c.init = 1; }
+    if (fl & NF_BLEND) {
+        x.map(T(1) - starfract, starfract * istar);
+        c.init = 1;
+    }
+    if (fl & NF_STAR) {
+        x.map(T(0), istar);
+        c.init = 1;
+    }
+    clever_elem<T>(L, x, ds, pt_of(a), pt_of(b), a.lw, b.lw, c, ovs);
+    if (c.alpl0 * ds < T(-0.01)) maser = 1;
+}
 
 }  // namespace rl

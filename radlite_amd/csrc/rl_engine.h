@@ -55,6 +55,7 @@ struct ItemDev {
     long long hot_off;         // FP32: the inclination's segment records, in bytes from the
     long long aux_off;         // batch's record buffer (so that the kernels see global memory)
     long long rec0;            // first node record
+    long long blk0;            // first block record (rl_blocks.h)
     long long img0;            // first image value ([ray][channel])
     long long chan0;           // per channel: dnu at chan0, velo at chan0+nfr, the star's
                                // intensity at chan0+2nfr, the outer boundary's at chan0+3nfr
@@ -72,11 +73,13 @@ struct BatchLaunch {
     const ItemDev *items;      // device
     const CellRec *cells;      // [slots][ncell]
     void *rec;
+    void *blk;                 // block records, or null (every segment integrated)
     RayInfo *rinfo;
     const double *chan;
     double *image, *partial, *flux;
     unsigned char *cmask;      // optional [image layout]: 1 where integrated
     double d2;
+    const int *sel;            // device [nitems] the items' indices
     const long long *tile0;    // device [nitems+1] first tile of each item
     long long ntiles;
     unsigned long long *ovs, *counter;

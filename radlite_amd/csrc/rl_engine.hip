@@ -31,6 +31,8 @@
 #include "rl_traj.h"
 #include "rl_adjoint.h"
 #include "rl_fwd32.h"
+#include "rl_blocks.h"
+#include "rl_walk.h"
 
 namespace rl {
 
@@ -494,46 +496,6 @@ __device__ inline void finish_window(int ray, int lane, double umin, double umax
     }
 }
 
-// FP64 parity path: node values as the reference holds them (one wave
-// per ray)
-__device__ inline void nodes_ray_exact(int ray, int lane, const long long *__restrict__ off,
-                                       const GeoNode *__restrict__ geo,
-                                       const CellRec *__restrict__ cells,
-                                       NodeRec<double> *__restrict__ rec,
-                                       RayInfo *__restrict__ rinfo, int nfr,
-                                       const double *__restrict__ velo, double aks2,
-                                       int skip_mode) {
-    const long long b = off[ray];
-    const int n = (int)(off[ray + 1] - b);
-    double umin = 1.0e300, umax = -1.0e300;
-    for (int k = lane; k < n; k += 64) {
-        const GeoNode gn = geo[b + k];
-        double v[5];
-        node_interp(gn, cells, v);
-        NodeRec<double> r;
-        r.ds = gn.ds; r.u = gn.u;
-        r.jd = v[CR_JD]; r.ad = v[CR_AD]; r.lw = v[CR_LW]; r.nu = v[CR_NU]; r.nl = v[CR_NL];
-        r.flag = (double)(gn.flag >> 2);
-        rec[b + k] = r;
-        // window from the node preceding each segment (telescope.F:4265-4270)
-        if (k + 1 < n && v[CR_NU] + v[CR_NL] > LEVTHRES) {
-            umin = fmin(umin, gn.u);
-            umax = fmax(umax, gn.u);
-        }
-    }
-    finish_window(ray, lane, umin, umax, nfr, velo, aks2, skip_mode, n, rinfo);
-}
-
-__global__ void __launch_bounds__(64)
-k_nodes(int nrays, const long long *__restrict__ off, const GeoNode *__restrict__ geo,
-        const CellRec *__restrict__ cells, NodeRec<double> *__restrict__ rec,
-        RayInfo *__restrict__ rinfo, int nfr, const double *__restrict__ velo,
-        double aks2, int skip_mode) {
-    if ((int)blockIdx.x >= nrays) return;
-    nodes_ray_exact(blockIdx.x, threadIdx.x, off, geo, cells, rec, rinfo, nfr, velo, aks2,
-                    skip_mode);
-}
-
 // per-node scale for the FP32 records: the dust opacity where there is
 // dust, else the largest line coefficient, else 1
 __device__ inline void scaled_node(const double v[5], const LineConst &lc, double &sig,
@@ -543,6 +505,106 @@ __device__ inline void scaled_node(const double v[5], const LineConst &lc, doubl
     sig = v[CR_AD];
     if (!(sig > 0.0)) sig = fmax(fmax(fabs(dc), fabs(jc)), fabs(v[CR_JD]));
     if (!(sig > 0.0)) sig = 1.0;
+}
+
+// FP64 parity path: node values as the reference holds them, and the
+// line-free blocks (blk null: none) (one wave per ray)
+__device__ inline void nodes_ray_exact(int ray, int lane, const long long *__restrict__ off,
+                                       const GeoNode *__restrict__ geo,
+                                       const CellRec *__restrict__ cells,
+                                       NodeRec<double> *__restrict__ rec,
+                                       BlkRec *__restrict__ blk,
+                                       RayInfo *__restrict__ rinfo, int nfr,
+                                       const double *__restrict__ velo, double aks2,
+                                       int skip_mode, const LineConst &lc) {
+    const long long b = off[ray];
+    const int n = (int)(off[ray + 1] - b);
+    if (blk) blk += blk_of(b, ray);
+    double umin = 1.0e300, umax = -1.0e300;
+    // the last lane's node of the previous 64, for this 64's first segment
+    double jd_c = 0.0, ad_c = 0.0, u_c = 0.0, lw_c = 0.0;
+    float jr_c = 0.0f, wl_c = 0.0f;
+    int bits_c = 2;
+    for (int k0 = 0; k0 < n; k0 += 64) {
+        const int k = k0 + lane;
+        const bool act = k < n;
+        const GeoNode gn = geo[b + (act ? k : n - 1)];
+        double v[5];
+        node_interp(gn, cells, v);
+        const int fl = gn.flag >> 2;
+        if (act) {
+            NodeRec<double> r;
+            r.ds = gn.ds; r.u = gn.u;
+            r.jd = v[CR_JD]; r.ad = v[CR_AD]; r.lw = v[CR_LW]; r.nu = v[CR_NU]; r.nl = v[CR_NL];
+            r.flag = (double)fl;
+            rec[b + k] = r;
+            // window from the node preceding each segment (telescope.F:4265-4270)
+            if (k + 1 < n && v[CR_NU] + v[CR_NL] > LEVTHRES) {
+                umin = fmin(umin, gn.u);
+                umax = fmax(umax, gn.u);
+            }
+        }
+        if (!blk) continue;
+        // the dust element of segment k from the node before it, as
+        // integ_elem forms it with a line of 0
+        const double jc = lc.hknu * v[CR_NU] * lc.A;
+        const double dc = lc.hknu * (v[CR_NL] * lc.Bdu - v[CR_NU] * lc.Bud);
+        const float jr = fmaxf(blk_ratio(jc, v[CR_JD]), blk_ratio(dc, v[CR_AD]));
+        const bool fin = fabs(jc) + fabs(dc) < (double)INFINITY;
+        double jd_p = __shfl_up(v[CR_JD], 1), ad_p = __shfl_up(v[CR_AD], 1);
+        double u_p = __shfl_up(gn.u, 1), lw_p = __shfl_up(v[CR_LW], 1);
+        float jr_p = __shfl_up(jr, 1);
+        const int bits = (dc < 0.0 ? 1 : 0) | (fin ? 2 : 0);
+        int bits_p = __shfl_up(bits, 1);
+        if (lane == 0) {
+            jd_p = jd_c; ad_p = ad_c; u_p = u_c; lw_p = lw_c; jr_p = jr_c; bits_p = bits_c;
+        }
+        const bool inv_p = (bits_p & 1) != 0, fin_p = (bits_p & 2) != 0;
+        const double lwav = 0.5 * (lw_p + v[CR_LW]);
+        // the widest and narrowest profile of the two segments at node k-1
+        float wl_p = __shfl_up((float)lwav, 1);
+        if (lane == 0) wl_p = wl_c;
+        const float wl = (float)lwav;
+        if (k <= 1) wl_p = wl;
+        const float wmax = fmaxf(wl, wl_p), wmin = fminf(wl, wl_p);
+        double A = 1.0, B = 0.0;
+        float lo = INFINITY, hi = -INFINITY;
+        bool ovf = false;
+        if (act && k > 0) {
+            const double ds = (fl & NF_RESET) ? 0.0 : gn.ds;
+            int ov = 0;
+            double S0 = 0.0;
+            qdr_map<double>(jd_p, ad_p, v[CR_JD], v[CR_AD], ds, ov, S0, false, A, B);
+            ovf = ov != 0;
+            const float norm = 0.56419583546f / ((float)lc.c_aa * wmin);
+            const float z = blk_zcut<double>(fmaxf(jr, jr_p) * norm, inv_p || dc < 0.0) *
+                            (3.33567e-6f / SQRT_LOG2E) * wmax;
+            lo = fminf((float)u_p, (float)gn.u) - z;
+            hi = fmaxf((float)u_p, (float)gn.u) + z;
+            // never free: the star's intensity, which follows the channel, and
+            // a line that is not a number anywhere if it is not one here
+            if ((fl & (NF_BLEND | NF_STAR)) || !fin_p || !fin) { lo = -INFINITY; hi = INFINITY; }
+        }
+        blk_store(lane, k, n, A, B, lo, hi, ovf, blk);
+        jd_c = __shfl(v[CR_JD], 63);
+        ad_c = __shfl(v[CR_AD], 63);
+        u_c = __shfl(gn.u, 63);
+        lw_c = __shfl(v[CR_LW], 63);
+        jr_c = __shfl(jr, 63);
+        wl_c = __shfl(wl, 63);
+        bits_c = __shfl(bits, 63);
+    }
+    finish_window(ray, lane, umin, umax, nfr, velo, aks2, skip_mode, n, rinfo);
+}
+
+__global__ void __launch_bounds__(64)
+k_nodes(int nrays, const long long *__restrict__ off, const GeoNode *__restrict__ geo,
+        const CellRec *__restrict__ cells, NodeRec<double> *__restrict__ rec,
+        RayInfo *__restrict__ rinfo, int nfr, const double *__restrict__ velo,
+        double aks2, int skip_mode, LineConst lc) {
+    if ((int)blockIdx.x >= nrays) return;
+    nodes_ray_exact(blockIdx.x, threadIdx.x, off, geo, cells, rec, nullptr, rinfo, nfr, velo,
+                    aks2, skip_mode, lc);
 }
 
 // scaled records (FP32 performance path; both precisions of the adjoint):
@@ -641,20 +703,29 @@ k_segrec(long long nnodes, const long long *__restrict__ off, int nrays,
     seg_record(gn, first, up, lwp, interp_field(gn, lw), hot[k], aux[k]);
 }
 
-// per item, one wave per ray: the scaled line records and the NONREDUNDANT
-// window (telescope.F:4265-4270) of the FP32 batched forward
+// per item, one wave per ray: the scaled line records, the line-free
+// blocks (blk null: none) and the NONREDUNDANT window (telescope.F:4265-4270)
+// of the FP32 batched forward
 __device__ inline void nodes_ray_line(int ray, int lane, const long long *__restrict__ off,
                                       const GeoNode *__restrict__ geo,
                                       const CellRec *__restrict__ cells,
-                                      NodeLine *__restrict__ rec, RayInfo *__restrict__ rinfo,
+                                      NodeLine *__restrict__ rec,
+                                      BlkRec *__restrict__ blk,
+                                      RayInfo *__restrict__ rinfo,
                                       int nfr, const double *__restrict__ velo, double aks2,
                                       int skip_mode, const LineConst &lc) {
     const long long b = off[ray];
     const int n = (int)(off[ray + 1] - b);
+    if (blk) blk += blk_of(b, ray);
     const double inv_nu0 = 1.0 / fabs(lc.nu0);
     double umin = 1.0e300, umax = -1.0e300;
-    for (int k = lane; k < n; k += 64) {
-        const GeoNode gn = geo[b + k];
+    // the last lane's node of the previous 64, for this 64's first segment
+    NodeLine q_c{0.0f, 0.0f, 0.0f, 0.0f};
+    float u_c = 0.0f, lw_c = 0.0f, wl_c = 0.0f;
+    for (int k0 = 0; k0 < n; k0 += 64) {
+        const int k = k0 + lane;
+        const bool act = k < n;
+        const GeoNode gn = geo[b + (act ? k : n - 1)];
         double v[5];
         node_interp(gn, cells, v);
         double sig, jc, dc;
@@ -665,11 +736,69 @@ __device__ inline void nodes_ray_line(int ray, int lane, const long long *__rest
         r.jdh = (float)(v[CR_JD] / sig);
         r.jcl = (float)(jc / sig * inv_nu0);
         r.dcl = (float)(dc / sig * inv_nu0);
-        rec[b + k] = r;
-        if (k + 1 < n && v[CR_NU] + v[CR_NL] > LEVTHRES) {
-            umin = fmin(umin, gn.u);
-            umax = fmax(umax, gn.u);
+        if (act) {
+            rec[b + k] = r;
+            if (k + 1 < n && v[CR_NU] + v[CR_NL] > LEVTHRES) {
+                umin = fmin(umin, gn.u);
+                umax = fmax(umax, gn.u);
+            }
         }
+        if (!blk) continue;
+        // the dust element of segment k from the node before it, as elem32
+        // forms it with a line of 0
+        const float u1 = (float)gn.u, lw1 = (float)v[CR_LW];
+        NodeLine p;
+        p.sig = __shfl_up(r.sig, 1);
+        p.jdh = __shfl_up(r.jdh, 1);
+        p.jcl = __shfl_up(r.jcl, 1);
+        p.dcl = __shfl_up(r.dcl, 1);
+        float u_p = __shfl_up(u1, 1), lw_p = __shfl_up(lw1, 1);
+        if (lane == 0) { p = q_c; u_p = u_c; lw_p = lw_c; }
+        const float wl = 0.5f * (lw_p + lw1);
+        // the widest and narrowest profile of the two segments at node k-1
+        float wl_p = __shfl_up(wl, 1);
+        if (lane == 0) wl_p = wl_c;
+        if (k <= 1) wl_p = wl;
+        const float wmax = fmaxf(wl, wl_p), wmin = fminf(wl, wl_p);
+        double A = 1.0, B = 0.0;
+        float lo = INFINITY, hi = -INFINITY;
+        bool ovf = false;
+        if (act && k > 0) {
+            const int fl = gn.flag >> 2;
+            const float hds = (fl & NF_RESET) ? 0.0f : (float)(0.5 * gn.ds);
+            Car32 c;
+            const float ah0 = nl_adh(p.sig), ah1 = nl_adh(r.sig);
+            c.sa0 = fabsf(p.sig) * ah0;
+            c.sj0 = fabsf(p.sig) * p.jdh;
+            c.ah0 = ah0;
+            c.S0 = ah0 > 0.0f ? FOps<float>::sdiv(p.jdh, ah0) : 0.0f;
+            float e0, q;
+            elem_map32(hds, 0.0f, 0.0f, 0.0f, fabsf(r.sig), ah1, r.jdh, c, ovf, e0, q);
+            A = 1.0 - (double)e0;
+            B = (double)q;
+            const float M = fmaxf(fmaxf(blk_ratio(p.jcl, p.jdh), blk_ratio(p.dcl, ah0)),
+                                  fmaxf(blk_ratio(r.jcl, r.jdh), blk_ratio(r.dcl, ah1)));
+            const float ng = 0.56419583546f / (3.33567e-6f * wmin);
+            const float most = (fabsf(p.jcl) + fabsf(p.dcl) + fabsf(r.jcl) + fabsf(r.dcl)) * ng;
+            const float z = blk_zcut<float>(M * ng, p.dcl < 0.0f || r.dcl < 0.0f) *
+                            (3.33567e-6f / SQRT_LOG2E) * wmax;
+            lo = fminf(u_p, u1) - z;
+            hi = fmaxf(u_p, u1) + z;
+            // never free: the star's intensity, which follows the channel, and
+            // a line that is not a number anywhere if it is not one here
+            if ((fl & (NF_BLEND | NF_STAR)) || !(most < INFINITY)) {
+                lo = -INFINITY;
+                hi = INFINITY;
+            }
+        }
+        blk_store(lane, k, n, A, B, lo, hi, ovf, blk);
+        q_c.sig = __shfl(r.sig, 63);
+        q_c.jdh = __shfl(r.jdh, 63);
+        q_c.jcl = __shfl(r.jcl, 63);
+        q_c.dcl = __shfl(r.dcl, 63);
+        u_c = __shfl(u1, 63);
+        lw_c = __shfl(lw1, 63);
+        wl_c = __shfl(wl, 63);
     }
     finish_window(ray, lane, umin, umax, nfr, velo, aks2, skip_mode, n, rinfo);
 }
@@ -695,37 +824,40 @@ k_nodes_fast(int nrays, const long long *__restrict__ off, const GeoNode *__rest
 // ---------------------------------------------------------------------
 // formal solution
 // ---------------------------------------------------------------------
+// One lane's ray, block by block as the wave walk (rl_walk.h) takes it (blk
+// null: every segment integrated).
 template <typename T>
-__device__ inline T trace_one(const NodeRec<T> *__restrict__ rec, int n, const LineK<T> &L,
+__device__ inline T trace_one(const NodeRec<T> *__restrict__ rec,
+                              const BlkRec *__restrict__ blk, int n, const LineK<T> &L,
                               T I0, T istar, T starfract, int &ovs, int &maser,
                               T *tau = nullptr) {
-    T I = I0;
+    Acc<T, false> x{I0, T(1)};
     Carry<T> c;
     c.init = 1; c.phi0 = T(0); c.srcl0 = T(0); c.alpl0 = T(0); c.S0 = T(0);
-    NodeRec<T> a = rec[0];
-    Pt<T> pa{a.jd, a.ad, a.u, a.nu, a.nl};
-    T lwa = a.lw;
+    bool fresh = true;
+    NodeRec<T> a{};
     for (int k = 1; k < n; k++) {
-        NodeRec<T> b = rec[k];
-        T ds = b.ds;
-        int fl = (int)b.flag;
-        if (fl & NF_RESET) { ds = T(0); c.init = 1; }
-        if (fl & NF_BLEND) {
-            I = (T(1) - starfract) * I + starfract * istar;
-            c.init = 1;
+        if (blk && (k == 1 || (k & (BLK - 1)) == 0)) {
+            const BlkRec r = blk[k >> BLK_LOG];
+            if (blk_free(r, L.uch)) {
+                x.map(r.A, r.B);
+                ovs += blk_overshoots(r);
+                fresh = true;
+                k |= BLK - 1;
+                continue;
+            }
         }
-        if (fl & NF_STAR) {
-            I = istar;
-            c.init = 1;
+        if (fresh) {
+            a = rec[k - 1];
+            if (k > 1) carry_of<T>(L, rec[k - 2], a, c);
+            fresh = false;
         }
-        Pt<T> pb{b.jd, b.ad, b.u, b.nu, b.nl};
-        clever_elem<T>(L, I, ds, pa, pb, lwa, b.lw, c, ovs);
-        if (c.alpl0 * ds < T(-0.01)) maser = 1;
-        pa = pb;
-        lwa = b.lw;
+        const NodeRec<T> b = rec[k];
+        segment_exact<T>(L, x, a, b, istar, starfract, c, ovs, maser);
+        a = b;
     }
     if (tau) *tau = c.tau;
-    return I;
+    return x.I;
 }
 
 // node records of the batched forward: exact FP64 records, or the FP32
@@ -737,14 +869,16 @@ template <typename T> struct PvRecOf { using type = NodeRec<double>; };
 template <> struct PvRecOf<float> { using type = FastRec; };
 
 template <typename T>
-__device__ inline double trace_dispatch(const typename RecOf<T>::type *rec, const SegHot *hot,
-                                        const SegAux *aux, long long b, int n,
+__device__ inline double trace_dispatch(const typename RecOf<T>::type *rec,
+                                        const BlkRec *blk, const SegHot *hot,
+                                        const SegAux *aux, long long b, int ray, int n,
                                         const LineConst &lc, double dnu, double velo,
                                         double istar, double I0, T sf, int &ovs, int &maser);
 
 template <>
-__device__ inline double trace_dispatch<double>(const NodeRec<double> *rec, const SegHot *,
-                                                const SegAux *, long long b, int n,
+__device__ inline double trace_dispatch<double>(const NodeRec<double> *rec,
+                                                const BlkRec *blk, const SegHot *,
+                                                const SegAux *, long long b, int ray, int n,
                                                 const LineConst &lc, double dnu, double velo,
                                                 double istar, double I0, double sf, int &ovs,
                                                 int &maser) {
@@ -752,17 +886,19 @@ __device__ inline double trace_dispatch<double>(const NodeRec<double> *rec, cons
     L.nu0 = lc.nu0; L.c_aa = lc.c_aa; L.hknu = lc.hknu;
     L.A = lc.A; L.Bud = lc.Bud; L.Bdu = lc.Bdu;
     L.dnu = dnu; L.uch = velo;
-    return trace_one<double>(rec + b, n, L, I0, istar, sf, ovs, maser);
+    return trace_one<double>(rec + b, blk ? blk + blk_of(b, ray) : nullptr, n, L, I0, istar, sf,
+                             ovs, maser);
 }
 
 template <>
-__device__ inline double trace_dispatch<float>(const NodeLine *rec, const SegHot *hot,
-                                               const SegAux *aux, long long b, int n,
+__device__ inline double trace_dispatch<float>(const NodeLine *rec,
+                                               const BlkRec *blk, const SegHot *hot,
+                                               const SegAux *aux, long long b, int ray, int n,
                                                const LineConst &, double, double velo,
                                                double istar, double I0, float sf, int &ovs,
                                                int &maser) {
-    return (double)trace_split(hot + b, aux + b, rec + b, n, (float)velo, (float)I0,
-                               (float)istar, sf, ovs, maser);
+    return trace_split(hot + b, aux + b, rec + b, blk ? blk + blk_of(b, ray) : nullptr, n,
+                       (float)velo, I0, (float)istar, sf, ovs, maser);
 }
 
 // image placeholder of a channel left out by NONREDUNDANT skipping (a NaN
@@ -778,31 +914,6 @@ __device__ inline unsigned char window_mask(int ray, int ch, const RayInfo *__re
     if (skip_mode != 0 || ray == 0 || ch == 0) return 1;
     const RayInfo ri = rinfo[ray];
     return velo[ch] <= (double)ri.mx + aks2 && velo[ch] >= (double)ri.mn - aks2;
-}
-
-// one (ray, channel) of make_image_circular's loop (telescope.F:550-613):
-// integrated, or marked for the lazy-continuum pass when NONREDUNDANT
-// skipping leaves it out of the ray's window
-template <typename T>
-__device__ inline double formal_one(int ray, int ch, const long long *__restrict__ off,
-                                    const typename RecOf<T>::type *__restrict__ rec,
-                                    const SegHot *__restrict__ hot,
-                                    const SegAux *__restrict__ aux,
-                                    const RayInfo *__restrict__ rinfo,
-                                    const double *__restrict__ dnu,
-                                    const double *__restrict__ velo,
-                                    const double *__restrict__ istar,
-                                    const double *__restrict__ i0, const LineConst &lc,
-                                    double aks2, int skip_mode, int &ovs, int &maser) {
-    const RayInfo ri = rinfo[ray];
-    bool doit = true;
-    if (skip_mode == 0 && ray > 0 && ch > 0 && ch != ri.cont) {
-        doit = velo[ch] <= (double)ri.mx + aks2 && velo[ch] >= (double)ri.mn - aks2;
-    }
-    if (!doit) return __longlong_as_double(SKIPPED_BITS);   // filled by k_fixup
-    T sf = ray == 0 ? (T)lc.starfract : T(0);
-    return trace_dispatch<T>(rec, hot, aux, off[ray], ri.n, lc, dnu[ch], velo[ch], istar[ch],
-                             i0[ch], sf, ovs, maser);
 }
 
 __global__ void k_flux_partial(int nfr, int nrings, int nphi, int rings_per_chunk,
@@ -882,7 +993,7 @@ k_formal_posvel(int nrays, int nfr, int nx, int ny, const long long *__restrict_
                 L.nu0 = lc.nu0; L.c_aa = lc.c_aa; L.hknu = lc.hknu;
                 L.A = lc.A; L.Bud = lc.Bud; L.Bdu = lc.Bdu;
                 L.dnu = dnu[ch]; L.uch = velo[ch];
-                I = trace_one<double>(rec + b, n, L, i0[ch], istar[ch], 0.0, ovs, maser, &t);
+                I = trace_one<double>(rec + b, nullptr, n, L, i0[ch], istar[ch], 0.0, ovs, maser, &t);
             } else {
                 FastLine L{(float)lc.nu0, (float)dnu[ch], (float)velo[ch]};
                 float tf = 0.0f;
@@ -924,7 +1035,7 @@ void launch_posvel(hipStream_t st, const PosvelLaunch &a) {
     auto *rec = reinterpret_cast<typename PvRecOf<T>::type *>(a.rec);
     if constexpr (std::is_same<T, double>::value)
         hipLaunchKernelGGL(k_nodes, dim3(a.nrays), dim3(64), 0, st, a.nrays, a.off, a.geo,
-                           a.cells, rec, a.rinfo, a.nfr, a.velo, a.aks2, 1);
+                           a.cells, rec, a.rinfo, a.nfr, a.velo, a.aks2, 1, a.lc);
     else
         hipLaunchKernelGGL(k_nodes_fast<float>, dim3(a.nrays), dim3(64), 0, st, a.nrays, a.off,
                            a.geo, a.cells, rec, 0ll, a.rinfo, a.nfr, a.velo, a.aks2, 1, a.lc);
@@ -1008,7 +1119,7 @@ void launch_cells(hipStream_t st, int ncell, int nlev, int nlines, int line, int
 template <typename T>
 __global__ void __launch_bounds__(64)
 k_nodes_batch(const ItemDev *__restrict__ items, const CellRec *__restrict__ cells_all,
-              int ncell, void *rec_all, RayInfo *__restrict__ rinfo_all,
+              int ncell, void *rec_all, void *blk_all, RayInfo *__restrict__ rinfo_all,
               const double *__restrict__ chan_all) {
     const ItemDev &it = items[blockIdx.y];
     const int ray = blockIdx.x;
@@ -1018,11 +1129,13 @@ k_nodes_batch(const ItemDev *__restrict__ items, const CellRec *__restrict__ cel
     if constexpr (std::is_same<T, double>::value)
         nodes_ray_exact(ray, threadIdx.x, it.off, it.geo, cells,
                         reinterpret_cast<NodeRec<double> *>(rec_all) + it.rec0,
-                        rinfo_all + it.rinfo0, it.nfr, velo, it.aks2, it.skip_mode);
+                        blk_all ? reinterpret_cast<BlkRec *>(blk_all) + it.blk0 : nullptr,
+                        rinfo_all + it.rinfo0, it.nfr, velo, it.aks2, it.skip_mode, it.lc);
     else
         nodes_ray_line(ray, threadIdx.x, it.off, it.geo, cells,
-                       reinterpret_cast<NodeLine *>(rec_all) + it.rec0, rinfo_all + it.rinfo0,
-                       it.nfr, velo, it.aks2, it.skip_mode, it.lc);
+                       reinterpret_cast<NodeLine *>(rec_all) + it.rec0,
+                       blk_all ? reinterpret_cast<BlkRec *>(blk_all) + it.blk0 : nullptr,
+                       rinfo_all + it.rinfo0, it.nfr, velo, it.aks2, it.skip_mode, it.lc);
 }
 
 __global__ void k_zero_u64(unsigned long long *p, int n) {
@@ -1036,44 +1149,126 @@ __device__ inline const R *seg_ptr(const void *rec_all, long long off) {
     return reinterpret_cast<const R *>(static_cast<const char *>(rec_all) + off);
 }
 
-// Lane -> (ray, channel) of a tile.  cw == 0: the item's (ray, channel)
-// pairs in ray-major order, 64 per tile (a wave may span several rays);
-// cw in {16, 32, 64}: 64/cw rays per wave, cw consecutive channels each.
-__device__ inline bool tile_lane(int cw, long long lt, int lane, int nrays, int nfr, int &ray,
-                                 int &ch) {
-    if (cw == 0) {
-        const long long g = lt * 64 + lane;
-        if (g >= (long long)nrays * nfr) return false;
-        ray = (int)(g / nfr);
-        ch = (int)(g - (long long)ray * nfr);
-        return true;
-    }
-    const int chunks = (nfr + cw - 1) / cw, rows = 64 / cw;
-    const long long rb = lt / chunks;
-    const int cc = (int)(lt - rb * chunks);
-    ray = (int)(rb * rows) + lane / cw;
-    ch = cc * cw + (lane % cw);
-    return ray < nrays && ch < nfr;
+__device__ inline const BlkRec *blk_ptr(const void *blk_all, long long blk0) {
+    return blk_all ? reinterpret_cast<const BlkRec *>(blk_all) + blk0 : nullptr;
 }
 
-// Persistent formal solution over all tiles of all items: each wave takes
-// the next tile from a device counter until every tile is taken, so the
-// grid drains by itself; items of any size share the machine.
-#define RL_FORMAL_BATCH_PARAMS                                                              \
-    const ItemDev *__restrict__ items, int nitems, const long long *__restrict__ tile0,     \
-        long long ntiles, int cw, const void *rec_all,                                      \
-        const RayInfo *__restrict__ rinfo_all, const double *__restrict__ chan_all,         \
-        double *__restrict__ image_all, unsigned long long *__restrict__ ovs_all,            \
-        int *__restrict__ maser_all, unsigned char *__restrict__ cmask_all,                 \
-        unsigned long long *counter
-#define RL_FORMAL_BATCH_ARGS                                                                \
-    items, nitems, tile0, ntiles, cw, rec_all, rinfo_all, chan_all, image_all, ovs_all,     \
-        maser_all, cmask_all, counter
+// One wave's tile: 64/cw rays of an item and cw consecutive channels of
+// each, lane -> (ray rb*rows + lane/cw, channel cc*cw + lane%cw).  Every lane
+// of make_image_circular's loop (telescope.F:550-613) is integrated, or marked
+// for the lazy-continuum pass where NONREDUNDANT skipping leaves it out.
+struct FormalBatch {
+    const ItemDev *items;
+    const int *sel;              // the launch's items
+    const long long *tile0;      // first tile of each of them
+    int nsel, cw;
+    long long ntiles;
+    const void *rec, *blk;
+    const RayInfo *rinfo;
+    const double *chan;
+    double *image;
+    unsigned long long *ovs;
+    int *maser;
+    unsigned char *cmask;
+    unsigned long long *counter;
+};
 
+// the launch's item of tile t: the last with tile0 <= t
+__device__ inline int tile_item(const FormalBatch &f, long long t) {
+    int lo = 0, hi = f.nsel;
+    while (hi - lo > 1) {
+        const int m = (lo + hi) >> 1;
+        if (f.tile0[m] <= t) lo = m; else hi = m;
+    }
+    return lo;
+}
+
+// Tile t: part `part` of `parts` of its rays' blocks (the intensity for one
+// part; else the part's map I -> P I + B, I0 the outer boundary's).  Returns
+// whether the lane has a (ray, channel) to write at image index ix, integrated
+// (doit) or to be marked.
+template <typename T, bool AFF>
+__device__ __forceinline__ bool formal_tile(const FormalBatch &f, WalkLds<T> &lds, long long t,
+                                            int part, int parts, int &item, int &ray, int &ch,
+                                            long long &ix, bool &doit, double &I, double &P,
+                                            double &I0, int &ovs, int &maser) {
+    const int lane = threadIdx.x & 63, cw = f.cw, cwl = 31 - __clz(cw);
+    const int lo = tile_item(f, t);
+    item = f.sel[lo];
+    const ItemDev &it = f.items[item];
+    const int chunks = (it.nfr + cw - 1) >> cwl;
+    const long long lt = t - f.tile0[lo], rb = lt / chunks;
+    ray = (int)(rb << (6 - cwl)) + (lane >> cwl);
+    ch = (int)(lt - rb * chunks) * cw + (lane & (cw - 1));
+    const bool on = ray < it.nrays && ch < it.nfr;
+    const int rc = min(ray, it.nrays - 1), cc = min(ch, it.nfr - 1);
+    const RayInfo ri = f.rinfo[it.rinfo0 + rc];
+    const double *dnu = f.chan + it.chan0, *velo = dnu + it.nfr, *istar = dnu + 2 * it.nfr,
+                 *i0 = dnu + 3 * it.nfr;
+    const double v = velo[cc];
+    doit = on;
+    if (it.skip_mode == 0 && rc > 0 && cc > 0 && cc != ri.cont)
+        doit = doit && v <= (double)ri.mx + it.aks2 && v >= (double)ri.mn - it.aks2;
+    const long long b = it.off[rc];
+    // the ray's blocks of this part
+    const int n = ray < it.nrays ? ri.n : 0, nb = n < 2 ? 0 : (n + BLK - 1) >> BLK_LOG;
+    const int j0 = nb * part / parts, j1 = nb * (part + 1) / parts;
+    const BlkRec *blk = f.blk ? reinterpret_cast<const BlkRec *>(f.blk) + it.blk0 + blk_of(b, rc)
+                              : nullptr;
+    I0 = i0[cc];
+    const T sf = rc == 0 ? (T)it.lc.starfract : T(0);
+    if constexpr (std::is_same<T, double>::value) {
+        LineK<double> L;
+        L.nu0 = it.lc.nu0; L.c_aa = it.lc.c_aa; L.hknu = it.lc.hknu;
+        L.A = it.lc.A; L.Bud = it.lc.Bud; L.Bdu = it.lc.Bdu;
+        L.dnu = dnu[cc]; L.uch = v;
+        Acc<double, AFF> x{AFF ? 0.0 : I0, 1.0};
+        walk_exact<AFF>(lds, cwl, reinterpret_cast<const NodeRec<double> *>(f.rec) + it.rec0 + b,
+                        blk, n, j0, j1, doit, L, x, istar[cc], sf, ovs, maser);
+        I = x.I;
+        P = x.P;
+    } else {
+        const char *base = static_cast<const char *>(f.rec);
+        Acc32<AFF> x{AFF ? 0.0 : I0, 1.0};
+        bool ovf = false;
+        walk_split<AFF>(lds, cwl, reinterpret_cast<const SegHot *>(base + it.hot_off) + b,
+                        reinterpret_cast<const SegAux *>(base + it.aux_off) + b,
+                        reinterpret_cast<const NodeLine *>(f.rec) + it.rec0 + b, blk, n, j0, j1,
+                        doit, (float)v, x, (float)istar[cc], sf, ovf, maser);
+        I = x.I;
+        P = x.P;
+        ovs += ovf ? 1 : 0;
+    }
+    ix = it.img0 + (long long)ray * it.nfr + ch;
+    return on;
+}
+
+// a finished lane's image value and mask, and the wave's warnings
+__device__ inline void formal_write(const FormalBatch &f, int item, int ray, int ch, bool on,
+                                    bool doit, long long ix, double I, int ovs, int maser) {
+    const ItemDev &it = f.items[item];
+    if (on) {
+        f.image[ix] = doit ? I : __longlong_as_double(SKIPPED_BITS);   // filled by k_fixup
+        if (f.cmask)
+            f.cmask[ix] = window_mask(ray, ch, f.rinfo + it.rinfo0, f.chan + it.chan0 + it.nfr,
+                                      it.aks2, it.skip_mode);
+    }
+    for (int m = 32; m >= 1; m >>= 1) {
+        ovs += __shfl_xor(ovs, m);
+        maser |= __shfl_xor(maser, m);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        if (ovs) atomicAdd(f.ovs + item, (unsigned long long)ovs);
+        if (maser) atomicOr(f.maser + item, 1);
+    }
+}
+
+// Persistent formal solution over all tiles of the launch's items: each wave
+// takes the next tile from a device counter until every tile is taken, so the
+// grid drains by itself; items of any size share the machine.
 template <typename T>
-__device__ __forceinline__ void formal_batch_body(RL_FORMAL_BATCH_PARAMS) {
-    const auto *rec_base = reinterpret_cast<const typename RecOf<T>::type *>(rec_all);
-    const int lane = threadIdx.x & 63;
+__device__ __forceinline__ void formal_batch_body(const FormalBatch &f) {
+    __shared__ WalkLds<T> lds[4];
     for (;;) {
         // Every lane executes the atomic (lane 0 adds 1, the others 0) and the
         // tile index is lane 0's result through readfirstlane, so it is
@@ -1081,111 +1276,52 @@ __device__ __forceinline__ void formal_batch_body(RL_FORMAL_BATCH_PARAMS) {
         // lane-0-only atomic broadcast with a shuffle leaves the exit
         // condition divergent to the compiler, which may then iterate the
         // other lanes without lane 0.
-        const unsigned long long mine = atomicAdd(counter, lane == 0 ? 1ull : 0ull);
+        const unsigned long long mine = atomicAdd(f.counter, (threadIdx.x & 63) == 0 ? 1ull : 0ull);
         const unsigned lo32 = __builtin_amdgcn_readfirstlane((unsigned)(mine & 0xffffffffull));
         const unsigned hi32 = __builtin_amdgcn_readfirstlane((unsigned)(mine >> 32));
         const unsigned long long t = ((unsigned long long)hi32 << 32) | lo32;
-        if (t >= (unsigned long long)ntiles) break;
-        // item of the tile: last item with tile0[item] <= t
-        int lo = 0, hi = nitems;
-        while (hi - lo > 1) {
-            const int m = (lo + hi) >> 1;
-            if (tile0[m] <= (long long)t) lo = m; else hi = m;
-        }
-        const ItemDev &it = items[lo];
-        int ray = 0, ch = 0, ovs = 0, maser = 0;
-        if (tile_lane(cw, (long long)t - tile0[lo], lane, it.nrays, it.nfr, ray, ch)) {
-            const double *dnu = chan_all + it.chan0;
-            const long long ix = it.img0 + (long long)ray * it.nfr + ch;
-            const double v =
-                formal_one<T>(ray, ch, it.off, rec_base + it.rec0,
-                              seg_ptr<SegHot>(rec_all, it.hot_off),
-                              seg_ptr<SegAux>(rec_all, it.aux_off),
-                              rinfo_all + it.rinfo0, dnu,
-                              dnu + it.nfr, dnu + 2 * it.nfr, dnu + 3 * it.nfr, it.lc, it.aks2,
-                              it.skip_mode, ovs, maser);
-            image_all[ix] = v;
-            if (cmask_all)
-                cmask_all[ix] = window_mask(ray, ch, rinfo_all + it.rinfo0, dnu + it.nfr,
-                                            it.aks2, it.skip_mode);
-        }
-        for (int m = 32; m >= 1; m >>= 1) {
-            ovs += __shfl_xor(ovs, m);
-            maser |= __shfl_xor(maser, m);
-        }
-        if (lane == 0) {
-            if (ovs) atomicAdd(ovs_all + lo, (unsigned long long)ovs);
-            if (maser) atomicOr(maser_all + lo, 1);
-        }
+        if (t >= (unsigned long long)f.ntiles) break;
+        int item, ray, ch, ovs = 0, maser = 0;
+        long long ix;
+        bool doit;
+        double I, P, I0;
+        const bool on = formal_tile<T, false>(f, lds[threadIdx.x >> 6], (long long)t, 0, 1, item,
+                                              ray, ch, ix, doit, I, P, I0, ovs, maser);
+        formal_write(f, item, ray, ch, on, doit, ix, I, ovs, maser);
     }
 }
 
-// FP64 (the primary template; FP32 is specialised below): held to 128
-// VGPRs, four waves per SIMD instead of three (139 registers)
+// FP64 (the primary template; FP32 is specialised below)
 template <typename T>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-k_formal_batch(RL_FORMAL_BATCH_PARAMS) {
-    formal_batch_body<T>(RL_FORMAL_BATCH_ARGS);
+k_formal_batch(FormalBatch f) {
+    formal_batch_body<T>(f);
 }
-// FP32 (split records): held to 64 VGPRs, eight waves per SIMD (79
-// unconstrained, six waves: 61.4 ms on the 400x200 disk's two
-// inclinations; 72, seven waves: 54.1 ms; 64: 52.3 ms).  What spills is
-// per-tile state and the sub-grid path's, outside the fast segment loop.
 template <>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8)))
-k_formal_batch<float>(RL_FORMAL_BATCH_PARAMS) {
-    formal_batch_body<float>(RL_FORMAL_BATCH_ARGS);
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FORMAL32_WAVES)))
+k_formal_batch<float>(FormalBatch f) {
+    formal_batch_body<float>(f);
 }
 
-// The same tiles on a static grid: wave w of block b takes tile 4b + w
-// (the hardware dispatcher balances blocks); no tile counter and no tile
-// loop.
+// The same tiles on a static grid: wave w of block b takes tile 4b + w.
 template <typename T>
-__global__ void __launch_bounds__(256)
-k_formal_tiles(const ItemDev *__restrict__ items, int nitems,
-               const long long *__restrict__ tile0, long long ntiles, int cw,
-               const void *rec_all, const RayInfo *__restrict__ rinfo_all,
-               const double *__restrict__ chan_all, double *__restrict__ image_all,
-               unsigned long long *__restrict__ ovs_all, int *__restrict__ maser_all,
-               unsigned char *__restrict__ cmask_all) {
-    const auto *rec_base = reinterpret_cast<const typename RecOf<T>::type *>(rec_all);
-    const int lane = threadIdx.x & 63;
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? FORMAL32_WAVES : 4)))
+k_formal_tiles(FormalBatch f) {
+    __shared__ WalkLds<T> lds[4];
     const long long t = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= ntiles) return;                       // whole waves
-    int lo = 0, hi = nitems;
-    while (hi - lo > 1) {
-        const int m = (lo + hi) >> 1;
-        if (tile0[m] <= t) lo = m; else hi = m;
-    }
-    const ItemDev &it = items[lo];
-    int ray = 0, ch = 0, ovs = 0, maser = 0;
-    if (tile_lane(cw, t - tile0[lo], lane, it.nrays, it.nfr, ray, ch)) {
-        const double *dnu = chan_all + it.chan0;
-        const long long ix = it.img0 + (long long)ray * it.nfr + ch;
-        const double v =
-            formal_one<T>(ray, ch, it.off, rec_base + it.rec0,
-                          seg_ptr<SegHot>(rec_all, it.hot_off),
-                          seg_ptr<SegAux>(rec_all, it.aux_off),
-                          rinfo_all + it.rinfo0, dnu,
-                          dnu + it.nfr, dnu + 2 * it.nfr, dnu + 3 * it.nfr, it.lc, it.aks2,
-                          it.skip_mode, ovs, maser);
-        image_all[ix] = v;
-        if (cmask_all)
-            cmask_all[ix] = window_mask(ray, ch, rinfo_all + it.rinfo0, dnu + it.nfr, it.aks2,
-                                        it.skip_mode);
-    }
-    for (int m = 32; m >= 1; m >>= 1) {
-        ovs += __shfl_xor(ovs, m);
-        maser |= __shfl_xor(maser, m);
-    }
-    if (lane == 0) {
-        if (ovs) atomicAdd(ovs_all + lo, (unsigned long long)ovs);
-        if (maser) atomicOr(maser_all + lo, 1);
-    }
+    if (t >= f.ntiles) return;                     // whole waves
+    int item, ray, ch, ovs = 0, maser = 0;
+    long long ix;
+    bool doit;
+    double I, P, I0;
+    const bool on = formal_tile<T, false>(f, lds[threadIdx.x >> 6], t, 0, 1, item, ray, ch, ix,
+                                          doit, I, P, I0, ovs, maser);
+    formal_write(f, item, ray, ch, on, doit, ix, I, ovs, maser);
 }
 
 template <typename T>
 __global__ void k_fixup_batch(const ItemDev *__restrict__ items, const void *rec_all,
+                              const void *blk_all,
                               const RayInfo *__restrict__ rinfo_all,
                               const double *__restrict__ chan_all, double *__restrict__ image_all,
                               unsigned long long *__restrict__ ovs_all,
@@ -1208,9 +1344,10 @@ __global__ void k_fixup_batch(const ItemDev *__restrict__ items, const void *rec
         if (cont != 0.0) {
             row[ch] = cont;
         } else {
-            row[ch] = trace_dispatch<T>(rec, seg_ptr<SegHot>(rec_all, it.hot_off),
-                                        seg_ptr<SegAux>(rec_all, it.aux_off), it.off[ray], ri.n,
-                                        it.lc, dnu[ch],
+            row[ch] = trace_dispatch<T>(rec, blk_ptr(blk_all, it.blk0),
+                                        seg_ptr<SegHot>(rec_all, it.hot_off),
+                                        seg_ptr<SegAux>(rec_all, it.aux_off), it.off[ray], ray,
+                                        ri.n, it.lc, dnu[ch],
                                         velo[ch], istar[ch], i0[ch], T(0), ovs, maser);
             cont = row[ch];
         }
@@ -1252,35 +1389,25 @@ void launch_batch_nodes(hipStream_t st, int fp64, const BatchLaunch &b) {
     dim3 g(b.max_rays, b.nitems);
     if (fp64)
         hipLaunchKernelGGL(k_nodes_batch<double>, g, dim3(64), 0, st, b.items, b.cells, b.ncell,
-                           b.rec, b.rinfo, b.chan);
+                           b.rec, b.blk, b.rinfo, b.chan);
     else
         hipLaunchKernelGGL(k_nodes_batch<float>, g, dim3(64), 0, st, b.items, b.cells, b.ncell,
-                           b.rec, b.rinfo, b.chan);
+                           b.rec, b.blk, b.rinfo, b.chan);
 }
 
 void launch_batch_formal(hipStream_t st, int fp64, const BatchLaunch &b, int cw, int nblocks,
                          long long ntiles) {
+    const FormalBatch f{b.items, b.sel, b.tile0, b.nitems, cw, ntiles, b.rec, b.blk, b.rinfo,
+                        b.chan, b.image, b.ovs, b.maser, b.cmask, b.counter};
     if (nblocks == 0) {           // static grid
         const unsigned g = (unsigned)((ntiles + 3) / 4);
-        if (fp64)
-            hipLaunchKernelGGL(k_formal_tiles<double>, dim3(g), dim3(256), 0, st, b.items,
-                               b.nitems, b.tile0, ntiles, cw, b.rec, b.rinfo, b.chan, b.image,
-                               b.ovs, b.maser, b.cmask);
-        else
-            hipLaunchKernelGGL(k_formal_tiles<float>, dim3(g), dim3(256), 0, st, b.items,
-                               b.nitems, b.tile0, ntiles, cw, b.rec, b.rinfo, b.chan, b.image,
-                               b.ovs, b.maser, b.cmask);
+        if (fp64) hipLaunchKernelGGL(k_formal_tiles<double>, dim3(g), dim3(256), 0, st, f);
+        else hipLaunchKernelGGL(k_formal_tiles<float>, dim3(g), dim3(256), 0, st, f);
         return;
     }
     hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, b.counter, 1);
-    if (fp64)
-        hipLaunchKernelGGL(k_formal_batch<double>, dim3(nblocks), dim3(256), 0, st, b.items,
-                           b.nitems, b.tile0, ntiles, cw, b.rec, b.rinfo, b.chan, b.image,
-                           b.ovs, b.maser, b.cmask, b.counter);
-    else
-        hipLaunchKernelGGL(k_formal_batch<float>, dim3(nblocks), dim3(256), 0, st, b.items,
-                           b.nitems, b.tile0, ntiles, cw, b.rec, b.rinfo, b.chan, b.image,
-                           b.ovs, b.maser, b.cmask, b.counter);
+    if (fp64) hipLaunchKernelGGL(k_formal_batch<double>, dim3(nblocks), dim3(256), 0, st, f);
+    else hipLaunchKernelGGL(k_formal_batch<float>, dim3(nblocks), dim3(256), 0, st, f);
 }
 
 void launch_batch_finish(hipStream_t st, int fp64, const BatchLaunch &b) {
@@ -1288,10 +1415,10 @@ void launch_batch_finish(hipStream_t st, int fp64, const BatchLaunch &b) {
         dim3 g((b.max_rays + 127) / 128, b.nitems);
         if (fp64)
             hipLaunchKernelGGL(k_fixup_batch<double>, g, dim3(128), 0, st, b.items, b.rec,
-                               b.rinfo, b.chan, b.image, b.ovs, b.maser, b.cmask);
+                               b.blk, b.rinfo, b.chan, b.image, b.ovs, b.maser, b.cmask);
         else
             hipLaunchKernelGGL(k_fixup_batch<float>, g, dim3(128), 0, st, b.items, b.rec,
-                               b.rinfo, b.chan, b.image, b.ovs, b.maser, b.cmask);
+                               b.blk, b.rinfo, b.chan, b.image, b.ovs, b.maser, b.cmask);
     }
 }
 

@@ -66,6 +66,25 @@ struct alignas(16) NodeLine {
 
 constexpr float SQRT_LOG2E = 1.20112240878644977f;
 
+// A block of BLK segments as a channel without the line sees it: outside
+// [lo, hi] (dnu/nu0) I <- A I + B; the low bits of lo count its elements that
+// overshoot (rl_blocks.h)
+constexpr int BLK_LOG = 3, BLK = 1 << BLK_LOG;
+struct BlkRec {
+    float lo, hi;
+    double A, B;
+};
+__host__ __device__ inline long long blk_of(long long b, int ray) { return (b >> BLK_LOG) + ray; }
+__host__ __device__ inline long long blk_count(long long nnodes, int nrays) {
+    return (nnodes >> BLK_LOG) + nrays;
+}
+template <typename T> __device__ inline bool blk_free(const BlkRec &r, T uch) {
+    return uch < (T)r.lo || uch > (T)r.hi;
+}
+__device__ inline int blk_overshoots(const BlkRec &r) {
+    return __float_as_int(r.lo) & (2 * BLK - 1);
+}
+
 __device__ inline float nl_adh(float sig) { return __float_as_int(sig) < 0 ? 0.0f : 1.0f; }
 __device__ inline bool seg_general(float hds) { return __float_as_int(hds) < 0; }
 __device__ inline float ex2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -101,59 +120,80 @@ __device__ inline void carry32(const Pt32 &p, float uch, float ag, float ng, Car
 
 // One element from the carried start point to an end point with scaled
 // values (sg, adh, jdh) and profile-weighted line coefficients jcn = jcl
-// ng, dcn = dcl ng at e: I <- I exp(-dtau) + min(Q, J_max) (qdr_src_2,
-// transfer.F:1498-1571); ovf is set on an overshoot (Q > 2 J_max).
-__device__ inline float elem32(float I, float hds, float e, float jcn, float dcn, float sg,
-                               float adh, float jdh, Car32 &c, bool &ovf) {
+// ng, dcn = dcl ng at e: the map I <- I + (q - I e0) with e0 = 1 - exp(-dtau),
+// q = min(Q, J_max) (qdr_src_2, transfer.F:1498-1571); ovf is set on an
+// overshoot (Q > 2 J_max).
+__device__ __forceinline__ void elem_map32(float hds, float e, float jcn, float dcn, float sg, float adh,
+                                  float jdh, Car32 &c, bool &ovf, float &e0, float &q) {
     const float ah1 = fmaf(dcn, e, adh);
     const float jh1 = fmaf(jcn, e, jdh);
     const float sa1 = sg * ah1, sj1 = sg * jh1;
     const float dtau = (c.sa0 + sa1) * hds;
     const float theomax = (c.sj0 + sj1) * hds;
     float wa, wb, xp, ra;
-    qdr_weights_f<float>(dtau, wa, wb, xp, ra);
+    qdr_weights_f<float>(dtau, wa, wb, xp, ra, e0);
     // source functions with the fall-backs of transfer.F:1528-1541
     const float q1 = ah1 > 0.0f ? FOps<float>::sdiv(jh1, ah1) : 0.0f;
     const float q0 = c.S0;
     const float s1 = c.ah0 > 0.0f ? q0 : (ah1 > 0.0f ? q1 : 0.0f);
     const float s2 = ah1 > 0.0f ? q1 : (c.ah0 > 0.0f ? q0 : 0.0f);
-    float q = dtau > 1e-9f ? fmaf(wa, s1, wb * s2) : theomax;   // 1e-9 is REAL*4
+    q = dtau > 1e-9f ? fmaf(wa, s1, wb * s2) : theomax;   // 1e-9 is REAL*4
     ovf = ovf || (q > 2.0f * theomax);
     q = fminf(q, theomax);
     c.sa0 = sa1;
     c.sj0 = sj1;
     c.ah0 = ah1;
     c.S0 = q1;
-    return fmaf(I, xp, q);
 }
 
+// What a lane carries along its ray: the intensity, or (AFF) the map I -> P I
+// + I' of the part of the ray it has passed.  In double precision (the
+// elements' values in single): the elements a channel does not see the line
+// in are the same maps for every such channel, taken one by one or composed,
+// so that channels on and off the line differ by the line alone and not by
+// the rounding of the dust's sum, of which a weak line is a small part.  e0 =
+// 1 - exp(-dtau) rather than exp(-dtau): thin elements keep their digits.
+template <bool AFF> struct Acc32 {
+    double I, P;
+    __device__ void step(float e0, float q) {
+        I = I + __builtin_fma(-I, (double)e0, (double)q);
+        if (AFF) P = __builtin_fma(-P, (double)e0, P);
+    }
+    __device__ void map(double A, double B) {
+        I = __builtin_fma(I, A, B);
+        if (AFF) P = P * A;
+    }
+};
+
 // an element ending at point p of the general path
-__device__ inline float elem_pt32(float I, float hds, const Pt32 &p, float uch, float ag,
-                                  float ng, Car32 &c, bool &ovf, float &e_out) {
+template <bool AFF>
+__device__ __forceinline__ void elem_pt32(Acc32<AFF> &x, float hds, const Pt32 &p, float uch, float ag,
+                                 float ng, Car32 &c, bool &ovf, float &e_out) {
     const float z = (uch - p.u) * ag;
     const float e = ex2(-(z * z));
     e_out = e;
-    return elem32(I, hds, e, p.jcl * ng, p.dcl * ng, p.sig, p.adh, p.jdh, c, ovf);
+    float e0, q;
+    elem_map32(hds, e, p.jcl * ng, p.dcl * ng, p.sig, p.adh, p.jdh, c, ovf, e0, q);
+    x.step(e0, q);
 }
 
 // The general path of segment k (nodes k-1 -> k): node flags (hole chord,
-// central-beam star blend, star intensity), the start point when the
-// element starts afresh (init), and the sub-grid of
+// central-beam star blend, star intensity: the element then starts afresh
+// from the start point under its own profile) and the sub-grid of
 // clever_integrate_element_linedust (line.F:4706-4800): points s_i =
 // sleft + (i-1) lg, i = 1..31, used where 0 < s_i < ds, the quantities
 // interpolated linearly in s, the width held at the segment's mean.
-__device__ inline float seg_general32(float I, const SegHot &h, const SegAux &a0,
-                                      const SegAux &a1, const NodeLine &q0, const NodeLine &q1,
-                                      float uch, float istar, float sf, int &init, Car32 &c,
-                                      bool &ovf, int &maser) {
+template <bool AFF>
+__device__ __forceinline__ void seg_general32(Acc32<AFF> &x, const SegHot &h, float u0, const SegAux &a1,
+                                     const NodeLine &q0, const NodeLine &q1, float uch,
+                                     float istar, float sf, Car32 &c, bool &ovf, int &maser) {
     float ds = 2.0f * fabsf(h.hds);                     // (float)ds, hds = (float)(ds/2)
     const int fl = a1.flag;
-    if (fl & NF_RESET) { ds = 0.0f; init = 1; }
-    if (fl & NF_BLEND) { I = (1.0f - sf) * I + sf * istar; init = 1; }
-    if (fl & NF_STAR) { I = istar; init = 1; }
-    const Pt32 p0 = pt_of(a0.u, q0), p1 = pt_of(a1.u, q1);
-    if (init) carry32(p0, uch, h.ag, h.ng, c);
-    init = 0;
+    if (fl & NF_RESET) ds = 0.0f;
+    if (fl & NF_BLEND) x.map((double)(1.0f - sf), (double)(sf * istar));
+    if (fl & NF_STAR) x.map(0.0, (double)istar);
+    const Pt32 p0 = pt_of(u0, q0), p1 = pt_of(a1.u, q1);
+    if (fl) carry32(p0, uch, h.ag, h.ng, c);
     float sa = 0.0f, e1 = 0.0f;
     if (a1.dls >= 0.0f) {                                 // 6x > 1 (line.F:4715)
         const float s_c = ds * (uch - p0.u) * a1.inv_du;
@@ -184,72 +224,74 @@ __device__ inline float seg_general32(float I, const SegHot &h, const SegAux &a0
                                  w0 * p0.adh + w1 * p1.adh, w0 * p0.jcl + w1 * p1.jcl,
                                  w0 * p0.dcl + w1 * p1.dcl};
                     float eb;
-                    I = elem_pt32(I, 0.5f * (s - sa), b, uch, h.ag, h.ng, c, ovf, eb);
+                    elem_pt32(x, 0.5f * (s - sa), b, uch, h.ag, h.ng, c, ovf, eb);
                     sa = s;
                 }
             }
         }
     }
-    I = elem_pt32(I, 0.5f * (ds - sa), p1, uch, h.ag, h.ng, c, ovf, e1);
+    elem_pt32(x, 0.5f * (ds - sa), p1, uch, h.ag, h.ng, c, ovf, e1);
     // maser flag (telescope.F:4295-4297): line alpha * ds < -0.01 at the end
     if (p1.sig * (p1.dcl * h.ng * e1) * ds < -0.01f) maser = 1;
-    return I;
 }
 
-// charintline on split records: one channel (uch = dnu/nu0) of one ray of n
-// nodes from the outer boundary intensity I0
-__device__ inline float trace_split(const SegHot *__restrict__ hot, const SegAux *__restrict__ aux,
-                                    const NodeLine *__restrict__ line, int n, float uch, float I0,
-                                    float istar, float sf, int &ovs, int &maser) {
-    float I = I0;
-    if (n < 2) return I;
+// segment k from the carry (hot, aux, line: at node k; the general path reads
+// the two before it as well)
+template <bool AFF>
+__device__ __forceinline__ void segment32(Acc32<AFF> &x, const SegHot *hot, const SegAux *aux,
+                                          const NodeLine *line, float uch, float istar, float sf,
+                                          Car32 &c, bool &ovf, int &maser) {
+    const SegHot h = *hot;
+    const NodeLine q = *line;
+    if (seg_general(h.hds)) {
+        seg_general32(x, h, aux[-1].u, load_aux(aux), line[-1], q, uch, istar, sf, c, ovf, maser);
+    } else {
+        const float z = fmaf(uch, h.ag, -h.uag);
+        const float e = ex2(-(z * z));
+        const float dcn = q.dcl * h.ng;
+        float e0, b;
+        elem_map32(h.hds, e, q.jcl * h.ng, dcn, fabsf(q.sig), nl_adh(q.sig), q.jdh, c, ovf, e0, b);
+        x.step(e0, b);
+        // maser flag; the line coefficient is negative only where the
+        // populations are inverted
+        if (q.dcl < 0.0f && fabsf(q.sig) * (dcn * e) * (2.0f * h.hds) < -0.01f) maser = 1;
+    }
+}
+
+// charintline (telescope.F:3889-4312) on split records, one lane: one channel
+// (uch = dnu/nu0) of one ray of n nodes from the outer boundary intensity I0,
+// block by block as the wave walk (rl_walk.h) takes it.
+__device__ inline double trace_split(const SegHot *__restrict__ hot, const SegAux *__restrict__ aux,
+                                     const NodeLine *__restrict__ line,
+                                     const BlkRec *__restrict__ blk, int n, float uch, double I0,
+                                     float istar, float sf, int &ovs, int &maser) {
+    Acc32<false> x{I0, 1.0};
+    if (n < 2) return I0;
     Car32 c;
-    int init = 1;
-    bool ovf = false;
-    // segment 1 starts the ray: the general path reads its start point
-    I = seg_general32(I, hot[1], aux[0], load_aux(aux + 1), line[0], line[1], uch, istar, sf,
-                      init, c, ovf, maser);
-    auto segment = [&](int k, const SegHot &h, const NodeLine &q) {
-        if (seg_general(h.hds)) {
-            I = seg_general32(I, h, aux[k - 1], load_aux(aux + k), line[k - 1], q, uch, istar, sf,
-                              init, c, ovf, maser);
-        } else {
-            const float z = fmaf(uch, h.ag, -h.uag);
-            const float e = ex2(-(z * z));
-            const float dcn = q.dcl * h.ng;
-            I = elem32(I, h.hds, e, q.jcl * h.ng, dcn, fabsf(q.sig), nl_adh(q.sig), q.jdh, c, ovf);
-            // maser flag; the line coefficient is negative only where the
-            // populations are inverted
-            if (q.dcl < 0.0f && fabsf(q.sig) * (dcn * e) * (2.0f * h.hds) < -0.01f) maser = 1;
+    bool ovf = false, fresh = true;
+    for (int k0 = 0; k0 < n; k0 += BLK) {
+        if (blk) {
+            const BlkRec r = blk[k0 >> BLK_LOG];
+            if (blk_free(r, uch)) {
+                x.map(r.A, r.B);
+                ovf = ovf || blk_overshoots(r) != 0;
+                fresh = true;
+                continue;
+            }
         }
-    };
-    // Segments 2.. in pairs, the records in two register sets (A: segments
-    // k, k+2, ..; B: k+1, k+3, ..): a set is reloaded right after its
-    // segment is done, so the load overlaps the other set's segment and no
-    // copies rotate the registers.
-    if (n > 2) {
-        int k = 2;
-        SegHot hA = hot[k];
-        NodeLine qA = line[k];
-        const int k1 = k + 1 < n ? k + 1 : k;
-        SegHot hB = hot[k1];
-        NodeLine qB = line[k1];
-        for (;;) {
-            segment(k, hA, qA);
-            if (k + 1 >= n) break;
-            const int ka = k + 2 < n ? k + 2 : n - 1;
-            hA = hot[ka];
-            qA = line[ka];
-            segment(k + 1, hB, qB);
-            if (k + 2 >= n) break;
-            const int kb = k + 3 < n ? k + 3 : n - 1;
-            hB = hot[kb];
-            qB = line[kb];
-            k += 2;
+        for (int k = max(k0, 1); k < min(n, k0 + BLK); k++) {
+            if (fresh) {
+                // the carry of node k-1 as the end of segment k-1 (its profile);
+                // the ray's first node under segment 1's
+                const SegHot hp = hot[k > 1 ? k - 1 : 1];
+                carry32(pt_of(aux[k - 1].u, line[k - 1]), uch, hp.ag, hp.ng, c);
+                fresh = false;
+            }
+            segment32(x, hot + k, aux + k, line + k, uch, istar, sf, c, ovf, maser);
         }
     }
     ovs += ovf ? 1 : 0;
-    return I;
+    return x.I;
 }
 
 }  // namespace rl
