@@ -240,8 +240,7 @@ int rl_plan(rl_ctx *ctx, int nitems, const rl_item *items, double *out);
 /* A call to rl_trace_lines_forward runs its items in batches: every
  * item of a batch is resident in device memory at once, and each stage
  * (cell tables, node records, formal solution, flux) is one launch for
- * the whole batch, the formal solution as a persistent kernel over a
- * device work counter.  Batches are cut so that their device memory,
+ * the whole batch.  Batches are cut so that their device memory,
  * with the trajectories of their inclinations, stays within the budget
  * (a batch holds at least one item): bytes > 0 sets it, 0 (the default)
  * uses 60% of the device memory free at the context's first trace. */
@@ -250,14 +249,13 @@ int rl_set_memory_budget(rl_ctx *ctx, double bytes);
 enum {
     RL_OPT_GRAPH = 1,     /* 1 (default): record each batch shape's launches in a
                              hipGraph and replay it; 0: launch directly */
-    RL_OPT_AUTOTUNE = 2,  /* 1 (default): time the tile mappings and the grid
-                             (static, or persistent over a work counter) once per
-                             batch shape and keep the fastest; 0: defaults */
-    RL_OPT_TILE = 3,      /* fix the tile mapping (turns the autotuner off):
-                             16/32/64 = channels per ray in a wave, 0 = the
-                             default, 16 */
-    RL_OPT_PERSISTENT = 4,/* with a fixed mapping: 1 (default) persistent grid
-                             over the work counter, 0 static grid */
+    RL_OPT_AUTOTUNE = 2,  /* accepted for callers that set it; nothing is timed:
+                             the formal solution has one mapping */
+    RL_OPT_TILE = 3,      /* the channels of a ray that a wave takes at a time, at
+                             most: 16/32/64, or 0, the default, all that fit */
+    RL_OPT_PERSISTENT = 4,/* after RL_OPT_TILE: 1 (default) persistent grid over a
+                             work counter, 0 a block per unit of work (as without
+                             RL_OPT_TILE) */
     RL_OPT_CKPT = 5       /* adjoint checkpoint interval: 0 (default) chosen
                              from the memory budget (1 when every segment's I
                              fits half of it, else up to 16), or fixed to
@@ -265,8 +263,8 @@ enum {
 };
 int rl_set_option(rl_ctx *ctx, int option, int value);
 
-/* Batches of the last forward call, and the tile mapping and grid the
- * last batch used (blocks = 0: static grid; > 0: persistent blocks). */
+/* Batches of the last forward call, and RL_OPT_TILE's value and the grid the
+ * last batch used (blocks = 0: a block per unit; > 0: persistent blocks). */
 int rl_last_batch_info(const rl_ctx *ctx, int *batches, int *tile_cw, int *blocks);
 
 /* Wait for all work of the context. */

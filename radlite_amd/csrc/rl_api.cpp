@@ -142,16 +142,15 @@ struct rl_ctx {
     std::vector<DevBuf> spare;
     std::vector<DevBuf> x_cnt;               // k_cross node counts per slot
     // batching
-    DevBuf d_items, d_sel, d_tile0, d_counter, d_cmask;
+    DevBuf d_items, d_unit0, d_counter, d_cmask;
     std::vector<rl::ItemDev> h_items;
-    std::vector<long long> h_tile0;
-    std::vector<int> h_sel;
+    std::vector<long long> h_unit0;
     size_t mem_budget = 0;            // 0: a share of the free device memory
     size_t auto_budget = 0;
     unsigned long long tick = 0;      // use counter of the ray sets
     size_t last_work = 0;             // work bytes of the last call's largest unit
     int last_chunks = 0;
-    bool use_graph = true, autotune = true;
+    bool use_graph = true;
     int fixed_cw = -1, fixed_persistent = 1, last_cw = 0, last_blocks = 0, last_batches = 0;
     int last_kblk = 0, fixed_kblk = 0, last_used_tape = 0;
     // inputs generation: bumped by every setter, so that a tape taken
@@ -160,7 +159,6 @@ struct rl_ctx {
     // bumped whenever the line-width field changes (the FP32 segment
     // records depend on it)
     unsigned long long lw_gen = 1;
-    std::map<std::string, std::pair<int, int>> tune;
     std::map<std::string, hipGraphExec_t> graphs;
     // adjoint buffers; the tape of rl_trace_lines_forward_tape
     std::vector<AdjItemBufs> tape;
@@ -1140,10 +1138,9 @@ static size_t item_bytes(const rl_ctx *c, const rl_item &it, const RaySet &rs) {
            (size_t)rs.nrings * it.nfr * 8 + (size_t)it.nfr * 32 + (size_t)rs.nrays * 16 + 64;
 }
 
-static long long tiles_of(int cw, int nrays, int nfr) {
-    if (cw == 0) cw = 16;
-    const int rows = 64 / cw;
-    return (long long)((nrays + rows - 1) / rows) * ((nfr + cw - 1) / cw);
+// units (ray, channel chunk) of an item under chunks of cw channels
+static long long units_of(int cw, int nrays, int nfr) {
+    return (long long)nrays * ((nfr + cw - 1) / cw);
 }
 
 // batches: consecutive items whose buffers, with the nodes of their
@@ -1175,7 +1172,24 @@ static size_t cut_batches(rl_ctx *c, int nitems, const rl_item *items,
     return most;
 }
 
-// One batch: items [i0, i1) of the call, all resident at once.
+// The formal solution's launch over a batch's items: channels per chunk, first
+// units u0 [nb + 1], and the blocks of the persistent grid (0: a block per unit).
+struct FormalPlan { int cw, nblk; };
+static int formal_plan(rl_ctx *c, int fp64, const std::vector<rl::ItemDev> &hi, FormalPlan &p,
+                       std::vector<long long> &u0) {
+    p.cw = rl::formal_chunk();
+    if (c->fixed_cw > 0) p.cw = std::min(p.cw, c->fixed_cw);
+    u0.assign(hi.size() + 1, 0);
+    for (size_t k = 0; k < hi.size(); k++)
+        u0[k + 1] = u0[k] + units_of(p.cw, hi[k].nrays, hi[k].nfr);
+    p.nblk = 0;
+    if (c->fixed_cw < 0 || !c->fixed_persistent) return 0;
+    int cu = 0;
+    HIPCHK(c, hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, c->device));
+    p.nblk = cu * rl::formal_blocks_per_cu(fp64);
+    return 0;
+}
+
 static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *flux,
                      double *image, unsigned char *cmask, unsigned *warn, size_t fo,
                      size_t io) {
@@ -1237,11 +1251,7 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
     HIPCHK(c, c->d_maser.ensure((size_t)((nb + 1) / 2) * 8));
     HIPCHK(c, c->d_counter.ensure(8));
     HIPCHK(c, c->d_items.ensure((size_t)nb * sizeof(rl::ItemDev)));
-    HIPCHK(c, c->d_tile0.ensure((size_t)(nb + 1) * 8));
-    HIPCHK(c, c->d_sel.ensure((size_t)nb * 4));
-    c->h_sel.resize(nb);
-    for (int k = 0; k < nb; k++) c->h_sel[k] = k;
-    if (int e = upload(c, c->d_sel, c->h_sel.data(), (size_t)nb * 4)) return e;
+    HIPCHK(c, c->d_unit0.ensure((size_t)(nb + 1) * 8));
     if (cmask) HIPCHK(c, c->d_cmask.ensure((size_t)img0));
     if (int e = upload(c, c->d_chan, chan.data(), nchan * 8)) return e;
     c->cells_line = -1;       // d_cells is rewritten below for this batch's lines
@@ -1264,28 +1274,20 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
     L.partial = c->d_partial.as<double>();
     L.flux = c->d_flux.as<double>();
     L.d2 = (1.0 * 3.08572e18) * (1.0 * 3.08572e18);
-    L.sel = c->d_sel.as<int>();
-    L.tile0 = c->d_tile0.as<long long>();
+    L.unit0 = c->d_unit0.as<long long>();
     L.ovs = c->d_ovs.as<unsigned long long>();
     L.counter = c->d_counter.as<unsigned long long>();
     L.maser = c->d_maser.as<int>();
     L.cmask = cmask ? c->d_cmask.as<unsigned char>() : nullptr;
-    // tile mapping: autotuned once per batch shape (rays per wave, channel
-    // tiling, persistent grid size)
-    int dev_cu = 0;
-    HIPCHK(c, hipDeviceGetAttribute(&dev_cu, hipDeviceAttributeMultiprocessorCount, c->device));
-    const int bpc = rl::formal_batch_blocks_per_cu(fp64);
     std::string shape = std::to_string(fp64);
     for (int k = 0; k < nb; k++)
         shape += ":" + std::to_string(hi[k].nrays) + "x" + std::to_string(hi[k].nfr) + "s" +
                  std::to_string(hi[k].skip_mode);
-    auto set_tiles = [&](int cw) -> int {
-        std::vector<long long> &t0 = c->h_tile0;
-        t0.assign(nb + 1, 0);
-        for (int k = 0; k < nb; k++) t0[k + 1] = t0[k] + tiles_of(cw, hi[k].nrays, hi[k].nfr);
-        L.ntiles = t0[nb];
-        return upload(c, c->d_tile0, t0.data(), (size_t)(nb + 1) * 8);
-    };
+    FormalPlan fp;
+    std::vector<long long> &u0 = c->h_unit0;
+    if (int e = formal_plan(c, fp64, hi, fp, u0)) return e;
+    L.nunits = u0[nb];
+    if (int e = upload(c, c->d_unit0, u0.data(), (size_t)(nb + 1) * 8)) return e;
     auto zero_counters = [&]() {
         rl::launch_zero_u64(c->stream, L.ovs, nb);
         rl::launch_zero_u64(c->stream, reinterpret_cast<unsigned long long *>(L.maser),
@@ -1302,45 +1304,8 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
                              c->d_ad.as<double>(), c->d_cells.as<CellRec>() + q * ncell);
         }
     };
-    int cw = 0, nblk = dev_cu * bpc;
-    auto tuned = c->tune.find(shape);
-    if (c->fixed_cw >= 0) {
-        cw = c->fixed_cw;
-        nblk = c->fixed_persistent ? dev_cu * bpc : 0;
-    } else if (tuned != c->tune.end()) {
-        cw = tuned->second.first;
-        nblk = tuned->second.second;
-    } else if (c->autotune) {
-        // trials on the first tiles of the batch (enough to fill the device
-        // several times): static grid or persistent grid, x tile mapping
-        cells();
-        rl::launch_batch_nodes(c->stream, fp64, L);
-        float best = 1e30f;
-        const int cws[4] = {0, 64, 32, 16};
-        const int grids[2] = {0, dev_cu * bpc};
-        for (int ci = 0; ci < 4; ci++) {
-            if (int e = set_tiles(cws[ci])) return e;
-            const long long ntr = std::min<long long>(L.ntiles, 64LL * 4 * dev_cu * bpc);
-            for (int gi = 0; gi < 2; gi++) {
-                zero_counters();
-                HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
-                rl::launch_batch_formal(c->stream, fp64, L, cws[ci] ? cws[ci] : 16, grids[gi], ntr);
-                HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
-                HIPCHK(c, hipEventSynchronize(c->ev[3]));
-                float t = 0;
-                HIPCHK(c, hipEventElapsedTime(&t, c->ev[2], c->ev[3]));
-                // the whole batch at this rate: tiles hold 64 lanes in every
-                // mapping, but a channel tiling leaves the lanes past the last
-                // channel idle, so the mappings have different tile counts
-                t = t / (float)ntr * (float)L.ntiles;
-                if (t < best) { best = t; cw = cws[ci]; nblk = grids[gi]; }
-            }
-        }
-        c->tune[shape] = {cw, nblk};
-    }
-    c->last_cw = cw;
-    c->last_blocks = nblk;
-    if (int e = set_tiles(cw)) return e;
+    c->last_cw = c->fixed_cw > 0 ? c->fixed_cw : 0;
+    c->last_blocks = fp.nblk;
     HIPCHK(c, hipMemsetAsync(c->d_err.p, 0, 4, c->stream));
     // the device stages; recorded once per (shape, buffers) into a graph
     auto stages = [&](bool timed) -> int {
@@ -1348,7 +1313,7 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
         cells();
         rl::launch_batch_nodes(c->stream, fp64, L);
         if (timed) HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
-        rl::launch_batch_formal(c->stream, fp64, L, cw ? cw : 16, nblk, L.ntiles);
+        rl::launch_batch_formal(c->stream, fp64, L, fp.cw, fp.nblk);
         rl::launch_batch_finish(c->stream, fp64, L);
         if (timed) HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
         rl::launch_batch_flux(c->stream, L);
@@ -1362,12 +1327,12 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
         auto add = [&](const void *p) { snprintf(buf, sizeof buf, ":%p", p); gkey += buf; };
         for (const void *p : {c->d_rec.p, c->d_blk.p, c->d_image.p, c->d_partial.p, c->d_flux.p,
                               c->d_rinfo.p, c->d_cells.p, c->d_ovs.p, c->d_maser.p,
-                              c->d_counter.p, c->d_items.p, c->d_sel.p, c->d_tile0.p, c->d_chan.p,
+                              c->d_counter.p, c->d_items.p, c->d_unit0.p, c->d_chan.p,
                               (void *)L.cmask,
                               c->d_rho.p, c->d_abund.p, c->d_lw.p, c->d_pops.p, c->d_jd.p,
                               c->d_ad.p})
             add(p);
-        snprintf(buf, sizeof buf, ":%d:%d:%d:%d:%d:%.17g", cw, nblk, c->nlev, c->nlines, ncell,
+        snprintf(buf, sizeof buf, ":%d:%d:%d:%d:%d:%.17g", fp.cw, fp.nblk, c->nlev, c->nlines, ncell,
                  molpg);
         gkey += buf;
         for (int ln : slot_line) {
@@ -1549,8 +1514,7 @@ extern "C" int rl_trace_lines_forward_ex(rl_ctx *c, int nitems, const rl_item *i
 // flux (and image) are written to the caller's device memory.  The items
 // run as one batch through the forward's kernels; the trajectories of
 // their inclinations must already be resident (built by an earlier
-// allocating call), and no graph or tile trial is made (a tile mapping the
-// autotuner chose earlier for the same batch shape is reused).
+// allocating call), and no graph is made.
 extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_item *items,
                                               double *flux_dev, double *image_dev,
                                               unsigned *warn) {
@@ -1617,25 +1581,10 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
         max_rings = std::max(max_rings, rs.nrings);
         any_skip |= it.skip_mode == RL_SKIP_REFERENCE;
     }
-    // tile mapping: the autotuner's earlier choice for this batch shape, else
-    // ray-major tiles on the persistent grid
-    int dev_cu = 0;
     HIPCHK(c, hipSetDevice(c->device));
-    HIPCHK(c, hipDeviceGetAttribute(&dev_cu, hipDeviceAttributeMultiprocessorCount, c->device));
-    std::string shape = std::to_string(fp64);
-    for (int k = 0; k < nb; k++)
-        shape += ":" + std::to_string(hi[k].nrays) + "x" + std::to_string(hi[k].nfr) + "s" +
-                 std::to_string(hi[k].skip_mode);
-    int cw = 0, nblk = dev_cu * rl::formal_batch_blocks_per_cu(fp64);
-    if (c->fixed_cw >= 0) {
-        cw = c->fixed_cw;
-        if (!c->fixed_persistent) nblk = 0;
-    } else {
-        auto tuned = c->tune.find(shape);
-        if (tuned != c->tune.end()) { cw = tuned->second.first; nblk = tuned->second.second; }
-    }
-    std::vector<long long> t0(nb + 1, 0);
-    for (int k = 0; k < nb; k++) t0[k + 1] = t0[k] + tiles_of(cw, hi[k].nrays, hi[k].nfr);
+    FormalPlan fp;
+    std::vector<long long> u0;
+    if (int e = formal_plan(c, fp64, hi, fp, u0)) return e;
     // the workspace layout, every part 256-byte aligned
     size_t used = 0;
     auto carve = [&](size_t bytes) {
@@ -1653,8 +1602,7 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
     const size_t o_maser = carve((size_t)((nb + 1) / 2) * 8);
     const size_t o_counter = carve(8);
     const size_t o_items = carve((size_t)nb * sizeof(rl::ItemDev));
-    const size_t o_tile0 = carve((size_t)(nb + 1) * 8);
-    const size_t o_sel = carve((size_t)nb * 4);
+    const size_t o_unit0 = carve((size_t)(nb + 1) * 8);
     // the block records where they still fit; without them every segment is
     // integrated
     const size_t bbytes = (size_t)blk0 * sizeof(rl::BlkRec);
@@ -1684,9 +1632,8 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
     L.flux = flux_dev;
     L.cmask = nullptr;
     L.d2 = (1.0 * 3.08572e18) * (1.0 * 3.08572e18);
-    L.tile0 = reinterpret_cast<const long long *>(ws + o_tile0);
-    L.sel = reinterpret_cast<const int *>(ws + o_sel);
-    L.ntiles = t0[nb];
+    L.unit0 = reinterpret_cast<const long long *>(ws + o_unit0);
+    L.nunits = u0[nb];
     L.ovs = reinterpret_cast<unsigned long long *>(ws + o_ovs);
     L.maser = reinterpret_cast<int *>(ws + o_maser);
     L.counter = reinterpret_cast<unsigned long long *>(ws + o_counter);
@@ -1696,12 +1643,8 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
                              c->stream));
     HIPCHK(c, hipMemcpyAsync(ws + o_items, hi.data(), (size_t)nb * sizeof(rl::ItemDev),
                              hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(ws + o_tile0, t0.data(), (size_t)(nb + 1) * 8,
+    HIPCHK(c, hipMemcpyAsync(ws + o_unit0, u0.data(), (size_t)(nb + 1) * 8,
                              hipMemcpyHostToDevice, c->stream));
-    std::vector<int> sel(nb);
-    for (int k = 0; k < nb; k++) sel[k] = k;
-    HIPCHK(c, hipMemcpyAsync(ws + o_sel, sel.data(), (size_t)nb * 4, hipMemcpyHostToDevice,
-                             c->stream));
     rl::launch_zero_u64(c->stream, L.ovs, nb);
     rl::launch_zero_u64(c->stream, reinterpret_cast<unsigned long long *>(L.maser), (nb + 1) / 2);
     for (size_t q = 0; q < slot_line.size(); q++) {
@@ -1716,7 +1659,7 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
     HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
     rl::launch_batch_nodes(c->stream, fp64, L);
     HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
-    rl::launch_batch_formal(c->stream, fp64, L, cw ? cw : 16, nblk, L.ntiles);
+    rl::launch_batch_formal(c->stream, fp64, L, fp.cw, fp.nblk);
     rl::launch_batch_finish(c->stream, fp64, L);
     HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
     rl::launch_batch_flux(c->stream, L);
@@ -1744,8 +1687,8 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
             warn[k] = (maser[k] ? RL_WARN_MASER : 0u) | (ovs[k] ? RL_WARN_OVERSHOOT : 0u);
     }
     c->counts[2] = (long long)ovs[nb - 1];
-    c->last_cw = cw;
-    c->last_blocks = nblk;
+    c->last_cw = c->fixed_cw > 0 ? c->fixed_cw : 0;
+    c->last_blocks = fp.nblk;
     c->last_batches = 1;
     return 0;
 }
@@ -1904,16 +1847,13 @@ extern "C" int rl_set_option(rl_ctx *c, int option, int value) {
     if (!c) return RL_E_ARG;
     switch (option) {
         case RL_OPT_GRAPH: c->use_graph = value != 0; return 0;
-        case RL_OPT_AUTOTUNE: c->autotune = value != 0; if (!value) c->tune.clear(); return 0;
+        case RL_OPT_AUTOTUNE: return 0;      // accepted: there is nothing to time
         case RL_OPT_TILE:
             if (value != 0 && value != 16 && value != 32 && value != 64)
                 return fail(c, RL_E_ARG, "rl_set_option: tile mapping must be 0, 16, 32 or 64");
-            c->tune.clear();
-            c->autotune = false;
             c->fixed_cw = value;
             return 0;
         case RL_OPT_PERSISTENT:
-            c->tune.clear();
             c->fixed_persistent = value != 0;
             return 0;
         case RL_OPT_CKPT:

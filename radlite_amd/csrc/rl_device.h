@@ -213,6 +213,12 @@ __device__ inline void clever_elem(const LineK<T> &L, Acc<T, AFF> &acc, T ds,
                 T f0 = -sleft / lg_ds, f1 = (ds - sleft) / lg_ds;
                 if (f0 > T(0) && f0 < T(40)) ilo = max(1, (int)f0);
                 if (f1 > T(-10) && f1 < T(40)) ihi = min(31, (int)f1 + 2);
+                // the margins that are not used, cut here: a wave's loop is as
+                // long as its longest lane's points
+                for (int q = 0; q < 2; q++) {
+                    if (!(sleft + T(ilo - 1) * lg_ds > T(0))) ilo++;
+                    if (!(sleft + T(ihi - 1) * lg_ds < ds)) ihi--;
+                }
             }
             for (int i = ilo; i <= ihi; i++) {
                 T s = sleft + T(i - 1) * lg_ds;
@@ -579,17 +585,17 @@ __device__ inline void carry_of(const LineK<T> &L, const NodeRec<T> &p, const No
 // the maser flag
 template <typename T, bool AFF>
 __device__ inline void segment_exact(const LineK<T> &L, Acc<T, AFF> &x, const NodeRec<T> &a,
-                                     const NodeRec<T> &b, T istar, T starfract, Carry<T> &c,
+                                     const NodeRec<T> &b, const double *istar, T starfract, Carry<T> &c,
                                      int &ovs, int &maser) {
     T ds = b.ds;
     const int fl = (int)b.flag;
     if (fl & NF_RESET) { ds = T(0); c.init = 1; }
     if (fl & NF_BLEND) {
-        x.map(T(1) - starfract, starfract * istar);
+        x.map(T(1) - starfract, starfract * (T)*istar);
         c.init = 1;
     }
     if (fl & NF_STAR) {
-        x.map(T(0), istar);
+        x.map(T(0), (T)*istar);
         c.init = 1;
     }
     clever_elem<T>(L, x, ds, pt_of(a), pt_of(b), a.lw, b.lw, c, ovs);

@@ -79,9 +79,8 @@ struct BatchLaunch {
     double *image, *partial, *flux;
     unsigned char *cmask;      // optional [image layout]: 1 where integrated
     double d2;
-    const int *sel;            // device [nitems] the items' indices
-    const long long *tile0;    // device [nitems+1] first tile of each item
-    long long ntiles;
+    const long long *unit0;    // device [nitems+1] first unit (ray, channel chunk) of each item
+    long long nunits;
     unsigned long long *ovs, *counter;
     int *maser;
 };
@@ -98,16 +97,17 @@ void launch_segrec(hipStream_t st, long long nnodes, const long long *off, int n
 constexpr size_t SCRATCH_BYTES = (size_t)256 << 20;
 constexpr int SCRATCH_MAX_DEVICES = 64;
 hipError_t scratch_attach(int device, void **out);
-// nblocks == 0: static grid over the first ntiles tiles; > 0: persistent
-// grid of nblocks blocks taking tiles from the work counter
-void launch_batch_formal(hipStream_t st, int fp64, const BatchLaunch &b, int cw, int nblocks,
-                         long long ntiles);
+// cw: the channels of a unit's chunk (at most formal_chunk()); nblocks == 0:
+// one block per unit; > 0: persistent grid of nblocks blocks taking units from
+// the work counter
+void launch_batch_formal(hipStream_t st, int fp64, const BatchLaunch &b, int cw, int nblocks);
+int formal_chunk();
 void launch_batch_finish(hipStream_t st, int fp64, const BatchLaunch &b);
 void launch_batch_flux(hipStream_t st, const BatchLaunch &b);
 void launch_zero_u64(hipStream_t st, unsigned long long *p, int n);
 void launch_rays_circular(hipStream_t st, int nrings, int nphi, const double *tab, double *x0,
                           double *z0);
-int formal_batch_blocks_per_cu(int fp64);
+int formal_blocks_per_cu(int fp64);
 
 // One item of the adjoint (scaled records of precision T, all channels).
 // A chunk is a range of the ray set's rays: nrays, nnodes and every

@@ -10,9 +10,9 @@
 //   k_nodes       one wave per ray: interpolated node records (FP64) +
 //                 the NONREDUNDANT window and continuum channel
 //   k_nodes_fast  the same as scaled records (FP32 mode, adjoint)
-//   k_formal_batch<T> / k_formal_tiles<T>  one lane per (ray, channel) of
-//                 many items: formal solution along the ray (charintline,
-//                 telescope.F:3889-4312)
+//   k_formal<T>   one wave per ray and chunk of channels of many items: formal
+//                 solution along the ray (charintline, telescope.F:3889-4312;
+//                 rl_walk.h)
 //   k_fixup_batch<T>  one thread per ray: the reference's lazy continuum
 //                 copies for skipped channels (telescope.F:583-611)
 //   k_flux_*      ring-weighted sums of the image into the spectrum
@@ -824,12 +824,12 @@ k_nodes_fast(int nrays, const long long *__restrict__ off, const GeoNode *__rest
 // ---------------------------------------------------------------------
 // formal solution
 // ---------------------------------------------------------------------
-// One lane's ray, block by block as the wave walk (rl_walk.h) takes it (blk
-// null: every segment integrated).
+// One lane's ray, block by block, each seen block from its own carry as
+// rl_walk.h takes it (blk null: every segment integrated).
 template <typename T>
 __device__ inline T trace_one(const NodeRec<T> *__restrict__ rec,
                               const BlkRec *__restrict__ blk, int n, const LineK<T> &L,
-                              T I0, T istar, T starfract, int &ovs, int &maser,
+                              T I0, const double *istar, T starfract, int &ovs, int &maser,
                               T *tau = nullptr) {
     Acc<T, false> x{I0, T(1)};
     Carry<T> c;
@@ -873,14 +873,15 @@ __device__ inline double trace_dispatch(const typename RecOf<T>::type *rec,
                                         const BlkRec *blk, const SegHot *hot,
                                         const SegAux *aux, long long b, int ray, int n,
                                         const LineConst &lc, double dnu, double velo,
-                                        double istar, double I0, T sf, int &ovs, int &maser);
+                                        const double *istar, double I0, T sf, int &ovs,
+                                        int &maser);
 
 template <>
 __device__ inline double trace_dispatch<double>(const NodeRec<double> *rec,
                                                 const BlkRec *blk, const SegHot *,
                                                 const SegAux *, long long b, int ray, int n,
                                                 const LineConst &lc, double dnu, double velo,
-                                                double istar, double I0, double sf, int &ovs,
+                                                const double *istar, double I0, double sf, int &ovs,
                                                 int &maser) {
     LineK<double> L;
     L.nu0 = lc.nu0; L.c_aa = lc.c_aa; L.hknu = lc.hknu;
@@ -895,10 +896,10 @@ __device__ inline double trace_dispatch<float>(const NodeLine *rec,
                                                const BlkRec *blk, const SegHot *hot,
                                                const SegAux *aux, long long b, int ray, int n,
                                                const LineConst &, double, double velo,
-                                               double istar, double I0, float sf, int &ovs,
+                                               const double *istar, double I0, float sf, int &ovs,
                                                int &maser) {
     return trace_split(hot + b, aux + b, rec + b, blk ? blk + blk_of(b, ray) : nullptr, n,
-                       (float)velo, I0, (float)istar, sf, ovs, maser);
+                       (float)velo, I0, istar, sf, ovs, maser);
 }
 
 // image placeholder of a channel left out by NONREDUNDANT skipping (a NaN
@@ -993,7 +994,7 @@ k_formal_posvel(int nrays, int nfr, int nx, int ny, const long long *__restrict_
                 L.nu0 = lc.nu0; L.c_aa = lc.c_aa; L.hknu = lc.hknu;
                 L.A = lc.A; L.Bud = lc.Bud; L.Bdu = lc.Bdu;
                 L.dnu = dnu[ch]; L.uch = velo[ch];
-                I = trace_one<double>(rec + b, nullptr, n, L, i0[ch], istar[ch], 0.0, ovs, maser, &t);
+                I = trace_one<double>(rec + b, nullptr, n, L, i0[ch], istar + ch, 0.0, ovs, maser, &t);
             } else {
                 FastLine L{(float)lc.nu0, (float)dnu[ch], (float)velo[ch]};
                 float tf = 0.0f;
@@ -1153,16 +1154,16 @@ __device__ inline const BlkRec *blk_ptr(const void *blk_all, long long blk0) {
     return blk_all ? reinterpret_cast<const BlkRec *>(blk_all) + blk0 : nullptr;
 }
 
-// One wave's tile: 64/cw rays of an item and cw consecutive channels of
-// each, lane -> (ray rb*rows + lane/cw, channel cc*cw + lane%cw).  Every lane
-// of make_image_circular's loop (telescope.F:550-613) is integrated, or marked
+// The formal solution of many items (rl_walk.h): a block takes one ray and one
+// chunk of its channels at a time, the unit u of the launch's list (f.unit0[k]
+// the first of item k, chunks of a ray together).  Every channel of
+// make_image_circular's loop (telescope.F:550-613) is integrated, or marked
 // for the lazy-continuum pass where NONREDUNDANT skipping leaves it out.
 struct FormalBatch {
     const ItemDev *items;
-    const int *sel;              // the launch's items
-    const long long *tile0;      // first tile of each of them
-    int nsel, cw;
-    long long ntiles;
+    const long long *unit0;      // first unit of each item
+    int nitems, cw;              // cw: channels of a chunk
+    long long nunits;
     const void *rec, *blk;
     const RayInfo *rinfo;
     const double *chan;
@@ -1170,153 +1171,139 @@ struct FormalBatch {
     unsigned long long *ovs;
     int *maser;
     unsigned char *cmask;
-    unsigned long long *counter;
+    unsigned long long *counter; // null: one unit per block
 };
 
-// the launch's item of tile t: the last with tile0 <= t
-__device__ inline int tile_item(const FormalBatch &f, long long t) {
-    int lo = 0, hi = f.nsel;
+// the item of unit u: the last with unit0 <= u
+__device__ inline int unit_item(const FormalBatch &f, long long u) {
+    int lo = 0, hi = f.nitems;
     while (hi - lo > 1) {
         const int m = (lo + hi) >> 1;
-        if (f.tile0[m] <= t) lo = m; else hi = m;
+        if (f.unit0[m] <= u) lo = m; else hi = m;
     }
     return lo;
 }
 
-// Tile t: part `part` of `parts` of its rays' blocks (the intensity for one
-// part; else the part's map I -> P I + B, I0 the outer boundary's).  Returns
-// whether the lane has a (ray, channel) to write at image index ix, integrated
-// (doit) or to be marked.
-template <typename T, bool AFF>
-__device__ __forceinline__ bool formal_tile(const FormalBatch &f, WalkLds<T> &lds, long long t,
-                                            int part, int parts, int &item, int &ray, int &ch,
-                                            long long &ix, bool &doit, double &I, double &P,
-                                            double &I0, int &ovs, int &maser) {
-    const int lane = threadIdx.x & 63, cw = f.cw, cwl = 31 - __clz(cw);
-    const int lo = tile_item(f, t);
-    item = f.sel[lo];
+template <typename T>
+__device__ __forceinline__ void formal_unit(const FormalBatch &f, WalkLds<T> &lds, long long u) {
+    constexpr int G = GROUPS;
+    const int lane = threadIdx.x;
+    const int item = unit_item(f, u);
     const ItemDev &it = f.items[item];
-    const int chunks = (it.nfr + cw - 1) >> cwl;
-    const long long lt = t - f.tile0[lo], rb = lt / chunks;
-    ray = (int)(rb << (6 - cwl)) + (lane >> cwl);
-    ch = (int)(lt - rb * chunks) * cw + (lane & (cw - 1));
-    const bool on = ray < it.nrays && ch < it.nfr;
-    const int rc = min(ray, it.nrays - 1), cc = min(ch, it.nfr - 1);
-    const RayInfo ri = f.rinfo[it.rinfo0 + rc];
+    const int chunks = (it.nfr + f.cw - 1) / f.cw;
+    const long long lu = u - f.unit0[item];
+    const int ray = (int)(lu / chunks), q = (int)(lu - (long long)ray * chunks);
+    const int width = (it.nfr + chunks - 1) / chunks;
     const double *dnu = f.chan + it.chan0, *velo = dnu + it.nfr, *istar = dnu + 2 * it.nfr,
                  *i0 = dnu + 3 * it.nfr;
-    const double v = velo[cc];
-    doit = on;
-    if (it.skip_mode == 0 && rc > 0 && cc > 0 && cc != ri.cont)
-        doit = doit && v <= (double)ri.mx + it.aks2 && v >= (double)ri.mn - it.aks2;
-    const long long b = it.off[rc];
-    // the ray's blocks of this part
-    const int n = ray < it.nrays ? ri.n : 0, nb = n < 2 ? 0 : (n + BLK - 1) >> BLK_LOG;
-    const int j0 = nb * part / parts, j1 = nb * (part + 1) / parts;
-    const BlkRec *blk = f.blk ? reinterpret_cast<const BlkRec *>(f.blk) + it.blk0 + blk_of(b, rc)
+    Chans ch;
+    ch.velo = velo;
+    ch.c0 = min(q * width, it.nfr);
+    ch.c1 = min(ch.c0 + width, it.nfr);
+    ch.ng = (ch.c1 - ch.c0 + 63) >> 6;
+    if (ch.c0 >= ch.c1) return;                  // the whole block
+    const RayInfo ri = f.rinfo[it.rinfo0 + ray];
+    const long long b = it.off[ray];
+    const int n = ri.n, nb = n < 2 ? 0 : (n + BLK - 1) >> BLK_LOG;
+    const BlkRec *blk = f.blk ? reinterpret_cast<const BlkRec *>(f.blk) + it.blk0 + blk_of(b, ray)
                               : nullptr;
-    I0 = i0[cc];
-    const T sf = rc == 0 ? (T)it.lc.starfract : T(0);
+    auto doit = [&](int c) {
+        if (it.skip_mode != 0 || ray == 0 || c == 0 || c == ri.cont) return true;
+        const double v = velo[c];
+        return v <= (double)ri.mx + it.aks2 && v >= (double)ri.mn - it.aks2;
+    };
+    const T sf = ray == 0 ? (T)it.lc.starfract : T(0);
+    int ovs = 0, maser = 0;
+    double I[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) I[g] = i0[min(ch.c0 + 64 * g + lane, it.nfr - 1)];
+    unsigned over = 0;
     if constexpr (std::is_same<T, double>::value) {
-        LineK<double> L;
-        L.nu0 = it.lc.nu0; L.c_aa = it.lc.c_aa; L.hknu = it.lc.hknu;
-        L.A = it.lc.A; L.Bud = it.lc.Bud; L.Bdu = it.lc.Bdu;
-        L.dnu = dnu[cc]; L.uch = v;
-        Acc<double, AFF> x{AFF ? 0.0 : I0, 1.0};
-        walk_exact<AFF>(lds, cwl, reinterpret_cast<const NodeRec<double> *>(f.rec) + it.rec0 + b,
-                        blk, n, j0, j1, doit, L, x, istar[cc], sf, ovs, maser);
-        I = x.I;
-        P = x.P;
+        const float4 *rec =
+            reinterpret_cast<const float4 *>(reinterpret_cast<const NodeRec<double> *>(f.rec) +
+                                             it.rec0 + b);
+        walk<double>(
+            lds, blk, nb, ch, I, over,
+            [&](int j, int piece) __attribute__((always_inline)) {
+                const int k = min(max((j << BLK_LOG) - 2 + (piece >> 2), 0), n - 1);
+                return rec[(size_t)k * 4 + (piece & 3)];
+            },
+            [&](int c) __attribute__((always_inline)) { return double2{velo[c], dnu[c]}; },
+            [&](const float4 *st, int j, int c, double2 v) __attribute__((always_inline)) {
+                if (!doit(c)) return Map{1.0, 0.0};
+                LineK<double> L;
+                L.nu0 = it.lc.nu0; L.c_aa = it.lc.c_aa; L.hknu = it.lc.hknu;
+                L.A = it.lc.A; L.Bud = it.lc.Bud; L.Bdu = it.lc.Bdu;
+                L.dnu = v.y;
+                L.uch = v.x;
+                return block_exact(st, j, n, L, istar + c, sf, ovs, maser);
+            },
+            [&](int g, int nov) __attribute__((always_inline)) {
+                const int c = ch.c0 + 64 * g + lane;
+                if (c < ch.c1 && doit(c)) ovs += nov;
+            });
     } else {
         const char *base = static_cast<const char *>(f.rec);
-        Acc32<AFF> x{AFF ? 0.0 : I0, 1.0};
-        bool ovf = false;
-        walk_split<AFF>(lds, cwl, reinterpret_cast<const SegHot *>(base + it.hot_off) + b,
-                        reinterpret_cast<const SegAux *>(base + it.aux_off) + b,
-                        reinterpret_cast<const NodeLine *>(f.rec) + it.rec0 + b, blk, n, j0, j1,
-                        doit, (float)v, x, (float)istar[cc], sf, ovf, maser);
-        I = x.I;
-        P = x.P;
-        ovs += ovf ? 1 : 0;
+        const float4 *hot = reinterpret_cast<const float4 *>(base + it.hot_off) + b;
+        const float4 *aux = reinterpret_cast<const float4 *>(base + it.aux_off) + b;
+        const float4 *line = reinterpret_cast<const float4 *>(f.rec) + it.rec0 + b;
+        walk<float>(
+            lds, blk, nb, ch, I, over,
+            [&](int j, int piece) __attribute__((always_inline)) {
+                constexpr int N = Nodes<float>::N;
+                const int w = piece < N ? piece : (piece < 2 * N ? piece - N : piece - 2 * N);
+                const int k = min(max((j << BLK_LOG) - 1 + w, 0), n - 1);
+                return (piece < N ? hot : (piece < 2 * N ? aux : line))[k];
+            },
+            [&](int c) __attribute__((always_inline)) { return (float)velo[c]; },
+            [&](const float4 *st, int j, int c, float v) __attribute__((always_inline)) {
+                if (!doit(c)) return Map{1.0, 0.0};
+                return block_split(st, j, n, v, istar + c, sf, maser);
+            },
+            [&](int g, int) __attribute__((always_inline)) { over |= 1u << g; });
     }
-    ix = it.img0 + (long long)ray * it.nfr + ch;
-    return on;
-}
-
-// a finished lane's image value and mask, and the wave's warnings
-__device__ inline void formal_write(const FormalBatch &f, int item, int ray, int ch, bool on,
-                                    bool doit, long long ix, double I, int ovs, int maser) {
-    const ItemDev &it = f.items[item];
-    if (on) {
-        f.image[ix] = doit ? I : __longlong_as_double(SKIPPED_BITS);   // filled by k_fixup
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        const int c = ch.c0 + 64 * g + lane;
+        if (c >= ch.c1) continue;
+        const bool on = doit(c);
+        const long long ix = it.img0 + (long long)ray * it.nfr + c;
+        f.image[ix] = on ? I[g] : __longlong_as_double(SKIPPED_BITS);    // filled by k_fixup
         if (f.cmask)
-            f.cmask[ix] = window_mask(ray, ch, f.rinfo + it.rinfo0, f.chan + it.chan0 + it.nfr,
-                                      it.aks2, it.skip_mode);
+            f.cmask[ix] = window_mask(ray, c, f.rinfo + it.rinfo0, velo, it.aks2, it.skip_mode);
+        if (on && ((over >> g) & 1)) ovs++;
     }
     for (int m = 32; m >= 1; m >>= 1) {
         ovs += __shfl_xor(ovs, m);
         maser |= __shfl_xor(maser, m);
     }
-    if ((threadIdx.x & 63) == 0) {
+    if (lane == 0) {
         if (ovs) atomicAdd(f.ovs + item, (unsigned long long)ovs);
         if (maser) atomicOr(f.maser + item, 1);
     }
 }
 
-// Persistent formal solution over all tiles of the launch's items: each wave
-// takes the next tile from a device counter until every tile is taken, so the
-// grid drains by itself; items of any size share the machine.
 template <typename T>
-__device__ __forceinline__ void formal_batch_body(const FormalBatch &f) {
-    __shared__ WalkLds<T> lds[4];
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? FORMAL32_WAVES : FORMAL64_WAVES)))
+k_formal(FormalBatch f) {
+    __shared__ WalkLds<T> lds;
+    // a unit per block, or (persistent) units from a device counter until all
+    // are taken, so the grid drains by itself
+    unsigned long long u = blockIdx.x;
     for (;;) {
-        // Every lane executes the atomic (lane 0 adds 1, the others 0) and the
-        // tile index is lane 0's result through readfirstlane, so it is
-        // wave-uniform (an SGPR) and the loop exit is a scalar branch.  A
-        // lane-0-only atomic broadcast with a shuffle leaves the exit
-        // condition divergent to the compiler, which may then iterate the
-        // other lanes without lane 0.
-        const unsigned long long mine = atomicAdd(f.counter, (threadIdx.x & 63) == 0 ? 1ull : 0ull);
-        const unsigned lo32 = __builtin_amdgcn_readfirstlane((unsigned)(mine & 0xffffffffull));
-        const unsigned hi32 = __builtin_amdgcn_readfirstlane((unsigned)(mine >> 32));
-        const unsigned long long t = ((unsigned long long)hi32 << 32) | lo32;
-        if (t >= (unsigned long long)f.ntiles) break;
-        int item, ray, ch, ovs = 0, maser = 0;
-        long long ix;
-        bool doit;
-        double I, P, I0;
-        const bool on = formal_tile<T, false>(f, lds[threadIdx.x >> 6], (long long)t, 0, 1, item,
-                                              ray, ch, ix, doit, I, P, I0, ovs, maser);
-        formal_write(f, item, ray, ch, on, doit, ix, I, ovs, maser);
+        if (f.counter) {
+            // Every lane executes the atomic (lane 0 adds 1, the others 0), and
+            // lane 0's result through readfirstlane is wave-uniform, so that
+            // the loop's exit is a scalar branch.
+            const unsigned long long mine = atomicAdd(f.counter, threadIdx.x == 0 ? 1ull : 0ull);
+            const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)mine);
+            const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(mine >> 32));
+            u = (unsigned long long)hi << 32 | lo;
+        }
+        if (u >= (unsigned long long)f.nunits) break;
+        formal_unit<T>(f, lds, (long long)u);
+        if (!f.counter) break;
     }
-}
-
-// FP64 (the primary template; FP32 is specialised below)
-template <typename T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-k_formal_batch(FormalBatch f) {
-    formal_batch_body<T>(f);
-}
-template <>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FORMAL32_WAVES)))
-k_formal_batch<float>(FormalBatch f) {
-    formal_batch_body<float>(f);
-}
-
-// The same tiles on a static grid: wave w of block b takes tile 4b + w.
-template <typename T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? FORMAL32_WAVES : 4)))
-k_formal_tiles(FormalBatch f) {
-    __shared__ WalkLds<T> lds[4];
-    const long long t = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= f.ntiles) return;                     // whole waves
-    int item, ray, ch, ovs = 0, maser = 0;
-    long long ix;
-    bool doit;
-    double I, P, I0;
-    const bool on = formal_tile<T, false>(f, lds[threadIdx.x >> 6], t, 0, 1, item, ray, ch, ix,
-                                          doit, I, P, I0, ovs, maser);
-    formal_write(f, item, ray, ch, on, doit, ix, I, ovs, maser);
 }
 
 template <typename T>
@@ -1348,7 +1335,7 @@ __global__ void k_fixup_batch(const ItemDev *__restrict__ items, const void *rec
                                         seg_ptr<SegHot>(rec_all, it.hot_off),
                                         seg_ptr<SegAux>(rec_all, it.aux_off), it.off[ray], ray,
                                         ri.n, it.lc, dnu[ch],
-                                        velo[ch], istar[ch], i0[ch], T(0), ovs, maser);
+                                        velo[ch], istar + ch, i0[ch], T(0), ovs, maser);
             cont = row[ch];
         }
     }
@@ -1395,19 +1382,15 @@ void launch_batch_nodes(hipStream_t st, int fp64, const BatchLaunch &b) {
                            b.rec, b.blk, b.rinfo, b.chan);
 }
 
-void launch_batch_formal(hipStream_t st, int fp64, const BatchLaunch &b, int cw, int nblocks,
-                         long long ntiles) {
-    const FormalBatch f{b.items, b.sel, b.tile0, b.nitems, cw, ntiles, b.rec, b.blk, b.rinfo,
-                        b.chan, b.image, b.ovs, b.maser, b.cmask, b.counter};
-    if (nblocks == 0) {           // static grid
-        const unsigned g = (unsigned)((ntiles + 3) / 4);
-        if (fp64) hipLaunchKernelGGL(k_formal_tiles<double>, dim3(g), dim3(256), 0, st, f);
-        else hipLaunchKernelGGL(k_formal_tiles<float>, dim3(g), dim3(256), 0, st, f);
-        return;
-    }
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, b.counter, 1);
-    if (fp64) hipLaunchKernelGGL(k_formal_batch<double>, dim3(nblocks), dim3(256), 0, st, f);
-    else hipLaunchKernelGGL(k_formal_batch<float>, dim3(nblocks), dim3(256), 0, st, f);
+void launch_batch_formal(hipStream_t st, int fp64, const BatchLaunch &b, int cw, int nblocks) {
+    // a launch holds fewer than 2^32 threads
+    if (nblocks == 0 && b.nunits * 64 >= 1ll << 31) nblocks = 1 << 16;
+    const FormalBatch f{b.items, b.unit0, b.nitems, cw, b.nunits, b.rec, b.blk, b.rinfo, b.chan,
+                        b.image, b.ovs, b.maser, b.cmask, nblocks > 0 ? b.counter : nullptr};
+    const unsigned grid = (unsigned)(nblocks > 0 ? nblocks : b.nunits);
+    if (nblocks > 0) hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, b.counter, 1);
+    if (fp64) hipLaunchKernelGGL(k_formal<double>, dim3(grid), dim3(64), 0, st, f);
+    else hipLaunchKernelGGL(k_formal<float>, dim3(grid), dim3(64), 0, st, f);
 }
 
 void launch_batch_finish(hipStream_t st, int fp64, const BatchLaunch &b) {
@@ -1463,12 +1446,14 @@ void launch_zero_u64(hipStream_t st, unsigned long long *p, int n) {
     if (n > 0) hipLaunchKernelGGL(k_zero_u64, dim3((n + 255) / 256), dim3(256), 0, st, p, n);
 }
 
-int formal_batch_blocks_per_cu(int fp64) {
+int formal_chunk() { return 64 * GROUPS; }
+
+int formal_blocks_per_cu(int fp64) {
     int nb = 0;
     if (fp64)
-        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_formal_batch<double>, 256, 0);
+        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_formal<double>, 64, 0);
     else
-        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_formal_batch<float>, 256, 0);
+        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_formal<float>, 64, 0);
     return nb > 0 ? nb : 1;
 }
 

@@ -177,32 +177,41 @@ __device__ __forceinline__ void elem_pt32(Acc32<AFF> &x, float hds, const Pt32 &
     x.step(e0, q);
 }
 
-// The general path of segment k (nodes k-1 -> k): node flags (hole chord,
-// central-beam star blend, star intensity: the element then starts afresh
-// from the start point under its own profile) and the sub-grid of
-// clever_integrate_element_linedust (line.F:4706-4800): points s_i =
-// sleft + (i-1) lg, i = 1..31, used where 0 < s_i < ds, the quantities
-// interpolated linearly in s, the width held at the segment's mean.
+// The general path of segment k (nodes k-1 -> k) up to its last element: node
+// flags (hole chord, central-beam star blend, star intensity: the element then
+// starts afresh from the start point under its own profile) and the sub-grid of
+// clever_integrate_element_linedust (line.F:4706-4800): points s_i = sleft +
+// (i-1) lg, i = 1..31, used where 0 < s_i < ds, the quantities interpolated
+// linearly in s, the width held at the segment's mean.  Returns ds; sa: the
+// last point's s.
 template <bool AFF>
-__device__ __forceinline__ void seg_general32(Acc32<AFF> &x, const SegHot &h, float u0, const SegAux &a1,
-                                     const NodeLine &q0, const NodeLine &q1, float uch,
-                                     float istar, float sf, Car32 &c, bool &ovf, int &maser) {
+__device__ __forceinline__ float seg_general32(Acc32<AFF> &x, const SegHot &h, float u0,
+                                      const SegAux &a1, const NodeLine &q0, const NodeLine &q1,
+                                      float uch, const double *istar, float sf, Car32 &c,
+                                      bool &ovf, float &sa) {
     float ds = 2.0f * fabsf(h.hds);                     // (float)ds, hds = (float)(ds/2)
     const int fl = a1.flag;
     if (fl & NF_RESET) ds = 0.0f;
-    if (fl & NF_BLEND) x.map((double)(1.0f - sf), (double)(sf * istar));
-    if (fl & NF_STAR) x.map(0.0, (double)istar);
-    const Pt32 p0 = pt_of(u0, q0), p1 = pt_of(a1.u, q1);
-    if (fl) carry32(p0, uch, h.ag, h.ng, c);
-    float sa = 0.0f, e1 = 0.0f;
+    if (fl & NF_BLEND) x.map((double)(1.0f - sf), (double)(sf * (float)*istar));
+    if (fl & NF_STAR) x.map(0.0, (double)(float)*istar);
+    if (fl) carry32(pt_of(u0, q0), uch, h.ag, h.ng, c);
+    sa = 0.0f;
     if (a1.dls >= 0.0f) {                                 // 6x > 1 (line.F:4715)
-        const float s_c = ds * (uch - p0.u) * a1.inv_du;
+        const float s_c = ds * (uch - u0) * a1.inv_du;
         const float sright = s_c + 3.0f * a1.dls, sleft = s_c - 3.0f * a1.dls;
         if (sright > 0.0f && sleft < ds) {
+            const Pt32 p0 = pt_of(u0, q0), p1 = pt_of(a1.u, q1);
             const float lg = (sright - sleft) * (1.0f / 30.0f);
             const float f0 = FOps<float>::fdiv(-sleft, lg), f1 = FOps<float>::fdiv(ds - sleft, lg);
-            const int ilo = f0 > 0.0f ? max(1, (int)fminf(f0, 40.0f)) : 1;
-            const int ihi = f1 < 40.0f ? min(31, (int)fmaxf(f1, -2.0f) + 2) : 31;
+            int i = f0 > 0.0f ? max(1, (int)fminf(f0, 40.0f)) : 1;
+            int ihi = f1 < 40.0f ? min(31, (int)fmaxf(f1, -2.0f) + 2) : 31;
+            // the bounds are at most two points too wide: cut here, so that a
+            // wave's loop is as long as its longest lane's points
+            auto at = [&](int i) { return sleft + (float)(i - 1) * lg; };
+            i += !(at(i) > 0.0f);
+            i += !(at(i) > 0.0f);
+            ihi -= !(at(ihi) < ds);
+            ihi -= !(at(ihi) < ds);
             // the nodes' scales relative to the larger; where both are below
             // the single-precision range (no optical depth to speak of) the
             // points are weighted equally
@@ -210,8 +219,8 @@ __device__ __forceinline__ void seg_general32(Acc32<AFF> &x, const SegHot &h, fl
             const float rel0 = sm > 0.0f ? p0.sig / sm : 1.0f;
             const float rel1 = sm > 0.0f ? p1.sig / sm : 1.0f;
             const float inv_ds = FOps<float>::fdiv(1.0f, ds);
-            for (int i = ilo; i <= ihi; i++) {
-                const float s = sleft + (float)(i - 1) * lg;
+            for (; i <= ihi; i++) {
+                const float s = at(i);
                 if (s > 0.0f && s < ds) {
                     // linear interpolation of the unscaled quantities
                     // (line.F:4775-4790) through relative weights
@@ -230,41 +239,44 @@ __device__ __forceinline__ void seg_general32(Acc32<AFF> &x, const SegHot &h, fl
             }
         }
     }
-    elem_pt32(x, 0.5f * (ds - sa), p1, uch, h.ag, h.ng, c, ovf, e1);
-    // maser flag (telescope.F:4295-4297): line alpha * ds < -0.01 at the end
-    if (p1.sig * (p1.dcl * h.ng * e1) * ds < -0.01f) maser = 1;
+    return ds;
 }
 
 // segment k from the carry (hot, aux, line: at node k; the general path reads
-// the two before it as well)
+// the node before it as well).  The last (or only) element of every segment is
+// one piece of code: in a wave whose lanes hold both kinds of segment it runs
+// once.
 template <bool AFF>
 __device__ __forceinline__ void segment32(Acc32<AFF> &x, const SegHot *hot, const SegAux *aux,
-                                          const NodeLine *line, float uch, float istar, float sf,
+                                          const NodeLine *line, float uch, const double *istar, float sf,
                                           Car32 &c, bool &ovf, int &maser) {
     const SegHot h = *hot;
     const NodeLine q = *line;
+    float hds = h.hds, ds = 2.0f * h.hds, z = fmaf(uch, h.ag, -h.uag);
     if (seg_general(h.hds)) {
-        seg_general32(x, h, aux[-1].u, load_aux(aux), line[-1], q, uch, istar, sf, c, ovf, maser);
-    } else {
-        const float z = fmaf(uch, h.ag, -h.uag);
-        const float e = ex2(-(z * z));
-        const float dcn = q.dcl * h.ng;
-        float e0, b;
-        elem_map32(h.hds, e, q.jcl * h.ng, dcn, fabsf(q.sig), nl_adh(q.sig), q.jdh, c, ovf, e0, b);
-        x.step(e0, b);
-        // maser flag; the line coefficient is negative only where the
-        // populations are inverted
-        if (q.dcl < 0.0f && fabsf(q.sig) * (dcn * e) * (2.0f * h.hds) < -0.01f) maser = 1;
+        const SegAux a = load_aux(aux);
+        float sa;
+        ds = seg_general32(x, h, aux[-1].u, a, line[-1], q, uch, istar, sf, c, ovf, sa);
+        hds = 0.5f * (ds - sa);
+        z = (uch - a.u) * h.ag;
     }
+    const float e = ex2(-(z * z));
+    const float dcn = q.dcl * h.ng, sig = fabsf(q.sig);
+    float e0, b;
+    elem_map32(hds, e, q.jcl * h.ng, dcn, sig, nl_adh(q.sig), q.jdh, c, ovf, e0, b);
+    x.step(e0, b);
+    // maser flag (telescope.F:4295-4297): line alpha * ds < -0.01 at the end;
+    // the line coefficient is negative only where the populations are inverted
+    if (q.dcl < 0.0f && sig * (dcn * e) * ds < -0.01f) maser = 1;
 }
 
 // charintline (telescope.F:3889-4312) on split records, one lane: one channel
 // (uch = dnu/nu0) of one ray of n nodes from the outer boundary intensity I0,
-// block by block as the wave walk (rl_walk.h) takes it.
+// block by block, each seen block from its own carry as rl_walk.h takes it.
 __device__ inline double trace_split(const SegHot *__restrict__ hot, const SegAux *__restrict__ aux,
                                      const NodeLine *__restrict__ line,
                                      const BlkRec *__restrict__ blk, int n, float uch, double I0,
-                                     float istar, float sf, int &ovs, int &maser) {
+                                     const double *istar, float sf, int &ovs, int &maser) {
     Acc32<false> x{I0, 1.0};
     if (n < 2) return I0;
     Car32 c;

@@ -1,49 +1,66 @@
-// The wave walk of the formal solution: 64/cw rays x cw channels per wave, the
-// rays' records through LDS block by block (rl_blocks.h).
+// The formal solution of one ray, all channels of a chunk, by one wave.
 //
-// A wave's lanes are on the same block of their rays: one whose line none of
-// a ray's lanes can see is one multiply-add, and the others' segments are
-// integrated by the lanes that see them.  (A lane that walked its own list of
-// blocks would meet the sub-gridded segments at another time than its
-// neighbours, and the wave would run through both kinds at every step: 54 ms
-// for the 400 x 200 disk's two inclinations, 50 ms without blocks, 26 ms in
-// step, 19 ms with the records through LDS.)
-// Whether a lane takes a block's map or its segments is the lane's own
-// matter, so results do not depend on which lanes share a wave.
+// Along a ray a channel sees the line in about a tenth of the blocks
+// (rl_blocks.h); in the others every channel takes the block's own map.  So the
+// (block, channel) pairs that see the line, a block's channels consecutive, are
+// taken 64 at a time, a lane each, as a stream along the ray:
 //
-// Sixteen channels per ray (cw = 16) keep the union of what the lanes see
-// small: with T = 1000 K (R/AU)^-1/2 and 200 channels over +-40 km/s the wave
-// integrates 19% of its segments (64 channels: 30%, 32: 28%, a lane alone:
-// 11%).
+//   stage      the nodes of the blocks that the 64 pairs begin, into LDS (the
+//              next blocks' loads are in flight while a batch is integrated)
+//   integrate  each lane its pair's map I -> P I + B, into LDS
+//   compose    a lane per channel: the maps of the blocks now complete, in
+//              order, the pair's where there is one, else the block's own
 //
-// The lanes of a ray load 16 block records at a time, one each, and for a
-// block that is integrated the records of its nodes, a 16-byte piece each, and
-// read them from LDS (broadcasts): three vector loads per lane and block
-// instead of two or more per lane and segment.
+// What bounds it: instruction issue, then the latency of a batch's steps.
+// Lanes that held one (ray, channel) each and met at every block that one of 16
+// channels saw had work in 38% of their instructions, and a ray of many blocks
+// was one serial chain; packed pairs fill 68%, and their chains are a block
+// long.  One launch, 400 x 200 disk, two inclinations, FP32: 19.3 -> 16.1 ms;
+// 200 x 100 disk, FP64: 4.8 -> 3.1 ms; 100 x 60 disk, FP64: 0.96 -> 0.40 ms;
+// 97 x 61 disk, FP32: 0.62 -> 0.27 ms.  (A wave per eighth of a ray, for
+// launches of few rays: 14 of 64 lanes with work, 1.22 ms for the 100 x 60
+// disk.  Without the loads in flight ahead of a batch: 19.0 against 16.1 ms.)
+//
+// A channel's maps are the same whatever else its wave holds, and are applied
+// one by one: results do not depend on chunks, batches or the launch.
 #pragma once
 #include "rl_device.h"
 #include "rl_fwd32.h"
 
 namespace rl {
 
-constexpr int WALK_WIN = 16;                // block records held at a time
-// waves per SIMD of the FP32 kernels: at 8 (64 registers) 36 values spill, the
-// sub-grid path's among them (400 x 200 disk 19.9 against 19.2 ms, 97 x 61
-// disk 0.68 against 0.63)
-constexpr int FORMAL32_WAVES = 6;
+// waves per SIMD that the kernels' registers are held to: FP32 in five, with
+// chunks of 128 channels, spilled in the element loop (22.9 against 19.0 ms for
+// the 400 x 200 disk); FP64 in two did not spill but waited (3.96 against 3.69
+// ms, 200 x 100 disk)
+constexpr int FORMAL32_WAVES = 4, FORMAL64_WAVES = 3;
 
-template <typename T> struct WalkLds;
-// nodes k0-1 .. k0+BLK-1 of a ray (clamped to the ray): SegHot, SegAux, NodeLine
-template <> struct WalkLds<float> {
-    static constexpr int N = BLK + 1;
-    BlkRec win[4][WALK_WIN];
-    float4 st[4][3 * N];
+// block records held at a time (a lane each); blocks whose nodes are in LDS, and
+// of these, those that one batch of pairs takes
+constexpr int RECS = 64, SLOTS = 11, BATCH_BLOCKS = 7;
+// a chunk has up to GROUPS groups of 64 channels: a ray's records are read once
+// per chunk, and the ring of a chunk's pairs leaves room for the four waves
+constexpr int GROUPS = 4;
+
+template <typename T> struct Nodes;
+// nodes k0-1 .. k0+BLK-1 of a block (clamped to the ray): SegHot, SegAux, NodeLine
+template <> struct Nodes<float> {
+    static constexpr int N = BLK + 1, PIECES = 3 * N, AHEAD = 128 / PIECES;
 };
 // nodes k0-2 .. k0+BLK-1
-template <> struct WalkLds<double> {
-    static constexpr int N = BLK + 2;
-    BlkRec win[4][WALK_WIN];
-    NodeRec<double> st[4][N];
+template <> struct Nodes<double> {
+    static constexpr int N = BLK + 2, PIECES = 4 * N, AHEAD = 128 / PIECES;
+};
+
+struct Map {
+    double P, B;
+};
+
+// one wave's share of LDS
+constexpr int RING = 64 * GROUPS + 64;                 // a chunk's pairs of one block + 64
+template <typename T> struct WalkLds {
+    Map map[RING];                                     // pair p at p % RING
+    float4 st[SLOTS][Nodes<T>::PIECES];
 };
 
 // LDS written by a wave's lanes is read by its other lanes: LDS operations
@@ -54,149 +71,216 @@ __device__ inline void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// the four 16-bit fields of a ballot over rays of 1 << cwl lanes, combined
-__device__ inline unsigned fold16(unsigned long long m, int cwl) {
-    unsigned r = (unsigned)m;
-    if (cwl < 6) r |= (unsigned)(m >> 32);
-    if (cwl < 5) r |= r >> 16;
-    return r & 0xffffu;
+__device__ inline int lane_of(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+__device__ inline double lane_of(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// FP32: the sign of a map's factor (never negative) marks an overshoot
+__device__ inline double mark(double P, bool ovf) { return copysign(P, ovf ? -1.0 : 1.0); }
+__device__ inline bool marked(double P) { return __double2hiint(P) < 0; }
+
+// the first channel of [c0, c1) whose velocity is not below x (above: not at or
+// below it), v ascending; est: its position if the channels were exactly even
+template <typename T>
+__device__ inline int channel_of(const double *__restrict__ v, int c0, int c1, float x, bool above,
+                                 T est) {
+    int c = (int)fmin(fmax(est, (T)c0), (T)c1);
+    const T b = (T)x;
+    auto before = [&](int k) { const T u = (T)v[k]; return above ? u <= b : u < b; };
+    while (c > c0 && !before(c - 1)) c--;
+    while (c < c1 && before(c)) c++;
+    return c;
 }
 
-// The blocks [j0, j1) of each ray.  free(A, B, overshoots): the lane takes the
-// block's map; stage(j): the ray's lanes load block j's nodes into LDS (called
-// for the rays that have a block j); integrate(j): the lane integrates it.
-// on: the lane has a channel to integrate; blk null: no block is free.
-template <typename T, typename Free, typename Stage, typename Integrate>
-__device__ __forceinline__ void walk(BlkRec (*win)[WALK_WIN], int cwl,
-                                     const BlkRec *__restrict__ blk, int j0, int j1, bool on,
-                                     float ulo, float uhi, T uch, const Free &free,
-                                     const Stage &stage, const Integrate &integrate) {
-    const int lane = threadIdx.x & 63, g = lane >> cwl, li = lane & ((1 << cwl) - 1);
-    // the ray's channels
-    if (!on) { ulo = INFINITY; uhi = -INFINITY; }
-    for (int m = 1; m < (1 << cwl); m <<= 1) {
-        ulo = fminf(ulo, __shfl_xor(ulo, m));
-        uhi = fmaxf(uhi, __shfl_xor(uhi, m));
-    }
-    for (int jw = j0; __any(jw < j1); jw += WALK_WIN) {
-        const bool act = li < WALK_WIN && jw + li < j1;
-        float lo = INFINITY, hi = -INFINITY;          // no block: the identity, free
-        double A = 1.0, B = 0.0;
-        if (act) {
-            lo = -INFINITY;
-            hi = INFINITY;
+// the channels of a chunk as a wave holds them
+struct Chans {
+    const double *velo;
+    int c0, c1, ng;             // [c0, c1), groups of 64
+};
+
+// The nb blocks of a ray: I[g] the intensity of channel c0 + 64 g + lane; over:
+// FP32, bit g set on an overshoot.  stage(j, piece): a piece of block j's
+// nodes; before(c): what channel c needs, loaded while the nodes arrive;
+// integrate(nodes, j, c, that): the map of block j for channel c; passed(g,
+// n): n overshoots of a block's own map.
+template <typename T, typename Stage, typename Before, typename Integrate,
+          typename Free>
+__device__ __forceinline__ void walk(WalkLds<T> &S, const BlkRec *__restrict__ blk, int nb,
+                                     const Chans &ch, double (&I)[GROUPS], unsigned &over,
+                                     const Stage &stage, const Before &before,
+                                     const Integrate &integrate, const Free &passed) {
+    using Pre = decltype(before(0));
+    constexpr int G = GROUPS;
+    const int lane = threadIdx.x & 63;
+    const T v0 = (T)ch.velo[ch.c0], v1 = (T)ch.velo[ch.c1 - 1];
+    const T inv = ch.c1 - ch.c0 > 1 ? (T)(ch.c1 - 1 - ch.c0) / (v1 - v0) : T(0);
+    const unsigned long long upto = (2ull << lane) - 1;
+    for (int jw = 0; jw < nb; jw += RECS) {
+        const int m = min(RECS, nb - jw);
+        // the blocks' records and channel ranges, a lane each
+        int cl = ch.c0, cnt = 0, nov = 0;
+        double bA = 1.0, bB = 0.0;
+        if (lane < m) {
+            float lo = -INFINITY, hi = INFINITY;
             if (blk) {
-                const BlkRec *r = blk + jw + li;
-                lo = r->lo; hi = r->hi; A = r->A; B = r->B;
+                const BlkRec *r = blk + jw + lane;
+                lo = r->lo; hi = r->hi; bA = r->A; bB = r->B;
+                nov = __float_as_int(lo) & (2 * BLK - 1);
             }
+            if (!(lo > hi)) {        // (-inf with an overshoot count is NaN)
+                cl = channel_of<T>(ch.velo, ch.c0, ch.c1, lo, false,
+                                   (T)ch.c0 + ((T)lo - v0) * inv);
+                cnt = max(0, channel_of<T>(ch.velo, ch.c0, ch.c1, hi, true,
+                                           (T)ch.c0 + ((T)hi - v0) * inv + T(1)) - cl);
+            }
+        }
+        int incl = cnt;                          // pairs up to and with the lane's block
+        for (int d = 1; d < RECS; d <<= 1) {
+            const int t = __shfl_up(incl, d);
+            if (lane >= d) incl += t;
+        }
+        const int st = incl - cnt, total = lane_of(incl, m - 1);
+        const bool some = cnt > 0, overs = __any(nov != 0);
+        // the blocks with pairs that are not in LDS yet, and of these the first
+        // `ahead` whose nodes are in registers (slots by rank)
+        unsigned long long rest = __ballot(some);
+        const int rank = __popcll(rest & (upto >> 1));
+        int staged = 0, ahead = 0;
+        float4 piece[2];
+        auto load = [&]() __attribute__((always_inline)) {
+            unsigned long long r = rest;
+            int j[Nodes<T>::AHEAD];
+            ahead = 0;
+#pragma unroll
+            for (int k = 0; k < Nodes<T>::AHEAD; k++) {
+                j[k] = __ffsll(r) - 1;
+                ahead += r != 0;
+                r &= r - 1;
+            }
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const int p = lane + 64 * q, k = p / Nodes<T>::PIECES;
+                int jk = j[0];
+#pragma unroll
+                for (int i = 1; i < Nodes<T>::AHEAD; i++) jk = k == i ? j[i] : jk;
+                if (k < ahead) piece[q] = stage(jw + jk, p - k * Nodes<T>::PIECES);
+            }
+        };
+        load();
+        for (int p0 = 0, b = 0; b < m;) {
+            int pend = total;
+            if (p0 < total) {
+                // the pairs p0 .. pend-1 of at most BATCH_BLOCKS blocks: the one
+                // that holds p0 (lane l0) and those that begin after it
+                const int l0 = 63 - __clzll(__ballot(some && st <= p0));
+                unsigned long long more = __ballot(some && st > p0 && st < p0 + 64);
+                pend = min(p0 + 64, total);
+                const int p = p0 + lane, r0 = lane_of(rank, l0);
+                int r = r0, r1 = r0, j = l0, c = lane_of(cl, l0) - lane_of(st, l0);
+                while (more) {
+                    const int l = __ffsll(more) - 1, s = lane_of(st, l);
+                    more &= more - 1;
+                    if (r1 + 1 - r0 == BATCH_BLOCKS) {
+                        pend = s;
+                        break;
+                    }
+                    r1++;
+                    const bool in = p >= s;
+                    r = in ? r1 : r;
+                    j = in ? l : j;
+                    c = in ? lane_of(cl, l) - s : c;
+                }
+                const Pre pre = before(min(c + p, ch.c1 - 1));
+                wave_lds_fence();
+                while (staged <= r1) {
+#pragma unroll
+                    for (int q = 0; q < 2; q++) {
+                        const int p = lane + 64 * q, k = p / Nodes<T>::PIECES;
+                        if (k < ahead)
+                            S.st[(staged + k) % SLOTS][p - k * Nodes<T>::PIECES] = piece[q];
+                    }
+                    staged += ahead;
+                    for (int k = 0; k < ahead; k++) rest &= rest - 1;
+                    load();
+                }
+                wave_lds_fence();
+                if (p < pend) {
+                    const Map q = integrate(S.st[r % SLOTS], jw + j, c + p, pre);
+                    int i = p0 % RING + lane;
+                    S.map[i >= RING ? i - RING : i] = q;
+                }
+                wave_lds_fence();
+            }
+            // the blocks complete at pair pend
+            const int e = __popcll(__ballot(lane < m && incl <= pend));
+            for (; b < e; b++) {
+                const int n = lane_of(cnt, b), c = lane_of(cl, b) - ch.c0;
+                const double A0 = lane_of(bA, b), B0 = lane_of(bB, b);
+                const int s = lane_of(st, b) % RING;
+                const int nv = overs ? lane_of(nov, b) : 0;
+#pragma unroll
+                for (int g = 0; g < G; g++) {
+                    if (g >= ch.ng) break;
+                    double mP = A0, mB = B0;
+                    if (c < 64 * g + 64 && c + n > 64 * g) {     // the group has pairs
+                        const int i = 64 * g + lane - c;
+                        if ((unsigned)i < (unsigned)n) {
+                            const Map q = S.map[s + i >= RING ? s + i - RING : s + i];
+                            mP = q.P;
+                            mB = q.B;
+                            if (sizeof(T) == 4) {
+                                over |= marked(mP) ? 1u << g : 0u;
+                                mP = fabs(mP);
+                            }
+                        } else if (nv > 0) {
+                            passed(g, nv);
+                        }
+                    } else if (nv > 0) {
+                        passed(g, nv);
+                    }
+                    I[g] = sizeof(T) == 4 ? __builtin_fma(I[g], mP, mB) : I[g] * mP + mB;
+                }
+            }
+            p0 = pend;
         }
         wave_lds_fence();
-        if (li < WALK_WIN) {
-            BlkRec *w = &win[g][li];
-            w->lo = lo; w->hi = hi; w->A = A; w->B = B;
-        }
-        const unsigned busy = fold16(__ballot(act && !(uhi < lo || ulo > hi)), cwl);
-        const unsigned have = fold16(__ballot(act), cwl);
-        const bool over = __any(act && (__float_as_int(lo) & (2 * BLK - 1)) != 0);
-        wave_lds_fence();
-        const int nw = 32 - __clz((int)have);
-        for (int b = 0; b < nw; b++) {
-            const BlkRec &w = win[g][b];
-            if (!((busy >> b) & 1)) {
-                free(w.A, w.B, over ? blk_overshoots(w) : 0);
-                continue;
-            }
-            const bool mine = jw + b < j1;
-            if (mine) stage(g, li, jw + b);
-            wave_lds_fence();
-            if (mine && on) {
-                if (blk_free(w, uch)) free(w.A, w.B, blk_overshoots(w));
-                else integrate(g, jw + b);
-            }
-            wave_lds_fence();
-        }
     }
 }
 
-// FP32: charintline (telescope.F:3889-4312) over the blocks [j0, j1) of a ray
-// of n nodes, on split records (rl_fwd32.h)
-template <bool AFF>
-__device__ __forceinline__ void walk_split(WalkLds<float> &S, int cwl,
-                                           const SegHot *__restrict__ hot,
-                                           const SegAux *__restrict__ aux,
-                                           const NodeLine *__restrict__ line,
-                                           const BlkRec *__restrict__ blk, int n, int j0, int j1,
-                                           bool on, float uch, Acc32<AFF> &x, float istar,
-                                           float sf, bool &ovf, int &maser) {
-    constexpr int N = WalkLds<float>::N;
+// FP32: block j of a ray of n nodes for one channel, on split records
+// (rl_fwd32.h) staged as Nodes<float> holds them
+__device__ __forceinline__ Map block_split(const float4 *st, int j, int n, float uch,
+                                           const double *istar, float sf, int &maser) {
+    constexpr int N = Nodes<float>::N;
+    const SegHot *sh = reinterpret_cast<const SegHot *>(st);
+    const SegAux *sa = reinterpret_cast<const SegAux *>(st + N);
+    const NodeLine *sl = reinterpret_cast<const NodeLine *>(st + 2 * N);
+    Acc32<true> x{0.0, 1.0};
     Car32 c;
-    bool fresh = true;
-    walk(S.win, cwl, blk, j0, j1, on, uch, uch, uch,
-         [&](double A, double B, int over) __attribute__((always_inline)) {
-             x.map(A, B);
-             ovf = ovf || over != 0;
-             fresh = true;
-         },
-         [&](int g, int li, int j) __attribute__((always_inline)) {
-             if (li >= N) return;
-             const int k = min(max((j << BLK_LOG) - 1 + li, 0), n - 1);
-             S.st[g][li] = reinterpret_cast<const float4 *>(hot)[k];
-             S.st[g][N + li] = reinterpret_cast<const float4 *>(aux)[k];
-             S.st[g][2 * N + li] = reinterpret_cast<const float4 *>(line)[k];
-         },
-         [&](int g, int j) __attribute__((always_inline)) {
-             const SegHot *sh = reinterpret_cast<const SegHot *>(S.st[g]);
-             const SegAux *sa = reinterpret_cast<const SegAux *>(S.st[g] + N);
-             const NodeLine *sl = reinterpret_cast<const NodeLine *>(S.st[g] + 2 * N);
-             const int k0 = j << BLK_LOG, i1 = min(BLK, n - k0);
-             if (fresh) {
-                 // the carry of node k0-1 as the end of segment k0-1 (its
-                 // profile); the ray's first node under segment 1's
-                 const int m = j > 0 ? 0 : 1;
-                 const SegHot hp = sh[2 * m];
-                 carry32(pt_of(sa[m].u, sl[m]), uch, hp.ag, hp.ng, c);
-                 fresh = false;
-             }
-             for (int i = j > 0 ? 0 : 1; i < i1; i++) {
-                 segment32(x, sh + i + 1, sa + i + 1, sl + i + 1, uch, istar, sf, c, ovf, maser);
-             }
-         });
+    bool ovf = false;
+    // the carry of node k0-1 as the end of segment k0-1 (its profile); the
+    // ray's first node under segment 1's
+    const int m = j > 0 ? 0 : 1, i1 = min(BLK, n - (j << BLK_LOG));
+    const SegHot hp = sh[2 * m];
+    carry32(pt_of(sa[m].u, sl[m]), uch, hp.ag, hp.ng, c);
+    for (int i = m; i < i1; i++)
+        segment32(x, sh + i + 1, sa + i + 1, sl + i + 1, uch, istar, sf, c, ovf, maser);
+    return Map{mark(x.P, ovf), x.I};
 }
 
 // FP64: the same on whole node records, with the reference's own arithmetic
-template <bool AFF>
-__device__ __forceinline__ void walk_exact(WalkLds<double> &S, int cwl,
-                                           const NodeRec<double> *__restrict__ rec,
-                                           const BlkRec *__restrict__ blk, int n, int j0, int j1,
-                                           bool on, const LineK<double> &L, Acc<double, AFF> &x,
-                                           double istar, double sf, int &ovs, int &maser) {
-    constexpr int N = WalkLds<double>::N;
+__device__ __forceinline__ Map block_exact(const float4 *st, int j, int n, const LineK<double> &L,
+                                           const double *istar, double sf, int &ovs, int &maser) {
+    const NodeRec<double> *sr = reinterpret_cast<const NodeRec<double> *>(st);
+    Acc<double, true> x{0.0, 1.0};
     Carry<double> c;
     c.init = 1; c.phi0 = 0.0; c.srcl0 = 0.0; c.alpl0 = 0.0; c.S0 = 0.0;
-    bool fresh = true;
-    const float uf = (float)L.uch;
-    walk(S.win, cwl, blk, j0, j1, on, nextafterf(uf, -INFINITY), nextafterf(uf, INFINITY), L.uch,
-         [&](double A, double B, int over) __attribute__((always_inline)) {
-             x.map(A, B);
-             ovs += over;
-             fresh = true;
-         },
-         [&](int g, int li, int j) __attribute__((always_inline)) {
-             const int k0 = (j << BLK_LOG) - 2;
-             for (int p = li; p < 4 * N; p += 1 << cwl) {
-                 const int k = min(max(k0 + (p >> 2), 0), n - 1);
-                 reinterpret_cast<float4 *>(S.st[g])[p] =
-                     reinterpret_cast<const float4 *>(rec)[(size_t)k * 4 + (p & 3)];
-             }
-         },
-         [&](int g, int j) __attribute__((always_inline)) {
-             const NodeRec<double> *sr = S.st[g];
-             const int k0 = j << BLK_LOG, i1 = min(BLK, n - k0);
-             if (fresh && j > 0) carry_of<double>(L, sr[0], sr[1], c);
-             fresh = false;
-             for (int i = j > 0 ? 0 : 1; i < i1; i++)
-                 segment_exact<double>(L, x, sr[i + 1], sr[i + 2], istar, sf, c, ovs, maser);
-         });
+    const int i1 = min(BLK, n - (j << BLK_LOG));
+    if (j > 0) carry_of<double>(L, sr[0], sr[1], c);
+    for (int i = j > 0 ? 0 : 1; i < i1; i++)
+        segment_exact<double>(L, x, sr[i + 1], sr[i + 2], istar, sf, c, ovs, maser);
+    return Map{x.P, x.I};
 }
 
 }  // namespace rl
