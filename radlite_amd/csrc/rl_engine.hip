@@ -29,6 +29,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include "rl_traj.h"
+#include "rl_cross.h"
 #include "rl_adjoint.h"
 #include "rl_fwd32.h"
 #include "rl_blocks.h"
@@ -67,8 +68,14 @@ constexpr int CROSS_BLOCK = 128, CROSS_LINE = 4;
 
 __global__ void __launch_bounds__(CROSS_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
 k_cross(GridView g, const double *__restrict__ tan2, CrossSets sets, int nmax, int *err,
-        int grid_in_lds) {
+        int grid_in_lds, int marked) {
     __shared__ CrossRec stage[CROSS_LINE][CROSS_BLOCK];
+    // marked: only the rays that k_cross_wave left
+    if (marked) {
+        const CrossSet &q = sets.s[blockIdx.y];
+        const int ray = blockIdx.x * blockDim.x + threadIdx.x;
+        if (!__syncthreads_or(ray < q.nrays && q.count[ray] == CROSS_SEQUENTIAL)) return;
+    }
     // the radii, cone angles and tan^2 table (a few KB) staged in LDS: the
     // merge reads them at every step
     extern __shared__ double lds_grid[];
@@ -93,7 +100,7 @@ k_cross(GridView g, const double *__restrict__ tan2, CrossSets sets, int nmax, i
     int *__restrict__ count = q.count;
     CrossRec *__restrict__ cr = q.cr;
     int ray = blockIdx.x * blockDim.x + threadIdx.x;
-    if (ray >= nrays) return;
+    if (ray >= nrays || (marked && count[ray] != CROSS_SEQUENTIAL)) return;
     if (q.bpix && !(q.bpix[ray] < q.bmax)) {     // telescope.F:2118: outside, not traced
         count[ray] = 0;
         return;
@@ -141,6 +148,26 @@ k_cross(GridView g, const double *__restrict__ tan2, CrossSets sets, int nmax, i
     count[ray] = n;
 }
 
+
+// The same with one wave per ray (rl_cross.h), for launches of few rays, where
+// the thread per ray is a serial chain of hundreds of square roots and quotients
+// on a nearly empty machine.
+__global__ void __launch_bounds__(64)
+k_cross_wave(GridView g, const double *__restrict__ tan2, CrossSets sets, int nmax, int *err) {
+    extern __shared__ double lds_cross[];
+    const CrossSet &q = sets.s[blockIdx.y];
+    const int ray = blockIdx.x;
+    if (ray >= q.nrays) return;
+    int n = 0, code = 0;
+    if (!(q.bpix && !(q.bpix[ray] < q.bmax)))    // telescope.F:2118: outside, not traced
+        n = cross_wave(g, tan2, q.x0[ray], q.z0[ray], q.theta0, q.costh0, q.sinth0,
+                       ray == 0 && q.central_blend, nmax, lds_cross, q.cr + (long long)ray * nmax,
+                       code);
+    if (threadIdx.x == 0) {
+        if (code) set_err(err, code);
+        q.count[ray] = n;
+    }
+}
 
 // Stage 2, one thread per node: position, cell, interpolation stencil,
 // local direction (telescope.F:3682-3718) and projected velocity
@@ -1052,6 +1079,14 @@ template void launch_posvel<float>(hipStream_t, const PosvelLaunch &);
 // ---------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------
+// One wave per ray up to this many rays of a launch.  A thread per ray takes as
+// long for 2,000 rays as for 60,000 (one chain), a wave per ray's time grows with
+// them: 60 x 40 cube, 1,920 rays, build of the trajectories 0.35 -> 0.09 ms; 100
+// x 60 disk, 7,041 rays, 0.60 -> 0.22 ms; 200 x 100, 34,049, 1.14 -> 0.81; 256 x
+// 128 x 4 inclinations, 68,100, 2.37 -> 2.23; 400 x 200 x 2, 267,266 (with 25 KB
+// of LDS a wave), 9.5 -> 13.9, so not there.
+constexpr long long CROSS_WAVE_RAYS = 80000;
+constexpr size_t CROSS_WAVE_LDS = 48 * 1024;
 void launch_cross(hipStream_t st, const GridDev &gd, const double *tan2, const CrossSets &sets,
                   int nmax, int *err) {
     GridView g{gd.nr, gd.ny, gd.rc, gd.tc, gd.rstar, gd.t_sorted};
@@ -1060,7 +1095,15 @@ void launch_cross(hipStream_t st, const GridDev &gd, const double *tan2, const C
     dim3 blk(CROSS_BLOCK), grd((most + CROSS_BLOCK - 1) / CROSS_BLOCK, sets.n);
     const size_t lds = (size_t)(gd.nr + 4 + gd.ny + 4 + gd.ny / 2 + 1) * sizeof(double);
     const int in_lds = lds <= 48 * 1024 ? 1 : 0;
-    hipLaunchKernelGGL(k_cross, grd, blk, in_lds ? lds : 0, st, g, tan2, sets, nmax, err, in_lds);
+    long long rays = 0;
+    for (int i = 0; i < sets.n; i++) rays += sets.s[i].nrays;
+    const size_t wl = cross_wave_lds(nmax);
+    const int wave = rays <= CROSS_WAVE_RAYS && wl <= CROSS_WAVE_LDS;
+    if (wave)
+        hipLaunchKernelGGL(k_cross_wave, dim3(most, sets.n), dim3(64), wl, st, g, tan2, sets, nmax,
+                           err);
+    hipLaunchKernelGGL(k_cross, grd, blk, in_lds ? lds : 0, st, g, tan2, sets, nmax, err, in_lds,
+                       wave);
 }
 
 // velocity [cell][3] and width [cell] into one record per cell; the rays'
