@@ -461,12 +461,18 @@ __device__ inline bool subgrid_of(const FastRecT<T> &b, T ds, T u0, T uch, SubGr
     T sright = s_c + T(3) * b.dls, sleft = s_c - T(3) * b.dls;
     if (!(sright > T(0) && sleft < ds)) return false;
     T lg = (sright - sleft) * (T(1) / T(30));
-    // only bounds of the index range (the exact 0 < s < ds test follows)
+    // bounds of the index range (the exact 0 < s < ds test follows), at most
+    // two points too wide, and cut: a wave's loop is as long as its longest
+    // lane's points
     T f0 = FOps<T>::fdiv(-sleft, lg), f1 = FOps<T>::fdiv(ds - sleft, lg);
     sg.sleft = sleft;
     sg.lg = lg;
     sg.ilo = f0 > T(0) ? max(1, (int)FOps<T>::fmn(f0, T(40))) : 1;
     sg.ihi = f1 < T(40) ? min(31, (int)FOps<T>::fmx(f1, T(-2)) + 2) : 31;
+    for (int q = 0; q < 2; q++) {
+        if (!(sleft + (T)(sg.ilo - 1) * lg > T(0))) sg.ilo++;
+        if (!(sleft + (T)(sg.ihi - 1) * lg < ds)) sg.ihi--;
+    }
     return true;
 }
 
