@@ -40,11 +40,13 @@ __device__ inline void pg_zero(PGrad<T> &g) {
 // are the forward's values.  Accumulates into g0/g1 (the two points),
 // g_ds and g_lnaa (= dL/d ln inv_aa); returns dL/dI_in and, when
 // init == 0, the gradient on the carried start values in gjl0/gal0.
+// elem_rev_sum takes lam I_in in place of I_in, which enters nowhere else: with
+// sums over channels that share the element it gives the sum of their gradients.
 template <typename T>
-__device__ inline T elem_rev(const FastLineT<T> &L, T I_in, T lam, T ds, const FPtT<T> &p0,
-                             const FPtT<T> &p1, T z1, T phi1, T inv_aa, T norm, int init,
-                             T jl0c, T al0c, T gjl1, T gal1, PGrad<T> &g0, PGrad<T> &g1,
-                             T &g_ds, T &g_lnaa, T &gjl0, T &gal0) {
+__device__ inline T elem_rev_sum(const FastLineT<T> &L, T lamI, T lam, T ds, const FPtT<T> &p0,
+                                 const FPtT<T> &p1, T z1, T phi1, T inv_aa, T norm, int init,
+                                 T jl0c, T al0c, T gjl1, T gal1, PGrad<T> &g0, PGrad<T> &g1,
+                                 T &g_ds, T &g_lnaa, T &gjl0, T &gal0) {
     using O = FOps<T>;
     T z0 = T(0), phi0 = T(0), jl0 = jl0c, al0 = al0c;
     if (init) {
@@ -70,7 +72,7 @@ __device__ inline T elem_rev(const FastLineT<T> &L, T I_in, T lam, T ds, const F
 
     // I_out = I_in*xp + min(qraw, theomax)
     const T lam_in = lam * xp;
-    const T g_xp = lam * I_in;
+    const T g_xp = lamI;
     T g_q = T(0), g_th = T(0);
     if (qraw < theomax) g_q = lam; else g_th = lam;
     T g_wa = T(0), g_wb = T(0), g_s1 = T(0), g_s2 = T(0);
@@ -134,6 +136,15 @@ __device__ inline T elem_rev(const FastLineT<T> &L, T I_in, T lam, T ds, const F
     return lam_in;
 }
 
+template <typename T>
+__device__ inline T elem_rev(const FastLineT<T> &L, T I_in, T lam, T ds, const FPtT<T> &p0,
+                             const FPtT<T> &p1, T z1, T phi1, T inv_aa, T norm, int init,
+                             T jl0c, T al0c, T gjl1, T gal1, PGrad<T> &g0, PGrad<T> &g1,
+                             T &g_ds, T &g_lnaa, T &gjl0, T &gal0) {
+    return elem_rev_sum<T>(L, lam * I_in, lam, ds, p0, p1, z1, phi1, inv_aa, norm, init, jl0c,
+                           al0c, gjl1, gal1, g0, g1, g_ds, g_lnaa, gjl0, gal0);
+}
+
 // largest v over the wave (all lanes active), in a scalar register
 __device__ inline int wave_max(int v) {
     for (int o = 32; o >= 1; o >>= 1) v = max(v, __shfl_xor(v, o));
@@ -146,6 +157,16 @@ template <typename T>
 __device__ inline void profile_at(const FastLineT<T> &L, T u, T inv_aa, T norm, T &z, T &phi) {
     z = FOps<T>::fma(-L.nu0, u, L.dnu) * inv_aa;
     phi = norm * FOps<T>::ex(-(z * z));
+}
+
+// line values carried into segment k: node k-1 with segment k-1's profile
+// (z, phi: its argument and value, the end-point profile of segment k-1)
+template <typename T>
+__device__ inline void carried_in(const FastRecT<T> &a, const FastLineT<T> &L, T &jl, T &al,
+                                  T &z, T &phi) {
+    profile_at<T>(L, a.u, a.inv_aa, a.norm, z, phi);
+    jl = a.jch * phi;
+    al = a.dch * phi;
 }
 
 // dL/d(sub-point q at fraction e, with subpoint's normalised weights

@@ -56,6 +56,7 @@ struct DevBuf {
 // rl_trace_lines_forward_tape and rl_trace_lines_adjoint.
 struct AdjItemBufs {
     DevBuf rec, ckoff, ckpt;
+    long long nblk = 0;       // ckpt by blocks (rl_adj_blocks.h): how many; 0: by intervals
 };
 
 struct RaySet {
@@ -1965,6 +1966,20 @@ static int plan_adjoint(rl_ctx *c, const RaySet &rs, int nfr, bool tape, AdjPlan
     return 0;
 }
 
+// where a chunk's block checkpoints lie in its ckpt buffer: I, P and lambda per
+// (block, channel), the line-free sums per (block, 64 channels), the bounds
+struct AdjBlockBytes {
+    size_t ckP, lam, bsum, bounds, all;
+    AdjBlockBytes(long long nblk, int nfr, bool fp64) {
+        const size_t n = (size_t)nblk * nfr * (fp64 ? 8 : 4);
+        ckP = n;
+        lam = 2 * n;
+        bsum = (3 * n + 15) & ~(size_t)15;
+        bounds = bsum + (size_t)nblk * ((nfr + 63) / 64) * 16;
+        all = bounds + (size_t)nblk * 8;
+    }
+};
+
 static void fill_adj(rl_ctx *c, const rl_item &it, const ItemSetup &su, AdjItemBufs &ab, int K,
                      const AdjChunk &ch, rl::AdjLaunch &a) {
     const RaySet &rs = *su.rs;
@@ -1984,6 +1999,13 @@ static void fill_adj(rl_ctx *c, const rl_item &it, const ItemSetup &su, AdjItemB
     a.rinfo = c->d_rinfo.as<RayInfo>();
     a.ckpt = ab.ckpt.p;
     a.kblk = K;
+    const AdjBlockBytes bb(ab.nblk, nfr, c->precision == RL_FP64);
+    char *base = ab.ckpt.as<char>();
+    a.nblk = ab.nblk;
+    a.ckP = base + bb.ckP;
+    a.lam = base + bb.lam;
+    a.bsum = reinterpret_cast<double *>(base + bb.bsum);
+    a.bounds = base + bb.bounds;
     a.dnu = c->d_chan.as<double>();
     a.velo = a.dnu + nfr;
     a.istar = a.dnu + 2 * nfr;
@@ -2045,8 +2067,25 @@ static int adj_forward_chunk(rl_ctx *c, const rl_item &it, const ItemSetup &su, 
         const long long n = rs.off[ch.r0 + r + 1] - rs.off[ch.r0 + r];
         ckoff[r + 1] = ckoff[r] + (n >= 2 ? (n - 1 + K - 1) / K : 0);
     }
+    // I before every segment (K = 1) is held, but by blocks: I at their starts is
+    // enough for the reverse sweep by pairs (fit on the 200 x 100 disk, FP32, 20.2 ->
+    // 12.9 ms), in less memory unless the rays are a few nodes long.  An interval of more
+    // segments is asked for or taken to save memory, and keeps its own layout.
+    size_t bytes = (size_t)ckoff[nr] * nfr * tsz;
+    ab.nblk = 0;
+    if (K == 1) {
+        std::vector<long long> bo(nr + 1, 0);
+        for (int r = 0; r < nr; r++)
+            bo[r + 1] = bo[r] + rl::adjoint_ray_blocks(rs.off[ch.r0 + r + 1] - rs.off[ch.r0 + r]);
+        const AdjBlockBytes bb(bo[nr], nfr, c->precision == RL_FP64);
+        if (bo[nr] && bb.all <= bytes) {
+            ab.nblk = bo[nr];
+            ckoff.swap(bo);
+            bytes = bb.all;
+        }
+    }
     if (int e = upload(c, ab.ckoff, ckoff.data(), ckoff.size() * 8)) return e;
-    HIPCHK(c, ab.ckpt.ensure((size_t)ckoff[nr] * nfr * tsz));
+    HIPCHK(c, ab.ckpt.ensure(bytes));
     HIPCHK(c, ab.rec.ensure((size_t)(ch.n1 - ch.n0) * rl::fast_rec_size(c->precision == RL_FP64)));
     rl::AdjLaunch a;
     fill_adj(c, it, su, ab, K, ch, a);

@@ -381,6 +381,7 @@ template <typename T> struct FastCarryT {
     T sa0 = T(0), sj0 = T(0), ah0 = T(0), S0 = T(0), al0 = T(0);
     int init = 1;
     T u0 = T(0), tau = T(0), tau_c = T(0);
+    T P = T(1);                 // dI/d(I at the start): the product of the elements' factors
 };
 
 // the carry of a start point p0 with line values jl0, al0 (/ sig)
@@ -433,6 +434,7 @@ __device__ inline void elem_core(const FastLineT<T> &L, T &I, T ds, const Start 
     ovs += q > T(2) * theomax;
     q = O::fmn(q, theomax);
     I = O::fma(I, xp, q);
+    c.P = c.P * xp;
     c.sa0 = p1.sig * ah1;
     c.sj0 = p1.sig * jh1;
     c.ah0 = ah1;
@@ -518,8 +520,12 @@ __device__ inline void segment_fast(const FastRecT<T> &b, const FastRecT<T> *pre
     // its lanes has one (a reset segment's ds is already 0 in the record)
     if (__builtin_amdgcn_ballot_w64(fl != 0)) {
         if (fl & NF_RESET) { ds = T(0); c.init = 1; }
-        if (fl & NF_BLEND) { I = (T(1) - starfract) * I + starfract * istar; c.init = 1; }
-        if (fl & NF_STAR) { I = istar; c.init = 1; }
+        if (fl & NF_BLEND) {
+            I = (T(1) - starfract) * I + starfract * istar;
+            c.P = c.P * (T(1) - starfract);
+            c.init = 1;
+        }
+        if (fl & NF_STAR) { I = istar; c.P = T(0); c.init = 1; }
     }
     // one call for the last (or only) element of every segment: a segment
     // integrated whole has sa = 0 and ds - 0 = ds exactly, and its start

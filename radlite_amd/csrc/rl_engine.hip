@@ -34,6 +34,7 @@
 #include "rl_fwd32.h"
 #include "rl_blocks.h"
 #include "rl_walk.h"
+#include "rl_adj_blocks.h"
 
 namespace rl {
 
@@ -1507,14 +1508,15 @@ int formal_blocks_per_cu(int fp64) {
 // lane per (ray, channel), keeping I before every kblk-th segment.  A call
 // covers rays ray0.. of the ray set (a chunk): off is the chunk's slice of
 // the node CSR (global node indices), rec, ckoff, ckpt and image are the
-// chunk's own, node0 its first node.
-template <typename T>
+// chunk's own, node0 its first node.  BLOCKS: I before every block's first
+// segment, and in ckP the block's factor dI_out/dI_in.
+template <typename T, bool BLOCKS>
 __global__ void __launch_bounds__(256)
 k_adj_fwd(int nrays, int nfr, int ray0, long long node0, const long long *__restrict__ off,
           const long long *__restrict__ ckoff, const FastRecT<T> *__restrict__ rec,
           const double *__restrict__ dnu, const double *__restrict__ velo,
           const double *__restrict__ istar, const double *__restrict__ i0, LineConst lc,
-          double *__restrict__ image, T *__restrict__ ckpt, int kblk) {
+          double *__restrict__ image, T *__restrict__ ckpt, T *__restrict__ ckP, int kblk) {
     const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= (long long)nrays * nfr) return;
     const int ray = (int)(g / nfr), ch = (int)(g - (long long)ray * nfr);
@@ -1532,17 +1534,24 @@ k_adj_fwd(int nrays, int nfr, int ray0, long long node0, const long long *__rest
     // (a countdown: a remainder by the run-time kblk costs an emulated
     // division per segment)
     T *ck = ckpt + ckoff[ray] * nfr + ch;
+    T *cp = BLOCKS ? ckP + ckoff[ray] * nfr + ch : nullptr;
     int until = 0;                           // segments until the next checkpoint
     for (int k = 1; k < n; k++) {
-        if (until == 0) {
+        if (BLOCKS ? k == 1 || (k & (BLK - 1)) == 0 : until == 0) {
             *ck = I;
             ck += nfr;
             until = kblk;
+            if (BLOCKS && k > 1) {
+                *cp = c.P;
+                cp += nfr;
+                c.P = T(1);
+            }
         }
         until--;
         const FastRecT<T> r = rec[b + k];
         segment_fast<T>(r, rec + b + k - 1, point_of<T>(r), L, I, ist, sf, c, ovs);
     }
+    if (BLOCKS) *cp = c.P;
     image[g] = (double)I;
 }
 
@@ -1604,16 +1613,6 @@ struct BlockNodeSum {
         if (++n == RED_N) flush(gnode);
     }
 };
-
-// line values carried into segment k: node k-1 with segment k-1's profile
-// (z, phi: its argument and value, the end-point profile of segment k-1)
-template <typename T>
-__device__ inline void carried_in(const FastRecT<T> &a, const FastLineT<T> &L, T &jl, T &al,
-                                  T &z, T &phi) {
-    profile_at<T>(L, a.u, a.inv_aa, a.norm, z, phi);
-    jl = a.jch * phi;
-    al = a.dch * phi;
-}
 
 // reverse pass: one wave per ray, over its channels in groups of 64 (in
 // order); per node the gradients on (jd, ad, jc, dc) / sig and per segment
@@ -1778,6 +1777,109 @@ k_adj_rev<float>(int nrays, int nfr, int nphi, int ray0, long long node0,
                         gflux, ring_w, center_w, d2, ckpt, gnode, kblk, nw);
 }
 
+// ---- the reverse sweep by (block, channel) pairs (rl_adj_blocks.h)
+template <typename T>
+__global__ void __launch_bounds__(64)
+k_adj_bounds(AdjLaunch a) {
+    const int ray = blockIdx.x;
+    const long long b = a.off[ray] - a.node0;
+    adj_bounds<T>(threadIdx.x, reinterpret_cast<const FastRecT<T> *>(a.rec) + b,
+                  (int)(a.off[ray + 1] - a.off[ray]), (int)(a.ckoff[ray + 1] - a.ckoff[ray]),
+                  (T)a.lc.nu0, reinterpret_cast<float2 *>(a.bounds) + a.ckoff[ray]);
+}
+
+// lambda at the end of every block, backwards over a ray's blocks, and the sums
+// of lambda and lambda I over the channels that do not see the line there.  One
+// wave per ray and 64 channels; a stream of two loads and a store per (block,
+// channel), the loads of the next AHEAD blocks in flight.
+template <typename T>
+__global__ void __launch_bounds__(64)
+k_adj_lambda(AdjLaunch a, int ngrp) {
+    const int ray = blockIdx.x, grp = blockIdx.y, lane = threadIdx.x, nfr = a.nfr;
+    const long long o = a.ckoff[ray];
+    const int nb = (int)(a.ckoff[ray + 1] - o);
+    if (nb <= 0) return;
+    const int ch = grp * 64 + lane;
+    const bool active = ch < nfr;
+    const int chc = active ? ch : nfr - 1;
+    // flux = (center_w I_0 + sum_rings ring_w mean_phi I) / d2 (telescope.F:1386-1418)
+    const int rg = a.ray0 + ray;
+    const double w = rg == 0 ? a.center_w : a.ring_w[(rg - 1) / a.nphi] / (1.0 * a.nphi);
+    double lam = active ? (double)(T)(a.gflux[chc] * w / a.d2) : 0.0;
+    const T v = (T)a.velo[chc];
+    const T *I = reinterpret_cast<const T *>(a.ckpt) + o * nfr + chc;
+    const T *P = reinterpret_cast<const T *>(a.ckP) + o * nfr + chc;
+    T *out = reinterpret_cast<T *>(a.lam) + o * nfr + chc;
+    const float2 *bd = reinterpret_cast<const float2 *>(a.bounds) + o;
+    constexpr int AHEAD = 4;
+    T pi[AHEAD], pp[AHEAD];
+#pragma unroll
+    for (int q = 0; q < AHEAD; q++) {
+        const long long j = max(nb - 1 - q, 0);
+        pi[q] = I[j * nfr];
+        pp[q] = P[j * nfr];
+    }
+    for (int j0 = nb - 1; j0 >= 0; j0 -= AHEAD) {
+#pragma unroll
+        for (int q = 0; q < AHEAD; q++) {
+            const int j = j0 - q;
+            if (j < 0) break;
+            const double Ij = (double)pi[q], Pj = (double)pp[q];
+            const long long nx = max(j - AHEAD, 0);
+            pi[q] = I[nx * nfr];
+            pp[q] = P[nx * nfr];
+            if (active) out[(long long)j * nfr] = (T)lam;
+            const float2 b = bd[j];
+            const bool seen = !(b.x > b.y) && !(v < (T)b.x) && v <= (T)b.y;
+            double s0 = 0.0, s1 = 0.0;
+            if (__any(active && !seen)) {
+                s0 = seen ? 0.0 : lam;
+                s1 = seen ? 0.0 : lam * Ij;
+                for (int m = 32; m >= 1; m >>= 1) {
+                    s0 += __shfl_xor(s0, m);
+                    s1 += __shfl_xor(s1, m);
+                }
+            }
+            if (lane == 0) {
+                double *s = a.bsum + ((o + j) * ngrp + grp) * 2;
+                s[0] = s0;
+                s[1] = s1;
+            }
+            lam *= Pj;
+        }
+    }
+}
+
+// waves per SIMD that the registers are held to (FP32, fit on the 200 x 100 disk:
+// two 13.5 ms, three 12.9, four, which spill, 13.5)
+template <typename T> struct AdjPairWaves { static constexpr int n = 2; };
+template <> struct AdjPairWaves<float> { static constexpr int n = 3; };
+template <typename T>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AdjPairWaves<T>::n)))
+k_adj_pairs(AdjLaunch a, int ngrp) {
+    __shared__ AdjLds<T> lds;
+    const int ray = blockIdx.x;
+    const long long b = a.off[ray] - a.node0, o = a.ckoff[ray];
+    const int nb = (int)(a.ckoff[ray + 1] - o);
+    if (nb <= 0) return;
+    AdjRay<T> y;
+    y.rec = reinterpret_cast<const FastRecT<T> *>(a.rec) + b;
+    y.n = (int)(a.off[ray + 1] - a.off[ray]);
+    y.nb = nb;
+    y.nfr = a.nfr;
+    y.bounds = reinterpret_cast<const float2 *>(a.bounds) + o;
+    y.ckI = reinterpret_cast<const T *>(a.ckpt) + o * a.nfr;
+    y.lam = reinterpret_cast<const T *>(a.lam) + o * a.nfr;
+    y.bsum = a.bsum + o * ngrp * 2;
+    y.dnu = a.dnu;
+    y.velo = a.velo;
+    y.istar = a.istar;
+    y.nu0 = (T)a.lc.nu0;
+    y.sf = a.ray0 + ray == 0 ? (T)a.lc.starfract : T(0);
+    y.cai = (T)a.lc.c_aa;
+    adj_ray<T>(lds, y, ngrp, a.gnode + b * 5);
+}
+
 // ---- node -> cell transpose of the interpolation stencil (once per ray set)
 __device__ inline void stencil_weights(const GeoNode &gn, double w[4]) {
     const double dr = gn.dr, dt = gn.dt;
@@ -1907,9 +2009,18 @@ void launch_adjoint_fwd(hipStream_t st, const AdjLaunch &a) {
     hipLaunchKernelGGL(k_nodes_fast<T>, dim3(a.nrays), dim3(64), 0, st, a.nrays, a.off, a.geo,
                        a.cells, rec, a.node0, a.rinfo, a.nfr, a.velo, a.aks2, 1, a.lc);
     const long long total = (long long)a.nrays * a.nfr;
-    hipLaunchKernelGGL(k_adj_fwd<T>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
-                       a.nrays, a.nfr, a.ray0, a.node0, a.off, a.ckoff, rec, a.dnu, a.velo,
-                       a.istar, a.i0, a.lc, a.image, ck, a.kblk);
+    auto *cp = reinterpret_cast<T *>(a.ckP);
+    const dim3 grid((unsigned)((total + 255) / 256));
+    if (a.nblk) {
+        hipLaunchKernelGGL(k_adj_bounds<T>, dim3(a.nrays), dim3(64), 0, st, a);
+        hipLaunchKernelGGL((k_adj_fwd<T, true>), grid, dim3(256), 0, st, a.nrays, a.nfr, a.ray0,
+                           a.node0, a.off, a.ckoff, rec, a.dnu, a.velo, a.istar, a.i0, a.lc,
+                           a.image, ck, cp, a.kblk);
+    } else {
+        hipLaunchKernelGGL((k_adj_fwd<T, false>), grid, dim3(256), 0, st, a.nrays, a.nfr, a.ray0,
+                           a.node0, a.off, a.ckoff, rec, a.dnu, a.velo, a.istar, a.i0, a.lc,
+                           a.image, ck, cp, a.kblk);
+    }
 }
 
 // the spectrum of an item from its whole image (every chunk traced)
@@ -1931,10 +2042,15 @@ void launch_adjoint_rev(hipStream_t st, const AdjLaunch &a) {
     const int ngrp = (a.nfr + 63) / 64;
     int nw = std::min(ngrp, AdjRevWaves<T>::max);
     while (nw > 1 && adj_rev_lds<T>(nw) > 65536) nw--;
-    hipLaunchKernelGGL(k_adj_rev<T>, dim3(a.nrays), dim3(64 * nw), adj_rev_lds<T>(nw), st,
-                       a.nrays, a.nfr, a.nphi, a.ray0, a.node0, a.off, a.ckoff, rec, a.dnu,
-                       a.velo, a.istar, a.lc, a.gflux, a.ring_w, a.center_w, a.d2, ck, a.gnode,
-                       a.kblk, nw);
+    if (a.nblk) {
+        hipLaunchKernelGGL(k_adj_lambda<T>, dim3(a.nrays, ngrp), dim3(64), 0, st, a, ngrp);
+        hipLaunchKernelGGL(k_adj_pairs<T>, dim3(a.nrays), dim3(64), 0, st, a, ngrp);
+    } else {
+        hipLaunchKernelGGL(k_adj_rev<T>, dim3(a.nrays), dim3(64 * nw), adj_rev_lds<T>(nw), st,
+                           a.nrays, a.nfr, a.nphi, a.ray0, a.node0, a.off, a.ckoff, rec, a.dnu,
+                           a.velo, a.istar, a.lc, a.gflux, a.ring_w, a.center_w, a.d2, ck,
+                           a.gnode, a.kblk, nw);
+    }
     hipLaunchKernelGGL(k_node_conv, dim3((unsigned)((a.nnodes + 255) / 256)), dim3(256), 0, st,
                        a.nnodes, a.geo + a.node0, a.cells, a.gnode, a.lc, a.gtrue);
     hipLaunchKernelGGL(k_cell_gather, dim3(a.ncell), dim3(64), 0, st, a.ncell, a.st_off,
@@ -1949,6 +2065,7 @@ template void launch_adjoint_rev<double>(hipStream_t, const AdjLaunch &);
 template void launch_adjoint_rev<float>(hipStream_t, const AdjLaunch &);
 
 int adjoint_block_len() { return ADJ_K; }
+long long adjoint_ray_blocks(long long n) { return n >= 2 ? ((n - 1) >> BLK_LOG) + 1 : 0; }
 size_t fast_rec_size(int fp64) { return fp64 ? sizeof(FastRecT<double>) : sizeof(FastRecT<float>); }
 
 
