@@ -16,9 +16,9 @@
 // (ray, 64 channels), a segment at a time, stepped every lane through the
 // sub-grid points of the few channels at resonance.
 // 200 x 100 disk, 100 channels, FP32: reverse sweep 13.1 -> 6.9 ms (pairs 5.7,
-// lambda 1.0, bounds 0.2), and the forward pass, which writes a quarter of the
-// checkpoints' bytes, 4.3 -> 3.1 ms; 40 x 24 disk, 24 channels, FP64: 0.73 ->
-// 0.36 ms.
+// lambda 1.0, bounds 0.2), a fit's step 20.2 -> 11.5 ms with the forward by maps;
+// FP64 9.3 -> 4.6 ms with 32 angles; 40 x 24 disk, 24 channels, FP64, 1.6 -> 0.96.
+// Held to 128 registers it spills, with more than 168 too few waves are left.
 #pragma once
 #include "rl_adjoint.h"
 #include "rl_blocks.h"
@@ -42,19 +42,34 @@ template <typename T> struct AdjLds {
     int st[ADJ_WIN + 1];             // first pair of each block
 };
 
+// dust alone at a node
+template <typename T>
+__device__ inline FPtT<T> dust_of(const FastRecT<T> &a) {
+    return FPtT<T>{a.u, a.sig, a.jdh, a.adh, T(0), T(0)};
+}
+
 // the channel velocities [lo, hi] that see the line on the nb blocks of a ray
-// of n nodes (lane <-> block; -inf .. inf: every channel)
+// of n nodes (lane <-> block; -inf .. inf: every channel), and the blocks' dust
+// maps I -> x I + y
 template <typename T>
 __device__ inline void adj_bounds(int lane, const FastRecT<T> *__restrict__ rec, int n, int nb,
-                                  T nu0, float2 *__restrict__ out) {
+                                  T nu0, float2 *__restrict__ out, double2 *__restrict__ dust) {
+    const FastLineT<T> L{nu0, T(0), T(0)};
     const float scale = 0.8325546112f / (float)fabs(nu0);      // sqrt(ln 2)
     for (int j = lane; j < nb; j += 64) {
         float lo = INFINITY, hi = -INFINITY;
         const int k1 = min(j * BLK + BLK, n);
         int k = max(1, j * BLK);
         FastRecT<T> p = rec[k - 1];
+        double A = 1.0, B = 0.0;
         for (; k < k1; k++) {
             const FastRecT<T> r = rec[k];
+            FastCarryT<T> c;
+            T q = T(0);
+            int ovs = 0;
+            elem_fast<T>(L, q, r.ds, dust_of<T>(p), dust_of<T>(r), r.inv_aa, r.norm, c, ovs);
+            B = B * (double)c.P + (double)q;
+            A = A * (double)c.P;
             // the widest and narrowest profile at node k-1
             const bool two = k > 1;
             const float ia = (float)(two && p.inv_aa < r.inv_aa ? p.inv_aa : r.inv_aa);
@@ -75,13 +90,29 @@ __device__ inline void adj_bounds(int lane, const FastRecT<T> *__restrict__ rec,
             p = r;
         }
         out[j] = make_float2(lo, hi);
+        dust[j] = make_double2(A, B);
     }
 }
 
-// dust alone at a node
+// whether channel velocity v sees the line on a block of bounds b
+template <typename T> __device__ inline bool sees(float2 b, T v) {
+    return !(b.x > b.y) && !(v < (T)b.x) && v <= (T)b.y;
+}
+
+// the carry at the start of block j of a ray (rec: its first record)
 template <typename T>
-__device__ inline FPtT<T> dust_of(const FastRecT<T> &a) {
-    return FPtT<T>{a.u, a.sig, a.jdh, a.adh, T(0), T(0)};
+__device__ inline void block_carry(const FastRecT<T> *__restrict__ rec, int j,
+                                   const FastLineT<T> &L, FastCarryT<T> &c) {
+    const FastRecT<T> a = rec[max(j * BLK - 1, 0)];
+    c.u0 = a.u;
+    c.P = T(1);
+    c.init = 1;
+    if (j > 0) {
+        T jl0, al0, z_, phi_;
+        carried_in<T>(a, L, jl0, al0, z_, phi_);
+        carry_start<T>(point_of<T>(a), jl0, al0, c);
+        c.init = 0;
+    }
 }
 
 // the dust gradients of block j (rec: the ray's first record) from s0 = sum
@@ -148,6 +179,15 @@ template <typename T> struct AdjRay {
     T nu0, sf, cai;
 };
 
+// the channels cl .. cl + cnt - 1 that see the line on block j
+template <typename T>
+__device__ inline void block_channels(const AdjRay<T> &y, int j, T v0, T inv, int &cl, int &cnt) {
+    const float2 b = y.bounds[j];
+    if (b.x > b.y) return;
+    cl = channel_of<T>(y.velo, 0, y.nfr, b.x, false, ((T)b.x - v0) * inv);
+    cnt = max(0, channel_of<T>(y.velo, 0, y.nfr, b.y, true, ((T)b.y - v0) * inv + T(1)) - cl);
+}
+
 // a batch of pairs, a lane each: lane's block jl of the window that begins at
 // block jw, channel ch; on: the lane has a pair.  Blocks first .. last take part,
 // the pairs p0 .. pend-1.
@@ -165,14 +205,7 @@ __device__ __forceinline__ void pair_batch(AdjLds<T> &S, const AdjRay<T> &y, int
     // I before each of the block's segments, as the forward pass had it
     {
         FastCarryT<T> c;
-        const FastRecT<T> a = y.rec[max(kb - 1, 0)];
-        c.u0 = a.u;
-        if (j > 0) {
-            T jl0, al0, z_, phi_;
-            carried_in<T>(a, L, jl0, al0, z_, phi_);
-            carry_start<T>(point_of<T>(a), jl0, al0, c);
-            c.init = 0;
-        }
+        block_carry<T>(y.rec, j, L, c);
         int ovs = 0;
 #pragma unroll 1
         for (int i = 0; i < BLK; i++) {
@@ -257,6 +290,57 @@ __device__ __forceinline__ void pair_batch(AdjLds<T> &S, const AdjRay<T> &y, int
     flush(BLK + 1 - ADJ_ROWS - 1, BLK + 1 - ADJ_ROWS);
 }
 
+// forward: the maps of a ray's pairs, packed the same way (one wave), to outP and
+// outB [block][channel]
+template <typename T>
+__device__ __forceinline__ void adj_ray_maps(const AdjRay<T> &y, T *__restrict__ outP,
+                                             T *__restrict__ outB) {
+    const int lane = threadIdx.x & 63;
+    const T v0 = (T)y.velo[0], v1 = (T)y.velo[y.nfr - 1];
+    const T inv = y.nfr > 1 ? (T)(y.nfr - 1) / (v1 - v0) : T(0);
+    for (int jw = 0; jw < y.nb; jw += 64) {
+        const int m = min(64, y.nb - jw);
+        int cl = 0, cnt = 0;
+        if (lane < m) block_channels<T>(y, jw + lane, v0, inv, cl, cnt);
+        int incl = cnt;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int t = __shfl_up(incl, d);
+            if (lane >= d) incl += t;
+        }
+        const int st = incl - cnt, total = lane_of(incl, m - 1);
+#pragma unroll 1
+        for (int p0 = 0; p0 < total; p0 += 64) {
+            const int p = min(p0 + lane, total - 1);
+            int jl = 0;                       // the last block that begins at or before p
+            for (int d = 32; d >= 1; d >>= 1) {
+                const int t = __shfl(st, min(jl + d, 63));
+                if (jl + d < m && t <= p) jl += d;
+            }
+            const int ch = __shfl(cl, jl) + p - __shfl(st, jl);
+            const int j = jw + jl, kb = j * BLK;
+            const FastLineT<T> L{y.nu0, (T)y.dnu[ch], (T)y.velo[ch]};
+            const T ist = (T)y.istar[ch];
+            FastCarryT<T> c;
+            block_carry<T>(y.rec, j, L, c);
+            T B = T(0);
+            int ovs = 0;
+#pragma unroll 1
+            for (int i = 0; i < BLK; i++) {
+                const int k = kb + i;
+                if (k >= 1 && k < y.n) {
+                    const FastRecT<T> r = y.rec[k];
+                    segment_fast<T>(r, y.rec + k - 1, point_of<T>(r), L, B, ist, y.sf, c, ovs);
+                }
+            }
+            if (p0 + lane < total) {
+                const long long slot = (long long)j * y.nfr + ch;
+                outP[slot] = c.P;
+                outB[slot] = B;
+            }
+        }
+    }
+}
+
 // the node gradients of one ray (one wave)
 template <typename T>
 __device__ __forceinline__ void adj_ray(AdjLds<T> &S, const AdjRay<T> &y, int ngrp,
@@ -272,12 +356,7 @@ __device__ __forceinline__ void adj_ray(AdjLds<T> &S, const AdjRay<T> &y, int ng
         int cl = 0, cnt = 0;
         double s0 = 0.0, s1 = 0.0;
         if (lane < m) {
-            const float2 b = y.bounds[jw + lane];
-            if (!(b.x > b.y)) {
-                cl = channel_of<T>(y.velo, 0, y.nfr, b.x, false, ((T)b.x - v0) * inv);
-                cnt = max(0, channel_of<T>(y.velo, 0, y.nfr, b.y, true,
-                                           ((T)b.y - v0) * inv + T(1)) - cl);
-            }
+            block_channels<T>(y, jw + lane, v0, inv, cl, cnt);
             const double *s = y.bsum + (long long)(jw + lane) * ngrp * 2;
             for (int g = 0; g < ngrp; g++) {
                 s0 += s[2 * g];

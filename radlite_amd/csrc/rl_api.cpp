@@ -203,6 +203,7 @@ struct rl_ctx {
     std::vector<rl_item> tape_items;
     std::vector<double> tape_flux;
     unsigned long long tape_gen = 0;
+    unsigned long long pre_gen = 0;        // gen when rl_set_physics formed the tables
     int tape_kblk = 0;
     DevBuf d_stc_vals, d_stc_w, d_stc_off;    // a split item's chunk transpose
     DevBuf d_arec, d_ckpt, d_ckoff, d_gflux, d_gnode, d_gcell, d_grho, d_gabund, d_glw,
@@ -2073,16 +2074,18 @@ static int plan_adjoint(rl_ctx *c, const RaySet &rs, int nfr, bool tape, AdjPlan
 }
 
 // where a chunk's block checkpoints lie in its ckpt buffer: I, P and lambda per
-// (block, channel), the line-free sums per (block, 64 channels), the bounds
+// (block, channel), the line-free sums per (block, 64 channels), and per block
+// slot the dust maps and bounds
 struct AdjBlockBytes {
-    size_t ckP, lam, bsum, bounds, all;
-    AdjBlockBytes(long long nblk, int nfr, bool fp64) {
+    size_t ckP, lam, bsum, dust, bounds, all;
+    AdjBlockBytes(long long nblk, long long slots, int nfr, bool fp64) {
         const size_t n = (size_t)nblk * nfr * (fp64 ? 8 : 4);
         ckP = n;
         lam = 2 * n;
         bsum = (3 * n + 15) & ~(size_t)15;
-        bounds = bsum + (size_t)nblk * ((nfr + 63) / 64) * 16;
-        all = bounds + (size_t)nblk * 8;
+        dust = bsum + (size_t)nblk * ((nfr + 63) / 64) * 16;
+        bounds = dust + (size_t)slots * 16;
+        all = bounds + (size_t)slots * 8;
     }
 };
 
@@ -2105,12 +2108,14 @@ static void fill_adj(rl_ctx *c, const rl_item &it, const ItemSetup &su, AdjItemB
     a.rinfo = c->d_rinfo.as<RayInfo>();
     a.ckpt = ab.ckpt.p;
     a.kblk = K;
-    const AdjBlockBytes bb(ab.nblk, nfr, c->precision == RL_FP64);
+    const long long slots = rl::adjoint_block_slots(a.nnodes, a.nrays);
+    const AdjBlockBytes bb(ab.nblk, slots, nfr, c->precision == RL_FP64);
     char *base = ab.ckpt.as<char>();
     a.nblk = ab.nblk;
     a.ckP = base + bb.ckP;
     a.lam = base + bb.lam;
     a.bsum = reinterpret_cast<double *>(base + bb.bsum);
+    a.dust = base + bb.dust;
     a.bounds = base + bb.bounds;
     a.dnu = c->d_chan.as<double>();
     a.velo = a.dnu + nfr;
@@ -2173,17 +2178,23 @@ static int adj_forward_chunk(rl_ctx *c, const rl_item &it, const ItemSetup &su, 
         const long long n = rs.off[ch.r0 + r + 1] - rs.off[ch.r0 + r];
         ckoff[r + 1] = ckoff[r] + (n >= 2 ? (n - 1 + K - 1) / K : 0);
     }
-    // I before every segment (K = 1) is held, but by blocks: I at their starts is
-    // enough for the reverse sweep by pairs (fit on the 200 x 100 disk, FP32, 20.2 ->
-    // 12.9 ms), in less memory unless the rays are a few nodes long.  An interval of more
-    // segments is asked for or taken to save memory, and keeps its own layout.
+    // I before every segment (K = 1) held, and the tables formed on the device from
+    // the physics (rl_set_physics): by blocks, I at their starts being enough for
+    // the reverse sweep by pairs (fit on the 200 x 100 disk, FP32, 20.2 -> 11.5
+    // ms), in less memory unless the rays are a few nodes long.  The gradients on
+    // T, abundance and v_turb are the same to rounding.  Those on tables that a
+    // caller set keep the sweep by segments: in nearly empty cells dL/d rho and
+    // dL/d alpha are differences that cancel to 1e-6 (FP64) and, in FP32, to
+    // nothing, so that any other order of summation is seen there.  An interval of
+    // more segments is asked for or taken to save memory, with its own layout.
     size_t bytes = (size_t)ckoff[nr] * nfr * tsz;
+    const long long slots = rl::adjoint_block_slots(ch.n1 - ch.n0, nr);
     ab.nblk = 0;
-    if (K == 1) {
+    if (K == 1 && c->pre_ready && c->pre_gen == c->gen) {
         std::vector<long long> bo(nr + 1, 0);
         for (int r = 0; r < nr; r++)
             bo[r + 1] = bo[r] + rl::adjoint_ray_blocks(rs.off[ch.r0 + r + 1] - rs.off[ch.r0 + r]);
-        const AdjBlockBytes bb(bo[nr], nfr, c->precision == RL_FP64);
+        const AdjBlockBytes bb(bo[nr], slots, nfr, c->precision == RL_FP64);
         if (bo[nr] && bb.all <= bytes) {
             ab.nblk = bo[nr];
             ckoff.swap(bo);
@@ -2749,6 +2760,7 @@ extern "C" int rl_set_physics(rl_ctx *c, const double *T_gas, const double *T_du
     c->aksmax = mx;                          // line.F:3020-3033 (widths > 0 here)
     c->have_dust = true;
     c->pre_ready = 1;
+    c->pre_gen = c->gen;
     c->cells_line = -1;
     return 0;
 }

@@ -132,7 +132,8 @@ struct AdjLaunch {
     // starts; nblk 0: checkpoints every kblk segments
     long long nblk;                    // blocks of the chunk
     void *ckP, *lam;                   // T[nblk][nfr]: factor of a block, lambda at its end
-    void *bounds;                      // float2[nblk]
+    void *bounds, *dust;               // float2, double2 [adjoint_block_slots]: a ray's
+                                       // blocks from blk_of(its first node, ray)
     double *bsum;                      // [nblk][ceil(nfr/64)][2]
     const double *dnu, *velo, *istar;  // per channel
     const double *i0;                  // per channel: outer boundary intensity
@@ -226,6 +227,7 @@ template <typename T> void launch_adjoint_fwd(hipStream_t st, const AdjLaunch &a
 template <typename T> void launch_adjoint_rev(hipStream_t st, const AdjLaunch &a);
 void launch_adjoint_flux(hipStream_t st, const AdjLaunch &a);
 int adjoint_block_len();
+long long adjoint_block_slots(long long nodes, int rays);
 long long adjoint_ray_blocks(long long nodes);   // blocks of a ray of so many nodes
 // Stencil transpose (cell -> node entries) of a node set; with temp ==
 // nullptr only *temp_bytes is set.  keys/vals: 4*nnodes ints each (a, b);

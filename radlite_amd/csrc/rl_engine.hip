@@ -1508,15 +1508,14 @@ int formal_blocks_per_cu(int fp64) {
 // lane per (ray, channel), keeping I before every kblk-th segment.  A call
 // covers rays ray0.. of the ray set (a chunk): off is the chunk's slice of
 // the node CSR (global node indices), rec, ckoff, ckpt and image are the
-// chunk's own, node0 its first node.  BLOCKS: I before every block's first
-// segment, and in ckP the block's factor dI_out/dI_in.
-template <typename T, bool BLOCKS>
+// chunk's own, node0 its first node.
+template <typename T>
 __global__ void __launch_bounds__(256)
 k_adj_fwd(int nrays, int nfr, int ray0, long long node0, const long long *__restrict__ off,
           const long long *__restrict__ ckoff, const FastRecT<T> *__restrict__ rec,
           const double *__restrict__ dnu, const double *__restrict__ velo,
           const double *__restrict__ istar, const double *__restrict__ i0, LineConst lc,
-          double *__restrict__ image, T *__restrict__ ckpt, T *__restrict__ ckP, int kblk) {
+          double *__restrict__ image, T *__restrict__ ckpt, int kblk) {
     const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= (long long)nrays * nfr) return;
     const int ray = (int)(g / nfr), ch = (int)(g - (long long)ray * nfr);
@@ -1534,24 +1533,17 @@ k_adj_fwd(int nrays, int nfr, int ray0, long long node0, const long long *__rest
     // (a countdown: a remainder by the run-time kblk costs an emulated
     // division per segment)
     T *ck = ckpt + ckoff[ray] * nfr + ch;
-    T *cp = BLOCKS ? ckP + ckoff[ray] * nfr + ch : nullptr;
     int until = 0;                           // segments until the next checkpoint
     for (int k = 1; k < n; k++) {
-        if (BLOCKS ? k == 1 || (k & (BLK - 1)) == 0 : until == 0) {
+        if (until == 0) {
             *ck = I;
             ck += nfr;
             until = kblk;
-            if (BLOCKS && k > 1) {
-                *cp = c.P;
-                cp += nfr;
-                c.P = T(1);
-            }
         }
         until--;
         const FastRecT<T> r = rec[b + k];
         segment_fast<T>(r, rec + b + k - 1, point_of<T>(r), L, I, ist, sf, c, ovs);
     }
-    if (BLOCKS) *cp = c.P;
     image[g] = (double)I;
 }
 
@@ -1783,9 +1775,89 @@ __global__ void __launch_bounds__(64)
 k_adj_bounds(AdjLaunch a) {
     const int ray = blockIdx.x;
     const long long b = a.off[ray] - a.node0;
-    adj_bounds<T>(threadIdx.x, reinterpret_cast<const FastRecT<T> *>(a.rec) + b,
-                  (int)(a.off[ray + 1] - a.off[ray]), (int)(a.ckoff[ray + 1] - a.ckoff[ray]),
-                  (T)a.lc.nu0, reinterpret_cast<float2 *>(a.bounds) + a.ckoff[ray]);
+    const int n = (int)(a.off[ray + 1] - a.off[ray]);
+    adj_bounds<T>(threadIdx.x, reinterpret_cast<const FastRecT<T> *>(a.rec) + b, n,
+                  n >= 2 ? ((n - 1) >> BLK_LOG) + 1 : 0, (T)a.lc.nu0,
+                  reinterpret_cast<float2 *>(a.bounds) + blk_of(b, ray),
+                  reinterpret_cast<double2 *>(a.dust) + blk_of(b, ray));
+}
+
+// a wave's ray of an adjoint launch
+template <typename T>
+__device__ __forceinline__ AdjRay<T> adj_ray_of(const AdjLaunch &a, int ray, int ngrp) {
+    const long long b = a.off[ray] - a.node0, o = a.ckoff[ray];
+    AdjRay<T> y;
+    y.rec = reinterpret_cast<const FastRecT<T> *>(a.rec) + b;
+    y.n = (int)(a.off[ray + 1] - a.off[ray]);
+    y.nb = (int)(a.ckoff[ray + 1] - o);
+    y.nfr = a.nfr;
+    y.bounds = reinterpret_cast<const float2 *>(a.bounds) + blk_of(b, ray);
+    y.ckI = reinterpret_cast<const T *>(a.ckpt) + o * a.nfr;
+    y.lam = reinterpret_cast<const T *>(a.lam) + o * a.nfr;
+    y.bsum = a.bsum + o * ngrp * 2;
+    y.dnu = a.dnu;
+    y.velo = a.velo;
+    y.istar = a.istar;
+    y.nu0 = (T)a.lc.nu0;
+    y.sf = a.ray0 + ray == 0 ? (T)a.lc.starfract : T(0);
+    y.cai = (T)a.lc.c_aa;
+    return y;
+}
+
+// forward by blocks, I carried in double: the maps of the pairs that see the line (P into ckP, the
+// constant into ckpt), then one pass along the blocks that leaves I before each
+// block in ckpt and every channel's factor in ckP.  200 x 100 disk, 100
+// channels, FP32: a fit 12.9 -> 11.5 ms by it; 40 x 24 disk, 24 channels, FP64:
+// 1.21 -> 0.96 ms.
+template <typename T>
+__global__ void __launch_bounds__(64)
+k_adj_maps(AdjLaunch a) {
+    const int ray = blockIdx.x;
+    const AdjRay<T> y = adj_ray_of<T>(a, ray, 1);
+    if (y.nb <= 0) return;
+    const long long o = a.ckoff[ray] * a.nfr;
+    adj_ray_maps<T>(y, reinterpret_cast<T *>(a.ckP) + o, reinterpret_cast<T *>(a.ckpt) + o);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(64)
+k_adj_chain(AdjLaunch a) {
+    const int ray = blockIdx.x, ch = blockIdx.y * 64 + threadIdx.x, nfr = a.nfr;
+    if (ch >= nfr) return;
+    const long long b = a.off[ray] - a.node0, o = a.ckoff[ray];
+    const int nb = (int)(a.ckoff[ray + 1] - o);
+    double I = a.i0[ch];
+    const T v = (T)a.velo[ch];
+    T *pi = reinterpret_cast<T *>(a.ckpt) + o * nfr + ch;
+    T *pp = reinterpret_cast<T *>(a.ckP) + o * nfr + ch;
+    const float2 *bd = reinterpret_cast<const float2 *>(a.bounds) + blk_of(b, ray);
+    const double2 *dust = reinterpret_cast<const double2 *>(a.dust) + blk_of(b, ray);
+    constexpr int AHEAD = 8;             // the loads of as many blocks at a time
+    for (int j0 = 0; j0 < nb; j0 += AHEAD) {
+        double P[AHEAD], Q[AHEAD];
+        bool seen[AHEAD];
+#pragma unroll
+        for (int q = 0; q < AHEAD; q++) {
+            const int j = min(j0 + q, nb - 1);
+            seen[q] = sees<T>(bd[j], v);
+            const double2 d = dust[j];
+            P[q] = d.x;
+            Q[q] = d.y;
+            if (seen[q]) {
+                P[q] = (double)pp[(long long)j * nfr];
+                Q[q] = (double)pi[(long long)j * nfr];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < AHEAD; q++) {
+            const int j = j0 + q;
+            if (j >= nb) break;
+            pi[(long long)j * nfr] = (T)I;
+            if (!seen[q]) pp[(long long)j * nfr] = (T)P[q];
+            I = I * P[q] + Q[q];
+        }
+    }
+    a.image[(long long)ray * nfr + ch] = I;
 }
 
 // lambda at the end of every block, backwards over a ray's blocks, and the sums
@@ -1810,7 +1882,8 @@ k_adj_lambda(AdjLaunch a, int ngrp) {
     const T *I = reinterpret_cast<const T *>(a.ckpt) + o * nfr + chc;
     const T *P = reinterpret_cast<const T *>(a.ckP) + o * nfr + chc;
     T *out = reinterpret_cast<T *>(a.lam) + o * nfr + chc;
-    const float2 *bd = reinterpret_cast<const float2 *>(a.bounds) + o;
+    const float2 *bd = reinterpret_cast<const float2 *>(a.bounds) +
+                       blk_of(a.off[ray] - a.node0, ray);
     constexpr int AHEAD = 4;
     T pi[AHEAD], pp[AHEAD];
 #pragma unroll
@@ -1830,7 +1903,7 @@ k_adj_lambda(AdjLaunch a, int ngrp) {
             pp[q] = P[nx * nfr];
             if (active) out[(long long)j * nfr] = (T)lam;
             const float2 b = bd[j];
-            const bool seen = !(b.x > b.y) && !(v < (T)b.x) && v <= (T)b.y;
+            const bool seen = sees<T>(b, v);
             double s0 = 0.0, s1 = 0.0;
             if (__any(active && !seen)) {
                 s0 = seen ? 0.0 : lam;
@@ -1859,25 +1932,9 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AdjPair
 k_adj_pairs(AdjLaunch a, int ngrp) {
     __shared__ AdjLds<T> lds;
     const int ray = blockIdx.x;
-    const long long b = a.off[ray] - a.node0, o = a.ckoff[ray];
-    const int nb = (int)(a.ckoff[ray + 1] - o);
-    if (nb <= 0) return;
-    AdjRay<T> y;
-    y.rec = reinterpret_cast<const FastRecT<T> *>(a.rec) + b;
-    y.n = (int)(a.off[ray + 1] - a.off[ray]);
-    y.nb = nb;
-    y.nfr = a.nfr;
-    y.bounds = reinterpret_cast<const float2 *>(a.bounds) + o;
-    y.ckI = reinterpret_cast<const T *>(a.ckpt) + o * a.nfr;
-    y.lam = reinterpret_cast<const T *>(a.lam) + o * a.nfr;
-    y.bsum = a.bsum + o * ngrp * 2;
-    y.dnu = a.dnu;
-    y.velo = a.velo;
-    y.istar = a.istar;
-    y.nu0 = (T)a.lc.nu0;
-    y.sf = a.ray0 + ray == 0 ? (T)a.lc.starfract : T(0);
-    y.cai = (T)a.lc.c_aa;
-    adj_ray<T>(lds, y, ngrp, a.gnode + b * 5);
+    const AdjRay<T> y = adj_ray_of<T>(a, ray, ngrp);
+    if (y.nb <= 0) return;
+    adj_ray<T>(lds, y, ngrp, a.gnode + (a.off[ray] - a.node0) * 5);
 }
 
 // ---- node -> cell transpose of the interpolation stencil (once per ray set)
@@ -2005,21 +2062,17 @@ int build_stencil_transpose(hipStream_t st, long long nnodes, const GeoNode *geo
 template <typename T>
 void launch_adjoint_fwd(hipStream_t st, const AdjLaunch &a) {
     auto *rec = reinterpret_cast<FastRecT<T> *>(a.rec);
-    auto *ck = reinterpret_cast<T *>(a.ckpt);
     hipLaunchKernelGGL(k_nodes_fast<T>, dim3(a.nrays), dim3(64), 0, st, a.nrays, a.off, a.geo,
                        a.cells, rec, a.node0, a.rinfo, a.nfr, a.velo, a.aks2, 1, a.lc);
-    const long long total = (long long)a.nrays * a.nfr;
-    auto *cp = reinterpret_cast<T *>(a.ckP);
-    const dim3 grid((unsigned)((total + 255) / 256));
     if (a.nblk) {
         hipLaunchKernelGGL(k_adj_bounds<T>, dim3(a.nrays), dim3(64), 0, st, a);
-        hipLaunchKernelGGL((k_adj_fwd<T, true>), grid, dim3(256), 0, st, a.nrays, a.nfr, a.ray0,
-                           a.node0, a.off, a.ckoff, rec, a.dnu, a.velo, a.istar, a.i0, a.lc,
-                           a.image, ck, cp, a.kblk);
+        hipLaunchKernelGGL(k_adj_maps<T>, dim3(a.nrays), dim3(64), 0, st, a);
+        hipLaunchKernelGGL(k_adj_chain<T>, dim3(a.nrays, (a.nfr + 63) / 64), dim3(64), 0, st, a);
     } else {
-        hipLaunchKernelGGL((k_adj_fwd<T, false>), grid, dim3(256), 0, st, a.nrays, a.nfr, a.ray0,
-                           a.node0, a.off, a.ckoff, rec, a.dnu, a.velo, a.istar, a.i0, a.lc,
-                           a.image, ck, cp, a.kblk);
+        const long long total = (long long)a.nrays * a.nfr;
+        hipLaunchKernelGGL(k_adj_fwd<T>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
+                           a.nrays, a.nfr, a.ray0, a.node0, a.off, a.ckoff, rec, a.dnu, a.velo,
+                           a.istar, a.i0, a.lc, a.image, reinterpret_cast<T *>(a.ckpt), a.kblk);
     }
 }
 
@@ -2065,6 +2118,7 @@ template void launch_adjoint_rev<double>(hipStream_t, const AdjLaunch &);
 template void launch_adjoint_rev<float>(hipStream_t, const AdjLaunch &);
 
 int adjoint_block_len() { return ADJ_K; }
+long long adjoint_block_slots(long long nodes, int rays) { return (nodes >> BLK_LOG) + rays + 1; }
 long long adjoint_ray_blocks(long long n) { return n >= 2 ? ((n - 1) >> BLK_LOG) + 1 : 0; }
 size_t fast_rec_size(int fp64) { return fp64 ? sizeof(FastRecT<double>) : sizeof(FastRecT<float>); }
 
