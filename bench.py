@@ -53,7 +53,7 @@ def measured_valu_issue(precision):
     if not os.path.exists(path):
         return None
     for line in open(path):
-        if "VALU wave-instructions per CU-cycle" in line:
+        if "k_formal VALU wave-instructions per CU-cycle" in line:
             return float(line.split("=")[1].split()[0]) / 2.0
     return None
 
@@ -268,7 +268,7 @@ def bench_batched(args):
     channels each, 8 inclinations (512 items, 17,025 rays each); one step
     = ray sets and trajectories for the 8 inclinations + every item's
     spectrum in one rl_trace_lines_forward call (batches sized to HBM,
-    persistent formal kernel, graph replay, autotuned tiles)."""
+    graph replay)."""
     from radlite_amd import engine, synth
     ri, items, incl = synth.c3_inputs(0)
     incs = [x * 0.0174532925199 for x in incl]
@@ -565,7 +565,7 @@ def main():
     flops_per_rc = 40.0 * nseg
     peak_tf = FP32_PEAK_TFLOPS if args.precision == "fp32" else FP64_PEAK_TFLOPS
     achieved_tf = flops_per_rc * nominal / formal_s / 1e12
-    kname = "k_formal_batch" if tile_blocks else "k_formal_tiles"
+    kname = "k_formal"
     traffic = measured_traffic(args.precision, kname) if args.workload == "c2" else None
     hbm_gbs = traffic * nbatch / formal_s / 1e9 if traffic is not None else None
 
