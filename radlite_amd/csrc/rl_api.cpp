@@ -255,11 +255,11 @@ static int fail(rl_ctx *c, int code, const char *fmt, ...) {
 // thread to a slot: each moves every n-th piece, so that the threads' copies (and
 // the page faults of a fresh array, which cost more than the bus) run beside the
 // transfers.  The runtime's own way for such an array is one thread's.
-// 300 x 300 pixels x 100 channels from 34,049 rays (27 MB up, 72 MB down): 8.1 ->
-// 3.7 ms a call; two cubes of 52 MB: 13.1 -> 12.2 ms a call.  Eight threads and
-// arrays from 4 MB on got in the way of a program that itself computes on many
-// threads between calls: an image of 7 MB 2.0 -> 4.6 ms, the cubes 16.8 ms; at
-// 7 MB four threads gain nothing.
+// Resampling only, 300 x 300 pixels x 100 channels from 34,049 rays (27 MB up, 72
+// MB down): 8.1 -> 3.6 ms a call.  Image cubes keep the runtime's way: a program
+// that works on a cube with many threads of its own finds these in its way (two
+// cubes of 52 MB: 13.1 ms as they are, 12.2 to 15 with four threads, 16.8 with
+// eight; an image of 7 MB 2.0, 2.1 and 4.6).
 static bool pageable(const void *p) {
     hipPointerAttribute_t a;
     if (hipPointerGetAttributes(&a, p) != hipSuccess) {
@@ -318,7 +318,7 @@ static hipError_t copy_up(rl_ctx *c, void *dst, const void *src, size_t bytes) {
 
 static int upload(rl_ctx *c, DevBuf &b, const void *src, size_t bytes) {
     HIPCHK(c, b.ensure(bytes));
-    HIPCHK(c, copy_up(c, b.p, src, bytes));
+    HIPCHK(c, hipMemcpyAsync(b.p, src, bytes, hipMemcpyHostToDevice, c->stream));
     return 0;
 }
 
@@ -1473,8 +1473,11 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
     HIPCHK(c, hipMemcpyAsync(flux + fo, c->d_flux.p, (size_t)flux0 * 8, hipMemcpyDeviceToHost,
                              c->stream));
     if (image)
-        HIPCHK(c, copy_down(c, image + io, c->d_image.p, (size_t)img0 * 8));
-    if (cmask) HIPCHK(c, copy_down(c, cmask + io, c->d_cmask.p, (size_t)img0));
+        HIPCHK(c, hipMemcpyAsync(image + io, c->d_image.p, (size_t)img0 * 8,
+                                 hipMemcpyDeviceToHost, c->stream));
+    if (cmask)
+        HIPCHK(c, hipMemcpyAsync(cmask + io, c->d_cmask.p, (size_t)img0, hipMemcpyDeviceToHost,
+                                 c->stream));
     std::vector<unsigned long long> ovs(nb);
     std::vector<int> maser(nb + 1);
     HIPCHK(c, hipMemcpyAsync(ovs.data(), L.ovs, (size_t)nb * 8, hipMemcpyDeviceToHost,
@@ -1810,7 +1813,8 @@ extern "C" int rl_resample_image(rl_ctx *c, int nrays, int nfr, const double *im
     if (npix == 0) return 0;
     HIPCHK(c, hipSetDevice(c->device));
     DevBuf &d_img = c->d_rs_img, &d_vtx = c->d_rs_vtx, &d_w = c->d_rs_w, &d_out = c->d_rs_out;
-    if (int e = upload(c, d_img, image, (size_t)nrays * nfr * 8)) return e;
+    HIPCHK(c, d_img.ensure((size_t)nrays * nfr * 8));
+    HIPCHK(c, copy_up(c, d_img.p, image, (size_t)nrays * nfr * 8));
     if (int e = upload(c, d_vtx, vtx, nvt * 4)) return e;
     if (int e = upload(c, d_w, w, nvt * 8)) return e;
     HIPCHK(c, d_out.ensure((size_t)npix * nfr * 8));
@@ -1908,8 +1912,8 @@ extern "C" int rl_trace_lines_posvel(rl_ctx *c, int nitems, const rl_item *items
         double *oi = image + io, *ot = tau ? tau + io : nullptr;
         cen.assign(nextra ? nextra : 1, 0.0);
         unsigned long long flags[2] = {0, 0};
-        HIPCHK(c, copy_down(c, oi, L.image, npv * 8));
-        if (ot) HIPCHK(c, copy_down(c, ot, L.tau, npv * 8));
+        HIPCHK(c, hipMemcpyAsync(oi, L.image, npv * 8, hipMemcpyDeviceToHost, c->stream));
+        if (ot) HIPCHK(c, hipMemcpyAsync(ot, L.tau, npv * 8, hipMemcpyDeviceToHost, c->stream));
         if (nextra)
             HIPCHK(c, hipMemcpyAsync(cen.data(), L.extra, nextra * 8, hipMemcpyDeviceToHost,
                                      c->stream));
