@@ -96,7 +96,7 @@ __device__ inline void adj_bounds(int lane, const FastRecT<T> *__restrict__ rec,
 
 // whether channel velocity v sees the line on a block of bounds b
 template <typename T> __device__ inline bool sees(float2 b, T v) {
-    return !(b.x > b.y) && !(v < (T)b.x) && v <= (T)b.y;
+    return !(b.x > b.y) && !(v < (T)b.x) && !(v > (T)b.y);
 }
 
 // the carry at the start of block j of a ray (rec: its first record)
@@ -184,8 +184,7 @@ template <typename T>
 __device__ inline void block_channels(const AdjRay<T> &y, int j, T v0, T inv, int &cl, int &cnt) {
     const float2 b = y.bounds[j];
     if (b.x > b.y) return;
-    cl = channel_of<T>(y.velo, 0, y.nfr, b.x, false, ((T)b.x - v0) * inv);
-    cnt = max(0, channel_of<T>(y.velo, 0, y.nfr, b.y, true, ((T)b.y - v0) * inv + T(1)) - cl);
+    channels_in<T>(y.velo, 0, y.nfr, v0, inv, b.x, b.y, cl, cnt);
 }
 
 // a batch of pairs, a lane each: lane's block jl of the window that begins at

@@ -80,17 +80,26 @@ __device__ inline double lane_of(double v, int lane) {
 __device__ inline double mark(double P, bool ovf) { return copysign(P, ovf ? -1.0 : 1.0); }
 __device__ inline bool marked(double P) { return __double2hiint(P) < 0; }
 
-// the first channel of [c0, c1) whose velocity is not below x (above: not at or
-// below it), v ascending; est: its position if the channels were exactly even
+// the channels of [c0, c1) whose velocity lies in [lo, hi]: their first, cl, and
+// number, cnt.  v ascends, or descends for a line of negative rest frequency (v =
+// dnu/nu0), or is no number (a passband without end): such a channel is taken.
+// v0: v[c0]; inv: channels per velocity (negative descending, 0 for one channel).
 template <typename T>
-__device__ inline int channel_of(const double *__restrict__ v, int c0, int c1, float x, bool above,
-                                 T est) {
-    int c = (int)fmin(fmax(est, (T)c0), (T)c1);
-    const T b = (T)x;
-    auto before = [&](int k) { const T u = (T)v[k]; return above ? u <= b : u < b; };
-    while (c > c0 && !before(c - 1)) c--;
-    while (c < c1 && before(c)) c++;
-    return c;
+__device__ inline void channels_in(const double *__restrict__ v, int c0, int c1, T v0, T inv,
+                                   float lo, float hi, int &cl, int &cnt) {
+    const T s = inv < T(0) ? T(-1) : T(1);       // s v ascends
+    const T b0 = s * (T)(inv < T(0) ? hi : lo), b1 = s * (T)(inv < T(0) ? lo : hi);
+    // the number of channels that come before the bound, from where it would lie
+    // if the channels were exactly even
+    auto bound = [&](T est, auto before) {
+        int c = (int)fmin(fmax(est, (T)c0), (T)c1);
+        while (c > c0 && !before(c - 1)) c--;
+        while (c < c1 && before(c)) c++;
+        return c;
+    };
+    cl = bound((T)c0 + (s * b0 - v0) * inv, [&](int k) { return s * (T)v[k] < b0; });
+    cnt = max(0, bound((T)c0 + (s * b1 - v0) * inv + T(1),
+                       [&](int k) { return !(s * (T)v[k] > b1); }) - cl);
 }
 
 // the channels of a chunk as a wave holds them
@@ -128,12 +137,8 @@ __device__ __forceinline__ void walk(WalkLds<T> &S, const BlkRec *__restrict__ b
                 lo = r->lo; hi = r->hi; bA = r->A; bB = r->B;
                 nov = __float_as_int(lo) & (2 * BLK - 1);
             }
-            if (!(lo > hi)) {        // (-inf with an overshoot count is NaN)
-                cl = channel_of<T>(ch.velo, ch.c0, ch.c1, lo, false,
-                                   (T)ch.c0 + ((T)lo - v0) * inv);
-                cnt = max(0, channel_of<T>(ch.velo, ch.c0, ch.c1, hi, true,
-                                           (T)ch.c0 + ((T)hi - v0) * inv + T(1)) - cl);
-            }
+            if (!(lo > hi))          // (-inf with an overshoot count is NaN)
+                channels_in<T>(ch.velo, ch.c0, ch.c1, v0, inv, lo, hi, cl, cnt);
         }
         int incl = cnt;                          // pairs up to and with the lane's block
         for (int d = 1; d < RECS; d <<= 1) {
