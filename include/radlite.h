@@ -205,6 +205,9 @@ int rl_trace_lines_adjoint(rl_ctx *ctx, int nitems, const rl_item *items,
  * half of a training step.  flux as in rl_trace_lines_forward.  The tape
  * replaces the previous one and is dropped by rl_tape_release or
  * rl_destroy; any rl_set_* or rl_setup_rays_circular call makes it stale.
+ * With the tables of rl_set_physics and K = 1 it is taken by blocks (see
+ * rl_last_adjoint_pairs); the first rl_trace_lines_adjoint call that asks
+ * for a table's gradient retakes it by segments, and it stays so.
  * No counterpart in the reference (its trace has no adjoint). */
 int rl_trace_lines_forward_tape(rl_ctx *ctx, int nitems, const rl_item *items,
                                 double *flux);
@@ -217,6 +220,18 @@ int rl_tape_release(rl_ctx *ctx);
  * a range of rays at a time; the tape needs every item whole). */
 int rl_last_adjoint_info(const rl_ctx *ctx, int *ckpt_interval, int *used_tape,
                          int *chunks);
+
+/* How many blocks of 8 segments (summed over the items' rays) the last
+ * rl_trace_lines_adjoint call reversed by independent (block, channel)
+ * pairs; 0: it stepped every channel through every segment.  By pairs is
+ * taken where every table output is NULL, so that the gradients go on to
+ * rl_physics_adjoint alone, the tables are those of the last
+ * rl_set_physics (no rl_set_grid, _medium, _levels, _lines or _dust_line
+ * since) and the interval is 1.  The gradients on the physical fields are
+ * then the same to rounding, but for the line's own share of a block where
+ * its profile is below 2^-30 (FP32; FP64 2^-60) of the dust in every
+ * channel: that share is 0. */
+int rl_last_adjoint_pairs(const rl_ctx *ctx, long long *blocks);
 
 /* Device memory: out[0] the budget, out[1] bytes held by resident
  * trajectories (and adjoint transposes), out[2] work bytes of the last

@@ -191,6 +191,7 @@ struct rl_ctx {
     bool use_graph = true;
     int fixed_cw = -1, fixed_persistent = 1, last_cw = 0, last_blocks = 0, last_batches = 0;
     int last_kblk = 0, fixed_kblk = 0, last_used_tape = 0;
+    long long last_pair_blocks = 0;
     // inputs generation: bumped by every setter, so that a tape taken
     // before a change is not used after it
     unsigned long long gen = 1;
@@ -203,7 +204,9 @@ struct rl_ctx {
     std::vector<rl_item> tape_items;
     std::vector<double> tape_flux;
     unsigned long long tape_gen = 0;
-    unsigned long long pre_gen = 0;        // gen when rl_set_physics formed the tables
+    // the tables are those that rl_set_physics formed: cleared by the setters
+    // that replace one of them
+    bool phys_tables = false;
     int tape_kblk = 0;
     DevBuf d_stc_vals, d_stc_w, d_stc_off;    // a split item's chunk transpose
     DevBuf d_arec, d_ckpt, d_ckoff, d_gflux, d_gnode, d_gcell, d_grho, d_gabund, d_glw,
@@ -382,6 +385,7 @@ extern "C" int rl_last_stats(const rl_ctx *c, double *t, long long *n) {
 // ---------------------------------------------------------------------
 extern "C" int rl_set_grid(rl_ctx *c, int nr, const double *r, int nh, const double *th) {
     if (c) c->gen++;                         // invalidates a tape
+    if (c) c->phys_tables = false;
     if (!c || !r || !th || nr < 3 || nh < 2) return fail(c, RL_E_ARG, "rl_set_grid: bad args");
     HIPCHK(c, hipSetDevice(c->device));
     for (int i = 1; i < nr; i++)
@@ -431,6 +435,7 @@ extern "C" int rl_set_medium(rl_ctx *c, const double *rho, const double *abund,
                              const double *vel, const double *lw, double umass_av,
                              double aksmax) {
     if (c) c->gen++;                         // invalidates a tape
+    if (c) c->phys_tables = false;
     if (!c || !c->nr) return fail(c, RL_E_ARG, "rl_set_medium: set the grid first");
     if (!rho || !abund || !vel || !lw || !(umass_av > 0.0))
         return fail(c, RL_E_ARG, "rl_set_medium: bad args");
@@ -458,6 +463,7 @@ extern "C" int rl_set_medium(rl_ctx *c, const double *rho, const double *abund,
 
 extern "C" int rl_set_levels(rl_ctx *c, int nlev, const double *pops) {
     if (c) c->gen++;                         // invalidates a tape
+    if (c) c->phys_tables = false;
     if (!c || !c->nr || nlev < 2 || !pops) return fail(c, RL_E_ARG, "rl_set_levels: bad args");
     HIPCHK(c, hipSetDevice(c->device));
     c->nlev = nlev;
@@ -470,6 +476,7 @@ extern "C" int rl_set_levels(rl_ctx *c, int nlev, const double *pops) {
 extern "C" int rl_set_lines(rl_ctx *c, int nl, const double *nu0, const double *A,
                             const double *gu, const double *gl, const int *lu, const int *ll) {
     if (c) c->gen++;                         // invalidates a tape
+    if (c) c->phys_tables = false;
     if (!c || nl < 1 || !nu0 || !A || !gu || !gl || !lu || !ll)
         return fail(c, RL_E_ARG, "rl_set_lines: bad args");
     for (int i = 0; i < nl; i++) {                           // line.F:1739-1770
@@ -492,6 +499,7 @@ extern "C" int rl_set_lines(rl_ctx *c, int nl, const double *nu0, const double *
 
 extern "C" int rl_set_dust_line(rl_ctx *c, const double *jd, const double *ad) {
     if (c) c->gen++;                         // invalidates a tape
+    if (c) c->phys_tables = false;
     if (!c || !c->nr || !c->nlines || !jd || !ad)
         return fail(c, RL_E_ARG, "rl_set_dust_line: set grid and lines first");
     HIPCHK(c, hipSetDevice(c->device));
@@ -2171,9 +2179,10 @@ static int adj_setup(rl_ctx *c, const rl_item &it, int ii, ItemSetup &su, size_t
     return 0;
 }
 
-// the checkpointed forward of one chunk: node records, I every K segments
+// the checkpointed forward of one chunk: node records, I every K segments, or
+// (blocks, where it is possible) by blocks for the reverse sweep by pairs
 static int adj_forward_chunk(rl_ctx *c, const rl_item &it, const ItemSetup &su, int K,
-                             const AdjChunk &ch, AdjItemBufs &ab) {
+                             const AdjChunk &ch, AdjItemBufs &ab, bool blocks) {
     const RaySet &rs = *su.rs;
     const int nfr = it.nfr, nr = ch.r1 - ch.r0;
     const size_t tsz = c->precision == RL_FP64 ? 8 : 4;
@@ -2182,19 +2191,14 @@ static int adj_forward_chunk(rl_ctx *c, const rl_item &it, const ItemSetup &su, 
         const long long n = rs.off[ch.r0 + r + 1] - rs.off[ch.r0 + r];
         ckoff[r + 1] = ckoff[r] + (n >= 2 ? (n - 1 + K - 1) / K : 0);
     }
-    // I before every segment (K = 1) held, and the tables formed on the device from
-    // the physics (rl_set_physics): by blocks, I at their starts being enough for
-    // the reverse sweep by pairs (fit on the 200 x 100 disk, FP32, 20.2 -> 11.5
-    // ms), in less memory unless the rays are a few nodes long.  The gradients on
-    // T, abundance and v_turb are the same to rounding.  Those on tables that a
-    // caller set keep the sweep by segments: in nearly empty cells dL/d rho and
-    // dL/d alpha are differences that cancel to 1e-6 (FP64) and, in FP32, to
-    // nothing, so that any other order of summation is seen there.  An interval of
-    // more segments is asked for or taken to save memory, with its own layout.
+    // By blocks: I before every segment (K = 1) would fit, I at the blocks' starts
+    // is enough for the reverse sweep by pairs (fit on the 200 x 100 disk, FP32, 20.2
+    // -> 11.5 ms), in less memory unless the rays are a few nodes long.  An interval
+    // of more segments is asked for or taken to save memory, with its own layout.
     size_t bytes = (size_t)ckoff[nr] * nfr * tsz;
     const long long slots = rl::adjoint_block_slots(ch.n1 - ch.n0, nr);
     ab.nblk = 0;
-    if (K == 1 && c->pre_ready && c->pre_gen == c->gen) {
+    if (K == 1 && blocks) {
         std::vector<long long> bo(nr + 1, 0);
         for (int r = 0; r < nr; r++)
             bo[r + 1] = bo[r] + rl::adjoint_ray_blocks(rs.off[ch.r0 + r + 1] - rs.off[ch.r0 + r]);
@@ -2342,7 +2346,7 @@ extern "C" int rl_trace_lines_forward_tape(rl_ctx *c, int nitems, const rl_item 
         ItemSetup su;
         if (int e = adj_setup(c, it, ii, su, 0)) return e;
         const AdjChunk whole{0, su.rs->nrays, 0, su.rs->nnodes};
-        if (int e = adj_forward_chunk(c, it, su, Kt, whole, c->tape[ii])) return e;
+        if (int e = adj_forward_chunk(c, it, su, Kt, whole, c->tape[ii], c->phys_tables)) return e;
         if (int e = adj_flux(c, it, su, c->tape_flux.data() + fo)) return e;
         fo += it.nfr;
     }
@@ -2380,6 +2384,14 @@ extern "C" int rl_trace_lines_adjoint(rl_ctx *c, int nitems, const rl_item *item
     // on these items with the current inputs
     const bool use_tape = c->tape_gen == c->gen && same_items(c->tape_items, nitems, items);
     c->last_used_tape = use_tape ? 1 : 0;
+    c->last_pair_blocks = 0;
+    // By pairs where the gradients go on to the physical fields alone
+    // (rl_physics_adjoint), which are the same to rounding.  Those on the tables
+    // themselves are by segments: in nearly empty cells dL/d rho and dL/d alpha are
+    // differences that cancel to 1e-6 (FP64) and, in FP32, to nothing, so that any
+    // other order of summation is seen there.
+    const bool tables = g_rho || g_abund || g_lw || g_pops || g_jd || g_ad;
+    const bool pairs = c->phys_tables && !tables;
     size_t fo = 0;
     if (use_tape) {
         c->last_kblk = c->tape_kblk;
@@ -2391,7 +2403,16 @@ extern "C" int rl_trace_lines_adjoint(rl_ctx *c, int nitems, const rl_item *item
             if (int e = adj_setup(c, it, ii, su, 0)) return e;
             if (int e = upload(c, c->d_gflux, dL_dflux + fo, (size_t)it.nfr * 8)) return e;
             const AdjChunk whole{0, su.rs->nrays, 0, su.rs->nnodes};
-            if (int e = adj_reverse_chunk(c, it, su, c->tape_kblk, whole, c->tape[ii])) return e;
+            AdjItemBufs &ab = c->tape[ii];
+            if (tables && ab.nblk) {          // taken by blocks: retaken by segments, and kept so
+                if (int e = adj_forward_chunk(c, it, su, c->tape_kblk, whole, ab, false)) {
+                    c->tape_items.clear();
+                    return e;
+                }
+                c->last_used_tape = 0;
+            }
+            c->last_pair_blocks += ab.nblk;
+            if (int e = adj_reverse_chunk(c, it, su, c->tape_kblk, whole, ab)) return e;
             fo += it.nfr;
         }
     } else {
@@ -2424,8 +2445,9 @@ extern "C" int rl_trace_lines_adjoint(rl_ctx *c, int nitems, const rl_item *item
             if (!err) err = adj_setup(c, it, ii, su, p.work);
             if (!err) err = upload(c, c->d_gflux, dL_dflux + fo, (size_t)it.nfr * 8);
             for (size_t k = 0; k < p.chunks.size() && !err; k++) {
-                err = adj_forward_chunk(c, it, su, p.K, p.chunks[k], ab);
+                err = adj_forward_chunk(c, it, su, p.K, p.chunks[k], ab, pairs);
                 if (!err) err = adj_reverse_chunk(c, it, su, p.K, p.chunks[k], ab);
+                c->last_pair_blocks += ab.nblk;
             }
             if (!err) err = adj_flux(c, it, su, flux ? flux + fo : nullptr);
             c->last_kblk = std::max(c->last_kblk, p.K);
@@ -2469,6 +2491,12 @@ extern "C" int rl_last_adjoint_info(const rl_ctx *c, int *ckpt_interval, int *us
     if (ckpt_interval) *ckpt_interval = c->last_kblk;
     if (used_tape) *used_tape = c->last_used_tape;
     if (chunks) *chunks = c->last_chunks;
+    return 0;
+}
+
+extern "C" int rl_last_adjoint_pairs(const rl_ctx *c, long long *blocks) {
+    if (!c) return RL_E_ARG;
+    if (blocks) *blocks = c->last_pair_blocks;
     return 0;
 }
 
@@ -2696,6 +2724,7 @@ extern "C" int rl_set_physics(rl_ctx *c, const double *T_gas, const double *T_du
                               const double *log_abund, const double *vturb_kms, double m_mol,
                               double q_over) {
     if (c) c->gen++;                         // invalidates a tape
+    if (c) c->phys_tables = false;           // until they are formed
     if (!c || !T_gas || (!vturb_kms && !c->pre_alpha_on) || !(m_mol > 0.0))
         return fail(c, RL_E_ARG, "rl_set_physics: bad args");
     if (!c->have_medium || !c->nlines || !c->pre_nlev || !c->d_nu0.n)
@@ -2764,7 +2793,7 @@ extern "C" int rl_set_physics(rl_ctx *c, const double *T_gas, const double *T_du
     c->aksmax = mx;                          // line.F:3020-3033 (widths > 0 here)
     c->have_dust = true;
     c->pre_ready = 1;
-    c->pre_gen = c->gen;
+    c->phys_tables = true;
     c->cells_line = -1;
     return 0;
 }

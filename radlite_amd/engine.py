@@ -86,6 +86,7 @@ def load_library(path=LIB_PATH):
         "rl_trace_lines_forward_tape": (C.c_int, [vp, C.c_int, C.POINTER(RLItem), _dp]),
         "rl_tape_release": (C.c_int, [vp]),
         "rl_last_adjoint_info": (C.c_int, [vp, _ip, _ip, _ip]),
+        "rl_last_adjoint_pairs": (C.c_int, [vp, C.POINTER(C.c_longlong)]),
         "rl_memory_info": (C.c_int, [vp, _dp]),
         "rl_plan": (C.c_int, [vp, C.c_int, C.POINTER(RLItem), _dp]),
         "rl_set_level_data": (C.c_int, [vp, C.c_int, _dp, _dp]),
@@ -448,6 +449,13 @@ class Raytracer:
         self._chk(self.L.rl_last_adjoint_info(self.ctx, *[C.byref(x) for x in v]),
                   "rl_last_adjoint_info")
         return tuple(x.value for x in v)
+
+    def adjoint_pairs(self):
+        """Blocks of segments that the last adjoint reversed by (block,
+        channel) pairs; 0: by segments."""
+        v = C.c_longlong(0)
+        self._chk(self.L.rl_last_adjoint_pairs(self.ctx, C.byref(v)), "rl_last_adjoint_pairs")
+        return v.value
 
     def adjoint(self, items, dL_dflux, outputs=None):
         """Gradient of L with respect to the inputs the trace reads, given
