@@ -1285,16 +1285,23 @@ static size_t cut_batches(rl_ctx *c, int nitems, const rl_item *items,
     return most;
 }
 
-// The formal solution's launch over a batch's items: channels per chunk, first
-// units u0 [nb + 1], and the blocks of the persistent grid (0: a block per unit).
+// The formal solution's launches over a batch's items: channels per chunk, first
+// units u0 (twice [nb + 1]: those of the items of many channels, then of the items
+// of few; an item has none in the other list), and the blocks of the persistent
+// grid (0: a block per unit).
 struct FormalPlan { int cw, nblk; };
 static int formal_plan(rl_ctx *c, int fp64, const std::vector<rl::ItemDev> &hi, FormalPlan &p,
                        std::vector<long long> &u0) {
     p.cw = rl::formal_chunk();
     if (c->fixed_cw > 0) p.cw = std::min(p.cw, c->fixed_cw);
-    u0.assign(hi.size() + 1, 0);
-    for (size_t k = 0; k < hi.size(); k++)
-        u0[k + 1] = u0[k] + units_of(p.cw, hi[k].nrays, hi[k].nfr);
+    const size_t nb = hi.size();
+    u0.assign(2 * (nb + 1), 0);
+    for (int few = 0; few < 2; few++) {
+        long long *u = u0.data() + few * (nb + 1);
+        for (size_t k = 0; k < nb; k++)
+            u[k + 1] = u[k] + (rl::formal_few(hi[k].nfr) == (few != 0)
+                                   ? units_of(p.cw, hi[k].nrays, hi[k].nfr) : 0);
+    }
     p.nblk = 0;
     if (c->fixed_cw < 0 || !c->fixed_persistent) return 0;
     int cu = 0;
@@ -1364,7 +1371,7 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
     HIPCHK(c, c->d_maser.ensure((size_t)((nb + 1) / 2) * 8));
     HIPCHK(c, c->d_counter.ensure(8));
     HIPCHK(c, c->d_items.ensure((size_t)nb * sizeof(rl::ItemDev)));
-    HIPCHK(c, c->d_unit0.ensure((size_t)(nb + 1) * 8));
+    HIPCHK(c, c->d_unit0.ensure((size_t)(nb + 1) * 16));
     if (cmask) HIPCHK(c, c->d_cmask.ensure((size_t)img0));
     if (int e = upload(c, c->d_chan, chan.data(), nchan * 8)) return e;
     c->cells_line = -1;       // d_cells is rewritten below for this batch's lines
@@ -1399,8 +1406,9 @@ static int run_batch(rl_ctx *c, const rl_item *items, int i0, int i1, double *fl
     FormalPlan fp;
     std::vector<long long> &u0 = c->h_unit0;
     if (int e = formal_plan(c, fp64, hi, fp, u0)) return e;
-    L.nunits = u0[nb];
-    if (int e = upload(c, c->d_unit0, u0.data(), (size_t)(nb + 1) * 8)) return e;
+    L.nunits[0] = u0[nb];
+    L.nunits[1] = u0[2 * nb + 1];
+    if (int e = upload(c, c->d_unit0, u0.data(), (size_t)(nb + 1) * 16)) return e;
     auto zero_counters = [&]() {
         rl::launch_zero_u64(c->stream, L.ovs, nb);
         rl::launch_zero_u64(c->stream, reinterpret_cast<unsigned long long *>(L.maser),
@@ -1715,7 +1723,7 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
     const size_t o_maser = carve((size_t)((nb + 1) / 2) * 8);
     const size_t o_counter = carve(8);
     const size_t o_items = carve((size_t)nb * sizeof(rl::ItemDev));
-    const size_t o_unit0 = carve((size_t)(nb + 1) * 8);
+    const size_t o_unit0 = carve((size_t)(nb + 1) * 16);
     // the block records where they still fit; without them every segment is
     // integrated
     const size_t bbytes = (size_t)blk0 * sizeof(rl::BlkRec);
@@ -1746,7 +1754,8 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
     L.cmask = nullptr;
     L.d2 = (1.0 * 3.08572e18) * (1.0 * 3.08572e18);
     L.unit0 = reinterpret_cast<const long long *>(ws + o_unit0);
-    L.nunits = u0[nb];
+    L.nunits[0] = u0[nb];
+    L.nunits[1] = u0[2 * nb + 1];
     L.ovs = reinterpret_cast<unsigned long long *>(ws + o_ovs);
     L.maser = reinterpret_cast<int *>(ws + o_maser);
     L.counter = reinterpret_cast<unsigned long long *>(ws + o_counter);
@@ -1756,7 +1765,7 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
                              c->stream));
     HIPCHK(c, hipMemcpyAsync(ws + o_items, hi.data(), (size_t)nb * sizeof(rl::ItemDev),
                              hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(ws + o_unit0, u0.data(), (size_t)(nb + 1) * 8,
+    HIPCHK(c, hipMemcpyAsync(ws + o_unit0, u0.data(), (size_t)(nb + 1) * 16,
                              hipMemcpyHostToDevice, c->stream));
     rl::launch_zero_u64(c->stream, L.ovs, nb);
     rl::launch_zero_u64(c->stream, reinterpret_cast<unsigned long long *>(L.maser), (nb + 1) / 2);

@@ -79,8 +79,10 @@ struct BatchLaunch {
     double *image, *partial, *flux;
     unsigned char *cmask;      // optional [image layout]: 1 where integrated
     double d2;
-    const long long *unit0;    // device [nitems+1] first unit (ray, channel chunk) of each item
-    long long nunits;
+    // device, twice [nitems+1]: first unit (ray, channel chunk) of each item of
+    // many channels, and of few (formal_few); an item has none in the other list
+    const long long *unit0;
+    long long nunits[2];
     unsigned long long *ovs, *counter;
     int *maser;
 };
@@ -102,6 +104,7 @@ hipError_t scratch_attach(int device, void **out);
 // the work counter
 void launch_batch_formal(hipStream_t st, int fp64, const BatchLaunch &b, int cw, int nblocks);
 int formal_chunk();
+bool formal_few(int nfr);      // whether nfr channels are few for k_formal
 void launch_batch_finish(hipStream_t st, int fp64, const BatchLaunch &b);
 void launch_batch_flux(hipStream_t st, const BatchLaunch &b);
 void launch_zero_u64(hipStream_t st, unsigned long long *p, int n);

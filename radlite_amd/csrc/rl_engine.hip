@@ -1228,9 +1228,8 @@ __device__ inline int unit_item(const FormalBatch &f, long long u) {
     return lo;
 }
 
-template <typename T>
-__device__ __forceinline__ void formal_unit(const FormalBatch &f, WalkLds<T> &lds, long long u) {
-    constexpr int G = GROUPS;
+template <typename T, int G>
+__device__ __forceinline__ void formal_unit(const FormalBatch &f, WalkLds<T, G> &lds, long long u) {
     const int lane = threadIdx.x;
     const int item = unit_item(f, u);
     const ItemDev &it = f.items[item];
@@ -1266,7 +1265,17 @@ __device__ __forceinline__ void formal_unit(const FormalBatch &f, WalkLds<T> &ld
         const float4 *rec =
             reinterpret_cast<const float4 *>(reinterpret_cast<const NodeRec<double> *>(f.rec) +
                                              it.rec0 + b);
-        walk<double>(
+        auto exact = [&](const NodeRec<double> *sr, int j, int c, double2 v)
+                         __attribute__((always_inline)) {
+            if (!doit(c)) return Map{1.0, 0.0};
+            LineK<double> L;
+            L.nu0 = it.lc.nu0; L.c_aa = it.lc.c_aa; L.hknu = it.lc.hknu;
+            L.A = it.lc.A; L.Bud = it.lc.Bud; L.Bdu = it.lc.Bdu;
+            L.dnu = v.y;
+            L.uch = v.x;
+            return block_exact(sr, j, n, L, istar + c, sf, ovs, maser);
+        };
+        walk<double, G>(
             lds, blk, nb, ch, I, over,
             [&](int j, int piece) __attribute__((always_inline)) {
                 const int k = min(max((j << BLK_LOG) - 2 + (piece >> 2), 0), n - 1);
@@ -1274,13 +1283,11 @@ __device__ __forceinline__ void formal_unit(const FormalBatch &f, WalkLds<T> &ld
             },
             [&](int c) __attribute__((always_inline)) { return double2{velo[c], dnu[c]}; },
             [&](const float4 *st, int j, int c, double2 v) __attribute__((always_inline)) {
-                if (!doit(c)) return Map{1.0, 0.0};
-                LineK<double> L;
-                L.nu0 = it.lc.nu0; L.c_aa = it.lc.c_aa; L.hknu = it.lc.hknu;
-                L.A = it.lc.A; L.Bud = it.lc.Bud; L.Bdu = it.lc.Bdu;
-                L.dnu = v.y;
-                L.uch = v.x;
-                return block_exact(st, j, n, L, istar + c, sf, ovs, maser);
+                return exact(reinterpret_cast<const NodeRec<double> *>(st), j, c, v);
+            },
+            [&](int j, int c, double2 v) __attribute__((always_inline)) {
+                return exact(reinterpret_cast<const NodeRec<double> *>(rec) +
+                                 ((j << BLK_LOG) - 2), j, c, v);
             },
             [&](int g, int nov) __attribute__((always_inline)) {
                 const int c = ch.c0 + 64 * g + lane;
@@ -1291,7 +1298,7 @@ __device__ __forceinline__ void formal_unit(const FormalBatch &f, WalkLds<T> &ld
         const float4 *hot = reinterpret_cast<const float4 *>(base + it.hot_off) + b;
         const float4 *aux = reinterpret_cast<const float4 *>(base + it.aux_off) + b;
         const float4 *line = reinterpret_cast<const float4 *>(f.rec) + it.rec0 + b;
-        walk<float>(
+        walk<float, G>(
             lds, blk, nb, ch, I, over,
             [&](int j, int piece) __attribute__((always_inline)) {
                 constexpr int N = Nodes<float>::N;
@@ -1303,6 +1310,14 @@ __device__ __forceinline__ void formal_unit(const FormalBatch &f, WalkLds<T> &ld
             [&](const float4 *st, int j, int c, float v) __attribute__((always_inline)) {
                 if (!doit(c)) return Map{1.0, 0.0};
                 return block_split(st, j, n, v, istar + c, sf, maser);
+            },
+            [&](int j, int c, float v) __attribute__((always_inline)) {
+                if (!doit(c)) return Map{1.0, 0.0};
+                const int k = (j << BLK_LOG) - 1;
+                return block_split(reinterpret_cast<const SegHot *>(hot) + k,
+                                   reinterpret_cast<const SegAux *>(aux) + k,
+                                   reinterpret_cast<const NodeLine *>(line) + k, j, n, v,
+                                   istar + c, sf, maser);
             },
             [&](int g, int) __attribute__((always_inline)) { over |= 1u << g; });
     }
@@ -1327,10 +1342,12 @@ __device__ __forceinline__ void formal_unit(const FormalBatch &f, WalkLds<T> &ld
     }
 }
 
-template <typename T>
+// G: the groups of 64 channels of a chunk at most; 1 for items of few channels
+// (formal_few), whose walk takes sparse windows from memory
+template <typename T, int G>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? FORMAL32_WAVES : FORMAL64_WAVES)))
 k_formal(FormalBatch f) {
-    __shared__ WalkLds<T> lds;
+    __shared__ WalkLds<T, G> lds;
     // a unit per block, or (persistent) units from a device counter until all
     // are taken, so the grid drains by itself
     unsigned long long u = blockIdx.x;
@@ -1345,7 +1362,7 @@ k_formal(FormalBatch f) {
             u = (unsigned long long)hi << 32 | lo;
         }
         if (u >= (unsigned long long)f.nunits) break;
-        formal_unit<T>(f, lds, (long long)u);
+        formal_unit<T, G>(f, lds, (long long)u);
         if (!f.counter) break;
     }
 }
@@ -1426,15 +1443,31 @@ void launch_batch_nodes(hipStream_t st, int fp64, const BatchLaunch &b) {
                            b.rec, b.blk, b.rinfo, b.chan);
 }
 
-void launch_batch_formal(hipStream_t st, int fp64, const BatchLaunch &b, int cw, int nblocks) {
+// Up to a group of 64 channels the walk may take windows of few pairs a block from
+// memory (rl_walk.h).  The other items keep a kernel without that path, whose
+// registers it would spill: 200 x 100 disk, 100 channels, FP64, 4.62 -> 4.71 ms a call
+// with it, 400 x 200, 200 channels, FP32, 30.4 -> 30.6.
+bool formal_few(int nfr) { return nfr <= 64; }         // one group
+
+template <bool FEW>
+static void launch_formal(hipStream_t st, int fp64, const BatchLaunch &b, int cw, int nblocks) {
+    const long long n = b.nunits[FEW];
+    if (n == 0) return;
     // a launch holds fewer than 2^32 threads
-    if (nblocks == 0 && b.nunits * 64 >= 1ll << 31) nblocks = 1 << 16;
-    const FormalBatch f{b.items, b.unit0, b.nitems, cw, b.nunits, b.rec, b.blk, b.rinfo, b.chan,
-                        b.image, b.ovs, b.maser, b.cmask, nblocks > 0 ? b.counter : nullptr};
-    const unsigned grid = (unsigned)(nblocks > 0 ? nblocks : b.nunits);
+    if (nblocks == 0 && n * 64 >= 1ll << 31) nblocks = 1 << 16;
+    const FormalBatch f{b.items, b.unit0 + FEW * (b.nitems + 1), b.nitems, cw, n, b.rec, b.blk,
+                        b.rinfo, b.chan, b.image, b.ovs, b.maser, b.cmask,
+                        nblocks > 0 ? b.counter : nullptr};
+    const unsigned grid = (unsigned)(nblocks > 0 ? nblocks : n);
     if (nblocks > 0) hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, b.counter, 1);
-    if (fp64) hipLaunchKernelGGL(k_formal<double>, dim3(grid), dim3(64), 0, st, f);
-    else hipLaunchKernelGGL(k_formal<float>, dim3(grid), dim3(64), 0, st, f);
+    constexpr int G = FEW ? 1 : GROUPS;
+    if (fp64) hipLaunchKernelGGL((k_formal<double, G>), dim3(grid), dim3(64), 0, st, f);
+    else hipLaunchKernelGGL((k_formal<float, G>), dim3(grid), dim3(64), 0, st, f);
+}
+
+void launch_batch_formal(hipStream_t st, int fp64, const BatchLaunch &b, int cw, int nblocks) {
+    launch_formal<false>(st, fp64, b, cw, nblocks);
+    launch_formal<true>(st, fp64, b, cw, nblocks);
 }
 
 void launch_batch_finish(hipStream_t st, int fp64, const BatchLaunch &b) {
@@ -1495,9 +1528,9 @@ int formal_chunk() { return 64 * GROUPS; }
 int formal_blocks_per_cu(int fp64) {
     int nb = 0;
     if (fp64)
-        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_formal<double>, 64, 0);
+        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_formal<double, GROUPS>, 64, 0);
     else
-        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_formal<float>, 64, 0);
+        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_formal<float, GROUPS>, 64, 0);
     return nb > 0 ? nb : 1;
 }
 

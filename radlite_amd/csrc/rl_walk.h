@@ -11,6 +11,14 @@
 //   compose    a lane per channel: the maps of the blocks now complete, in
 //              order, the pair's where there is one, else the block's own
 //
+// A batch costs about the same full or not: at each of its 8 segments it waits for
+// the longest of its lanes' sub-grid loops.  With few channels the blocks that LDS
+// holds make up a small part of one, so that where a window of 64 blocks has that
+// few pairs they are taken 64 at a time from any number of blocks, each lane from
+// its block's nodes in memory.  Formal solution, one inclination, +-30 km/s: 400 x
+// 200 disk, 64 angles, 9 channels, FP32, 1.17 -> 0.65 ms, 40 channels 1.20 -> 0.88; FP64
+// 2.36 -> 1.16 and 2.47 -> 2.03; 100 x 60 disk, 50 channels, FP64, 0.87 -> 0.83 a call.
+//
 // What bounds it: instruction issue, then the latency of a batch's steps.
 // Lanes that held one (ray, channel) each and met at every block that one of 16
 // channels saw had work in 38% of their instructions, and a ray of many blocks
@@ -56,9 +64,9 @@ struct Map {
     double P, B;
 };
 
-// one wave's share of LDS
-constexpr int RING = 64 * GROUPS + 64;                 // a chunk's pairs of one block + 64
-template <typename T> struct WalkLds {
+// one wave's share of LDS, for chunks of up to 64 G channels
+template <typename T, int G> struct WalkLds {
+    static constexpr int RING = 64 * G + 64;           // a chunk's pairs of one block + 64
     Map map[RING];                                     // pair p at p % RING
     float4 st[SLOTS][Nodes<T>::PIECES];
 };
@@ -111,16 +119,19 @@ struct Chans {
 // The nb blocks of a ray: I[g] the intensity of channel c0 + 64 g + lane; over:
 // FP32, bit g set on an overshoot.  stage(j, piece): a piece of block j's
 // nodes; before(c): what channel c needs, loaded while the nodes arrive;
-// integrate(nodes, j, c, that): the map of block j for channel c; passed(g,
-// n): n overshoots of a block's own map.
-template <typename T, typename Stage, typename Before, typename Integrate,
+// integrate(nodes, j, c, that): the map of block j for channel c; direct(j, c,
+// that): the same from the nodes in memory (G = 1); passed(g, n): n overshoots of a
+// block's own map.
+template <typename T, int G, typename Stage, typename Before, typename Integrate, typename Direct,
           typename Free>
-__device__ __forceinline__ void walk(WalkLds<T> &S, const BlkRec *__restrict__ blk, int nb,
-                                     const Chans &ch, double (&I)[GROUPS], unsigned &over,
+__device__ __forceinline__ void walk(WalkLds<T, G> &S, const BlkRec *__restrict__ blk, int nb,
+                                     const Chans &ch, double (&I)[G], unsigned &over,
                                      const Stage &stage, const Before &before,
-                                     const Integrate &integrate, const Free &passed) {
+                                     const Integrate &integrate, const Direct &direct,
+                                     const Free &passed) {
     using Pre = decltype(before(0));
-    constexpr int G = GROUPS;
+    constexpr int RING = WalkLds<T, G>::RING;
+    constexpr bool FEW = G == 1;
     const int lane = threadIdx.x & 63;
     const T v0 = (T)ch.velo[ch.c0], v1 = (T)ch.velo[ch.c1 - 1];
     const T inv = ch.c1 - ch.c0 > 1 ? (T)(ch.c1 - 1 - ch.c0) / (v1 - v0) : T(0);
@@ -148,8 +159,11 @@ __device__ __forceinline__ void walk(WalkLds<T> &S, const BlkRec *__restrict__ b
         const int st = incl - cnt, total = lane_of(incl, m - 1);
         const bool some = cnt > 0, overs = __any(nov != 0);
         // the blocks with pairs that are not in LDS yet, and of these the first
-        // `ahead` whose nodes are in registers (slots by rank)
+        // `ahead` whose nodes are in registers (slots by rank); none where the
+        // pairs of BATCH_BLOCKS blocks do not fill a batch
         unsigned long long rest = __ballot(some);
+        const bool sparse = FEW && total * BATCH_BLOCKS < 64 * __popcll(rest);
+        if (sparse) rest = 0;
         const int rank = __popcll(rest & (upto >> 1));
         int staged = 0, ahead = 0;
         float4 piece[2];
@@ -175,7 +189,24 @@ __device__ __forceinline__ void walk(WalkLds<T> &S, const BlkRec *__restrict__ b
         load();
         for (int p0 = 0, b = 0; b < m;) {
             int pend = total;
-            if (p0 < total) {
+            if (sparse && p0 < total) {
+                pend = min(p0 + 64, total);
+                const int p = min(p0 + lane, pend - 1);
+                int j = 0;                       // the last block that begins at or before p
+                for (int d = RECS / 2; d >= 1; d >>= 1) {
+                    const int t = __shfl(st, min(j + d, 63));
+                    if (j + d < m && t <= p) j += d;
+                }
+                const int c = __shfl(cl, j) + p - __shfl(st, j);
+                const Pre pre = before(c);
+                wave_lds_fence();
+                if (p0 + lane < pend) {
+                    const Map q = direct(jw + j, c, pre);
+                    int i = p0 % RING + lane;
+                    S.map[i >= RING ? i - RING : i] = q;
+                }
+                wave_lds_fence();
+            } else if (p0 < total) {
                 // the pairs p0 .. pend-1 of at most BATCH_BLOCKS blocks: the one
                 // that holds p0 (lane l0) and those that begin after it
                 const int l0 = 63 - __clzll(__ballot(some && st <= p0));
@@ -226,7 +257,7 @@ __device__ __forceinline__ void walk(WalkLds<T> &S, const BlkRec *__restrict__ b
                 const int nv = overs ? lane_of(nov, b) : 0;
 #pragma unroll
                 for (int g = 0; g < G; g++) {
-                    if (g >= ch.ng) break;
+                    if (G > 1 && g >= ch.ng) break;
                     double mP = A0, mB = B0;
                     if (c < 64 * g + 64 && c + n > 64 * g) {     // the group has pairs
                         const int i = 64 * g + lane - c;
@@ -253,14 +284,11 @@ __device__ __forceinline__ void walk(WalkLds<T> &S, const BlkRec *__restrict__ b
     }
 }
 
-// FP32: block j of a ray of n nodes for one channel, on split records
-// (rl_fwd32.h) staged as Nodes<float> holds them
-__device__ __forceinline__ Map block_split(const float4 *st, int j, int n, float uch,
-                                           const double *istar, float sf, int &maser) {
-    constexpr int N = Nodes<float>::N;
-    const SegHot *sh = reinterpret_cast<const SegHot *>(st);
-    const SegAux *sa = reinterpret_cast<const SegAux *>(st + N);
-    const NodeLine *sl = reinterpret_cast<const NodeLine *>(st + 2 * N);
+// FP32: block j of a ray of n nodes for one channel on split records (rl_fwd32.h);
+// sh, sa, sl: those of node 8 j - 1
+__device__ __forceinline__ Map block_split(const SegHot *sh, const SegAux *sa, const NodeLine *sl,
+                                           int j, int n, float uch, const double *istar, float sf,
+                                           int &maser) {
     Acc32<true> x{0.0, 1.0};
     Car32 c;
     bool ovf = false;
@@ -274,10 +302,20 @@ __device__ __forceinline__ Map block_split(const float4 *st, int j, int n, float
     return Map{mark(x.P, ovf), x.I};
 }
 
-// FP64: the same on whole node records, with the reference's own arithmetic
-__device__ __forceinline__ Map block_exact(const float4 *st, int j, int n, const LineK<double> &L,
-                                           const double *istar, double sf, int &ovs, int &maser) {
-    const NodeRec<double> *sr = reinterpret_cast<const NodeRec<double> *>(st);
+// staged as Nodes<float> holds them
+__device__ __forceinline__ Map block_split(const float4 *st, int j, int n, float uch,
+                                           const double *istar, float sf, int &maser) {
+    constexpr int N = Nodes<float>::N;
+    return block_split(reinterpret_cast<const SegHot *>(st),
+                       reinterpret_cast<const SegAux *>(st + N),
+                       reinterpret_cast<const NodeLine *>(st + 2 * N), j, n, uch, istar, sf, maser);
+}
+
+// FP64: the same on whole node records, with the reference's own arithmetic; sr:
+// that of node 8 j - 2
+__device__ __forceinline__ Map block_exact(const NodeRec<double> *sr, int j, int n,
+                                           const LineK<double> &L, const double *istar, double sf,
+                                           int &ovs, int &maser) {
     Acc<double, true> x{0.0, 1.0};
     Carry<double> c;
     c.init = 1; c.phi0 = 0.0; c.srcl0 = 0.0; c.alpl0 = 0.0; c.S0 = 0.0;
