@@ -1080,13 +1080,20 @@ template void launch_posvel<float>(hipStream_t, const PosvelLaunch &);
 // ---------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------
-// One wave per ray up to this many rays of a launch.  A thread per ray takes as
-// long for 2,000 rays as for 60,000 (one chain), a wave per ray's time grows with
-// them: 60 x 40 cube, 1,920 rays, build of the trajectories 0.35 -> 0.09 ms; 100
-// x 60 disk, 7,041 rays, 0.60 -> 0.22 ms; 200 x 100, 34,049, 1.14 -> 0.81; 256 x
-// 128 x 4 inclinations, 68,100, 2.37 -> 2.23; 400 x 200 x 2, 267,266 (with 25 KB
-// of LDS a wave), 9.5 -> 13.9, so not there.
-constexpr long long CROSS_WAVE_RAYS = 80000;
+// One wave per ray up to this many rays of a launch, and bytes of LDS for them
+// together.  A thread per ray takes as long for 2,000 rays as for 40,000 (one chain);
+// a wave per ray's time grows with them, and with the LDS of a wave, of which fewer
+// then run at once (25 KB on a 400 x 200 grid: six to a compute unit).  Trajectories,
+// thread -> wave, ms, one inclination of 20 degrees / four from 20 to 65 (whose chains
+// are longer):
+//   100 x 60 grid, 8 KB a wave: 10,000 rays 0.76 -> 0.40, 60,000 1.05 -> 0.90 / 1.77 ->
+//     1.56, 80,000 1.16 -> 1.13 / 1.90 -> 1.65, 120,000 1.49 -> 1.68 / 2.21 -> 2.12
+//   200 x 100, 13 KB: 10,000 1.04 -> 0.58, 60,000 1.66 -> 1.56 / 2.44 -> 2.23, 80,000
+//     1.92 -> 2.10 / 2.72 -> 2.41, 120,000 2.51 -> 2.91 / 3.27 -> 3.24
+//   256 x 128, 17 KB: 60,000 1.96 -> 1.86 / 2.86 -> 2.50, 80,000 2.32 -> 2.67 / 3.17 -> 2.98
+//   400 x 200, 25 KB: 20,000 1.99 -> 1.29, 40,000 2.57 -> 2.53 / 3.04 -> 2.80, 60,000
+//     3.04 -> 3.62 / 3.79 -> 3.77, 80,000 3.50 -> 4.31 / 4.25 -> 4.73
+constexpr long long CROSS_WAVE_RAYS = 80000, CROSS_WAVE_BYTES = 1200000000;
 constexpr size_t CROSS_WAVE_LDS = 48 * 1024;
 void launch_cross(hipStream_t st, const GridDev &gd, const double *tan2, const CrossSets &sets,
                   int nmax, int *err) {
@@ -1099,7 +1106,8 @@ void launch_cross(hipStream_t st, const GridDev &gd, const double *tan2, const C
     long long rays = 0;
     for (int i = 0; i < sets.n; i++) rays += sets.s[i].nrays;
     const size_t wl = cross_wave_lds(nmax);
-    const int wave = rays <= CROSS_WAVE_RAYS && wl <= CROSS_WAVE_LDS;
+    const int wave = rays <= CROSS_WAVE_RAYS && rays * (long long)wl <= CROSS_WAVE_BYTES &&
+                     wl <= CROSS_WAVE_LDS;
     if (wave)
         hipLaunchKernelGGL(k_cross_wave, dim3(most, sets.n), dim3(64), wl, st, g, tan2, sets, nmax,
                            err);
