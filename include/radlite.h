@@ -178,7 +178,9 @@ int rl_trace_lines_posvel(rl_ctx *ctx, int nitems, const rl_item *items,
  * vtx[npix][nv] (-1: none) and weights w[npix][nv] (the barycentric
  * weights of the pixel in its triangle, times any per-vertex factor); out
  * receives [nfr][npix].  The reference has no such library routine: this
- * replaces the IDL post-processing of the lineposvelcirc file. */
+ * replaces the IDL post-processing of the lineposvelcirc file.  Its device
+ * buffers are kept for the next call where they take up to 1 GiB together,
+ * until a trace finds them above a tenth of its budget. */
 int rl_resample_image(rl_ctx *ctx, int nrays, int nfr, const double *image, int npix,
                       int nv, const int *vtx, const double *w, double *out);
 

@@ -137,7 +137,14 @@ struct rl_ctx {
     hipStream_t stream = nullptr;
     std::string err;
     Staging stage;
-    DevBuf d_rs_img, d_rs_vtx, d_rs_w, d_rs_out;     // rl_resample_image
+    // rl_resample_image's image, vertices, weights and output: kept up to KEEP bytes
+    // together, and given back when a trace finds them above a tenth of its budget
+    struct Resample {
+        static constexpr size_t KEEP = (size_t)1 << 30;
+        DevBuf img, vtx, w, out;
+        size_t held() const { return img.n + vtx.n + w.n + out.n; }
+        void release() { img = DevBuf(); vtx = DevBuf(); w = DevBuf(); out = DevBuf(); }
+    } rs_buf;
     // grid
     int nr = 0, nh = 0;
     std::vector<double> rc, tc;
@@ -836,16 +843,23 @@ static size_t ctx_budget(rl_ctx *c) {
         size_t fr = 0, tot = 0;
         if (hipMemGetInfo(&fr, &tot) != hipSuccess) fr = 0;
         c->auto_budget = (size_t)(0.6 * (double)fr) + resident_traj(c) + c->d_rec.n +
-                         c->d_image.n + c->d_partial.n + c->d_ckpt.n + c->d_arec.n;
+                         c->d_blk.n + c->d_image.n + c->d_partial.n + c->d_ckpt.n + c->d_arec.n +
+                         c->rs_buf.held();
     }
     return c->auto_budget;
 }
 
 // The forward's batch buffers and the adjoint's chunk buffers are kept
 // between calls for reuse; one kind is released when the other kind of
-// call starts and it holds more than a tenth of the budget.
+// call starts and it holds more than a tenth of the budget.  So are the resampling's
+// when either starts.
+static void release_resample(rl_ctx *c) {
+    if (c->rs_buf.held() * 10 > ctx_budget(c)) c->rs_buf.release();
+}
+
 static void release_forward_work(rl_ctx *c) {
-    if ((c->d_rec.n + c->d_cmask.n) * 10 > ctx_budget(c)) {
+    release_resample(c);
+    if ((c->d_rec.n + c->d_blk.n + c->d_cmask.n) * 10 > ctx_budget(c)) {
         (void)hipStreamSynchronize(c->stream);
         c->d_rec = DevBuf();
         c->d_blk = DevBuf();
@@ -854,6 +868,7 @@ static void release_forward_work(rl_ctx *c) {
 }
 
 static void release_adjoint_work(rl_ctx *c) {
+    release_resample(c);
     if ((c->d_arec.n + c->d_ckpt.n + c->d_gnode.n + c->d_gcell.n) * 10 > ctx_budget(c)) {
         (void)hipStreamSynchronize(c->stream);
         c->d_arec = DevBuf();
@@ -1819,6 +1834,25 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
 // PRO/imcir_conv.pro:161-181): out[ch][p] = sum_k w[p][k] image[vtx[p][k]][ch],
 // the triangulation weights formed by the caller.  Every vertex index is
 // checked against nrays before the launch.
+static int resample(rl_ctx *c, int nrays, int nfr, const double *image, int npix, int nv,
+                    const int *vtx, const double *w, double *out) {
+    const size_t nvt = (size_t)npix * nv;
+    rl_ctx::Resample &d = c->rs_buf;
+    HIPCHK(c, d.img.ensure((size_t)nrays * nfr * 8));
+    HIPCHK(c, copy_up(c, d.img.p, image, (size_t)nrays * nfr * 8));
+    if (int e = upload(c, d.vtx, vtx, nvt * 4)) return e;
+    if (int e = upload(c, d.w, w, nvt * 8)) return e;
+    HIPCHK(c, d.out.ensure((size_t)npix * nfr * 8));
+    HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
+    rl::launch_rect_gather(c->stream, npix, nfr, nv, d.vtx.as<int>(), d.w.as<double>(),
+                           d.img.as<double>(), d.out.as<double>());
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipEventRecord(c->ev[4], c->stream));
+    HIPCHK(c, copy_down(c, out, d.out.p, (size_t)npix * nfr * 8));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return 0;
+}
+
 extern "C" int rl_resample_image(rl_ctx *c, int nrays, int nfr, const double *image, int npix,
                                  int nv, const int *vtx, const double *w, double *out) {
     if (!c || nrays < 1 || nfr < 1 || npix < 0 || nv < 1 || !image || (npix && (!vtx || !w || !out)))
@@ -1829,26 +1863,12 @@ extern "C" int rl_resample_image(rl_ctx *c, int nrays, int nfr, const double *im
             return fail(c, RL_E_ARG, "rl_resample_image: vertex %d out of range", vtx[i]);
     if (npix == 0) return 0;
     HIPCHK(c, hipSetDevice(c->device));
-    DevBuf &d_img = c->d_rs_img, &d_vtx = c->d_rs_vtx, &d_w = c->d_rs_w, &d_out = c->d_rs_out;
-    HIPCHK(c, d_img.ensure((size_t)nrays * nfr * 8));
-    HIPCHK(c, copy_up(c, d_img.p, image, (size_t)nrays * nfr * 8));
-    if (int e = upload(c, d_vtx, vtx, nvt * 4)) return e;
-    if (int e = upload(c, d_w, w, nvt * 8)) return e;
-    HIPCHK(c, d_out.ensure((size_t)npix * nfr * 8));
-    HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
-    rl::launch_rect_gather(c->stream, npix, nfr, nv, d_vtx.as<int>(), d_w.as<double>(),
-                           d_img.as<double>(), d_out.as<double>());
-    HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipEventRecord(c->ev[4], c->stream));
-    HIPCHK(c, copy_down(c, out, d_out.p, (size_t)npix * nfr * 8));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    // kept for the next call unless they take much of the memory
-    if ((d_img.n + d_out.n + d_vtx.n + d_w.n) * 10 > ctx_budget(c)) {
-        d_img = DevBuf();
-        d_out = DevBuf();
-        d_vtx = DevBuf();
-        d_w = DevBuf();
+    const int err = resample(c, nrays, nfr, image, npix, nv, vtx, w, out);
+    if (err || c->rs_buf.held() > rl_ctx::Resample::KEEP) {
+        (void)hipStreamSynchronize(c->stream);
+        c->rs_buf.release();
     }
+    if (err) return err;
     float t = 0;
     (void)hipEventElapsedTime(&t, c->ev[1], c->ev[4]);
     for (int i = 0; i < 5; i++) c->t_ms[i] = 0.0;
