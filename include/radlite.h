@@ -133,8 +133,9 @@ int rl_trace_lines_forward_ex(rl_ctx *ctx, int nitems, const rl_item *items,
 /* rl_trace_lines_forward that allocates no device memory.  No counterpart
  * in the reference: it is for callers that cannot allocate (serving
  * loops, harnesses that forbid hipMalloc).  Every work buffer comes from
- * one fixed workspace of 256 MiB per GPU that the library holds for the
- * life of the process; items that need more (node records, 64 B per
+ * one fixed workspace of 256 MiB per GPU (and 416 MiB beside it, which the
+ * block records of whatever fits it never exceed) that the library holds for
+ * the life of the process; items that need more (node records, 64 B per
  * trajectory node and item, are most of it) are refused with 13.  flux_dev
  * (device memory, the layout of rl_trace_lines_forward's flux) receives
  * the spectra; image_dev (device memory, optional) the [nrays][nfr]

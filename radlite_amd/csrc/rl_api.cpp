@@ -233,7 +233,7 @@ struct rl_ctx {
     DevBuf d_gT, d_gTd, d_gvt, d_gla;
     // the library's fixed device workspace on this context's device (for
     // rl_trace_lines_forward_noalloc), or the lookup's failure
-    void *scratch = nullptr;
+    void *scratch = nullptr, *scratch_blocks = nullptr;
     std::string scratch_err;
     // stats
     double t_ms[5] = {0, 0, 0, 0, 0};
@@ -354,7 +354,7 @@ extern "C" int rl_create(rl_ctx **out, int device, int precision) {
         if (hipEventCreate(&e) != hipSuccess) { delete c; return RL_E_HIP; }
     // the fixed workspace's device address, once per device (the entry
     // points that do not use it work without it)
-    const hipError_t se = rl::scratch_attach(device, &c->scratch);
+    const hipError_t se = rl::scratch_attach(device, &c->scratch, &c->scratch_blocks);
     if (se != hipSuccess) c->scratch_err = hipGetErrorString(se);
     *out = c;
     return 0;
@@ -1738,18 +1738,18 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
     const size_t o_maser = carve((size_t)((nb + 1) / 2) * 8);
     const size_t o_counter = carve(8);
     const size_t o_items = carve((size_t)nb * sizeof(rl::ItemDev));
-    const size_t o_unit0 = carve((size_t)(nb + 1) * 16);
-    // the block records where they still fit; without them every segment is
-    // integrated
-    const size_t bbytes = (size_t)blk0 * sizeof(rl::BlkRec);
-    const bool with_blk = used + bbytes <= rl::SCRATCH_BYTES;
-    const size_t o_blk = with_blk ? carve(bbytes) : 0;
     if (used > rl::SCRATCH_BYTES)
         return fail(c, 13,
                     "rl_trace_lines_forward_noalloc: the items need %zu bytes of workspace, "
                     "more than its %zu (node records %lld x %zu B)", used, rl::SCRATCH_BYTES,
                     rec0, rsz);
+    // beside them (SCRATCH_BLOCKS is enough for whatever fits)
+    static_assert(sizeof(rl::BlkRec) == 24 && sizeof(rl::NodeLine) >= 16, "SCRATCH_BLOCKS");
+    used = 0;
+    const size_t o_unit0 = carve((size_t)(nb + 1) * 16);
+    const size_t o_blk = carve((size_t)blk0 * sizeof(rl::BlkRec));
     unsigned char *ws = static_cast<unsigned char *>(c->scratch);
+    unsigned char *wb = static_cast<unsigned char *>(c->scratch_blocks);
     for (auto &d : hi) {      // segment records relative to the record buffer
         d.hot_off -= (long long)(uintptr_t)(ws + o_rec);
         d.aux_off -= (long long)(uintptr_t)(ws + o_rec);
@@ -1760,7 +1760,7 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
     L.items = reinterpret_cast<const rl::ItemDev *>(ws + o_items);
     L.cells = reinterpret_cast<const CellRec *>(ws + o_cells);
     L.rec = ws + o_rec;
-    L.blk = with_blk ? ws + o_blk : nullptr;
+    L.blk = wb + o_blk;
     L.rinfo = reinterpret_cast<RayInfo *>(ws + o_rinfo);
     L.chan = reinterpret_cast<const double *>(ws + o_chan);
     L.image = image_dev ? image_dev : reinterpret_cast<double *>(ws + o_img);
@@ -1768,7 +1768,7 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
     L.flux = flux_dev;
     L.cmask = nullptr;
     L.d2 = (1.0 * 3.08572e18) * (1.0 * 3.08572e18);
-    L.unit0 = reinterpret_cast<const long long *>(ws + o_unit0);
+    L.unit0 = reinterpret_cast<const long long *>(wb + o_unit0);
     L.nunits[0] = u0[nb];
     L.nunits[1] = u0[2 * nb + 1];
     L.ovs = reinterpret_cast<unsigned long long *>(ws + o_ovs);
@@ -1780,7 +1780,7 @@ extern "C" int rl_trace_lines_forward_noalloc(rl_ctx *c, int nitems, const rl_it
                              c->stream));
     HIPCHK(c, hipMemcpyAsync(ws + o_items, hi.data(), (size_t)nb * sizeof(rl::ItemDev),
                              hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(ws + o_unit0, u0.data(), (size_t)(nb + 1) * 16,
+    HIPCHK(c, hipMemcpyAsync(wb + o_unit0, u0.data(), (size_t)(nb + 1) * 16,
                              hipMemcpyHostToDevice, c->stream));
     rl::launch_zero_u64(c->stream, L.ovs, nb);
     rl::launch_zero_u64(c->stream, reinterpret_cast<unsigned long long *>(L.maser), (nb + 1) / 2);

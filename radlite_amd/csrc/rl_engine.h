@@ -73,7 +73,7 @@ struct BatchLaunch {
     const ItemDev *items;      // device
     const CellRec *cells;      // [slots][ncell]
     void *rec;
-    void *blk;                 // block records, or null (every segment integrated)
+    void *blk;                 // block records
     RayInfo *rinfo;
     const double *chan;
     double *image, *partial, *flux;
@@ -93,12 +93,17 @@ void launch_segrec(hipStream_t st, long long nnodes, const long long *off, int n
                    const GeoNode *geo, const double *lw, SegHot *hot, SegAux *aux);
 
 // Fixed device workspace (rl_scratch.hip) of the allocation-free forward
-// entry point: SCRATCH_BYTES per GPU, resident while the process runs.
-// scratch_attach returns its device address on `device` (which must be
-// current), looked up once per device.
+// entry point: SCRATCH_BYTES per GPU, resident while the process runs, and beside
+// them SCRATCH_BLOCKS for the block records and the formal solution's unit lists
+// of whatever fits SCRATCH_BYTES: 24 B for 8 nodes and 24 B a ray, where those
+// hold at least 16 B a node and 16 B a ray (1.5 times), and 16 B an item, of which
+// they hold its ItemDev (an eighth).  scratch_attach returns their device
+// addresses on `device` (which must be current), taken once per device.
 constexpr size_t SCRATCH_BYTES = (size_t)256 << 20;
+constexpr size_t SCRATCH_BLOCKS = SCRATCH_BYTES / 8 * 13 + 4096;
+static_assert(sizeof(RayInfo) >= 16 && sizeof(ItemDev) >= 128, "SCRATCH_BLOCKS");
 constexpr int SCRATCH_MAX_DEVICES = 64;
-hipError_t scratch_attach(int device, void **out);
+hipError_t scratch_attach(int device, void **out, void **blocks);
 // cw: the channels of a unit's chunk (at most formal_chunk()); nblocks == 0:
 // one block per unit; > 0: persistent grid of nblocks blocks taking units from
 // the work counter

@@ -732,8 +732,8 @@ k_segrec(long long nnodes, const long long *__restrict__ off, int nrays,
 }
 
 // per item, one wave per ray: the scaled line records, the line-free
-// blocks (blk null: none) and the NONREDUNDANT window (telescope.F:4265-4270)
-// of the FP32 batched forward
+// blocks and the NONREDUNDANT window (telescope.F:4265-4270) of the FP32 batched
+// forward
 __device__ inline void nodes_ray_line(int ray, int lane, const long long *__restrict__ off,
                                       const GeoNode *__restrict__ geo,
                                       const CellRec *__restrict__ cells,
@@ -744,7 +744,7 @@ __device__ inline void nodes_ray_line(int ray, int lane, const long long *__rest
                                       int skip_mode, const LineConst &lc) {
     const long long b = off[ray];
     const int n = (int)(off[ray + 1] - b);
-    if (blk) blk += blk_of(b, ray);
+    blk += blk_of(b, ray);
     const double inv_nu0 = 1.0 / fabs(lc.nu0);
     double umin = 1.0e300, umax = -1.0e300;
     // the last lane's node of the previous 64, for this 64's first segment
@@ -771,7 +771,6 @@ __device__ inline void nodes_ray_line(int ray, int lane, const long long *__rest
                 umax = fmax(umax, gn.u);
             }
         }
-        if (!blk) continue;
         // the dust element of segment k from the node before it, as elem32
         // forms it with a line of 0
         const float u1 = (float)gn.u, lw1 = (float)v[CR_LW];
@@ -852,8 +851,9 @@ k_nodes_fast(int nrays, const long long *__restrict__ off, const GeoNode *__rest
 // ---------------------------------------------------------------------
 // formal solution
 // ---------------------------------------------------------------------
-// One lane's ray, block by block, each seen block from its own carry as
-// rl_walk.h takes it (blk null: every segment integrated).
+// One lane's ray, block by block: a seen block after a line-free one from its own
+// carry, as rl_walk.h takes every block (the same values), one after a seen one from
+// that one's (blk null: every segment integrated).
 template <typename T>
 __device__ inline T trace_one(const NodeRec<T> *__restrict__ rec,
                               const BlkRec *__restrict__ blk, int n, const LineK<T> &L,
@@ -915,8 +915,7 @@ __device__ inline double trace_dispatch<double>(const NodeRec<double> *rec,
     L.nu0 = lc.nu0; L.c_aa = lc.c_aa; L.hknu = lc.hknu;
     L.A = lc.A; L.Bud = lc.Bud; L.Bdu = lc.Bdu;
     L.dnu = dnu; L.uch = velo;
-    return trace_one<double>(rec + b, blk ? blk + blk_of(b, ray) : nullptr, n, L, I0, istar, sf,
-                             ovs, maser);
+    return trace_one<double>(rec + b, blk + blk_of(b, ray), n, L, I0, istar, sf, ovs, maser);
 }
 
 template <>
@@ -926,7 +925,7 @@ __device__ inline double trace_dispatch<float>(const NodeLine *rec,
                                                const LineConst &, double, double velo,
                                                const double *istar, double I0, float sf, int &ovs,
                                                int &maser) {
-    return trace_split(hot + b, aux + b, rec + b, blk ? blk + blk_of(b, ray) : nullptr, n,
+    return trace_split(hot + b, aux + b, rec + b, blk + blk_of(b, ray), n,
                        (float)velo, I0, istar, sf, ovs, maser);
 }
 
@@ -1182,12 +1181,12 @@ k_nodes_batch(const ItemDev *__restrict__ items, const CellRec *__restrict__ cel
     if constexpr (std::is_same<T, double>::value)
         nodes_ray_exact(ray, threadIdx.x, it.off, it.geo, cells,
                         reinterpret_cast<NodeRec<double> *>(rec_all) + it.rec0,
-                        blk_all ? reinterpret_cast<BlkRec *>(blk_all) + it.blk0 : nullptr,
+                        reinterpret_cast<BlkRec *>(blk_all) + it.blk0,
                         rinfo_all + it.rinfo0, it.nfr, velo, it.aks2, it.skip_mode, it.lc);
     else
         nodes_ray_line(ray, threadIdx.x, it.off, it.geo, cells,
                        reinterpret_cast<NodeLine *>(rec_all) + it.rec0,
-                       blk_all ? reinterpret_cast<BlkRec *>(blk_all) + it.blk0 : nullptr,
+                       reinterpret_cast<BlkRec *>(blk_all) + it.blk0,
                        rinfo_all + it.rinfo0, it.nfr, velo, it.aks2, it.skip_mode, it.lc);
 }
 
@@ -1203,7 +1202,7 @@ __device__ inline const R *seg_ptr(const void *rec_all, long long off) {
 }
 
 __device__ inline const BlkRec *blk_ptr(const void *blk_all, long long blk0) {
-    return blk_all ? reinterpret_cast<const BlkRec *>(blk_all) + blk0 : nullptr;
+    return reinterpret_cast<const BlkRec *>(blk_all) + blk0;
 }
 
 // The formal solution of many items (rl_walk.h): a block takes one ray and one
@@ -1256,8 +1255,7 @@ __device__ __forceinline__ void formal_unit(const FormalBatch &f, WalkLds<T, G> 
     const RayInfo ri = f.rinfo[it.rinfo0 + ray];
     const long long b = it.off[ray];
     const int n = ri.n, nb = n < 2 ? 0 : (n + BLK - 1) >> BLK_LOG;
-    const BlkRec *blk = f.blk ? reinterpret_cast<const BlkRec *>(f.blk) + it.blk0 + blk_of(b, ray)
-                              : nullptr;
+    const BlkRec *blk = blk_ptr(f.blk, it.blk0) + blk_of(b, ray);
     auto doit = [&](int c) {
         if (it.skip_mode != 0 || ray == 0 || c == 0 || c == ri.cont) return true;
         const double v = velo[c];

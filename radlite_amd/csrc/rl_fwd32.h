@@ -272,7 +272,8 @@ __device__ __forceinline__ void segment32(Acc32<AFF> &x, const SegHot *hot, cons
 
 // charintline (telescope.F:3889-4312) on split records, one lane: one channel
 // (uch = dnu/nu0) of one ray of n nodes from the outer boundary intensity I0,
-// block by block, each seen block from its own carry as rl_walk.h takes it.
+// block by block: a seen block after a line-free one from its own carry, as
+// rl_walk.h takes every block, one after a seen one from that one's.
 __device__ inline double trace_split(const SegHot *__restrict__ hot, const SegAux *__restrict__ aux,
                                      const NodeLine *__restrict__ line,
                                      const BlkRec *__restrict__ blk, int n, float uch, double I0,
@@ -282,14 +283,12 @@ __device__ inline double trace_split(const SegHot *__restrict__ hot, const SegAu
     Car32 c;
     bool ovf = false, fresh = true;
     for (int k0 = 0; k0 < n; k0 += BLK) {
-        if (blk) {
-            const BlkRec r = blk[k0 >> BLK_LOG];
-            if (blk_free(r, uch)) {
-                x.map(r.A, r.B);
-                ovf = ovf || blk_overshoots(r) != 0;
-                fresh = true;
-                continue;
-            }
+        const BlkRec r = blk[k0 >> BLK_LOG];
+        if (blk_free(r, uch)) {
+            x.map(r.A, r.B);
+            ovf = ovf || blk_overshoots(r) != 0;
+            fresh = true;
+            continue;
         }
         for (int k = max(k0, 1); k < min(n, k0 + BLK); k++) {
             if (fresh) {

@@ -142,12 +142,11 @@ __device__ __forceinline__ void walk(WalkLds<T, G> &S, const BlkRec *__restrict_
         int cl = ch.c0, cnt = 0, nov = 0;
         double bA = 1.0, bB = 0.0;
         if (lane < m) {
-            float lo = -INFINITY, hi = INFINITY;
-            if (blk) {
-                const BlkRec *r = blk + jw + lane;
-                lo = r->lo; hi = r->hi; bA = r->A; bB = r->B;
-                nov = __float_as_int(lo) & (2 * BLK - 1);
-            }
+            const BlkRec *r = blk + jw + lane;
+            const float lo = r->lo, hi = r->hi;
+            bA = r->A;
+            bB = r->B;
+            nov = __float_as_int(lo) & (2 * BLK - 1);
             if (!(lo > hi))          // (-inf with an overshoot count is NaN)
                 channels_in<T>(ch.velo, ch.c0, ch.c1, v0, inv, lo, hi, cl, cnt);
         }
