@@ -82,8 +82,10 @@ __device__ inline void adj_bounds(int lane, const FastRecT<T> *__restrict__ rec,
             const float z = (sqrtf(t) + 0.01f) * scale / ia;
             lo = fminf(lo, (float)fmin(p.u, r.u) - z);
             hi = fmaxf(hi, (float)fmax(p.u, r.u) + z);
-            // never free: the star's intensity, or a line that is no number
-            if (((int)r.flag & (NF_BLEND | NF_STAR)) || !(most < INFINITY) || !(z < INFINITY)) {
+            // never free: the star's intensity, or a line, a velocity or a width that
+            // is no number
+            if (((int)r.flag & (NF_BLEND | NF_STAR)) || !(most < INFINITY) || !(z < INFINITY) ||
+                !blk_sane(p.u, r.u, (float)r.inv_aa, (float)(two ? p.inv_aa : r.inv_aa))) {
                 lo = -INFINITY;
                 hi = INFINITY;
             }

@@ -41,6 +41,12 @@ __device__ inline float blk_zcut(float M, bool inverted) {
     return sqrtf(t) + 0.01f;                        // the bounds' own rounding
 }
 
+// whether a segment's velocities and the widths of the two segments at its start are
+// such that bounds can be given at all (a negative width has them the wrong way round)
+template <typename T> __device__ inline bool blk_sane(T u0, T u1, float w0, float w1) {
+    return fabs(u0) + fabs(u1) < (T)INFINITY && w0 > 0.0f && w1 > 0.0f;
+}
+
 // |x| / |d| as a ratio of line to dust: 0 without line, inf without dust
 template <typename T>
 __device__ inline float blk_ratio(T x, T d) {

@@ -610,8 +610,12 @@ __device__ inline void nodes_ray_exact(int ray, int lane, const long long *__res
             lo = fminf((float)u_p, (float)gn.u) - z;
             hi = fmaxf((float)u_p, (float)gn.u) + z;
             // never free: the star's intensity, which follows the channel, and
-            // a line that is not a number anywhere if it is not one here
-            if ((fl & (NF_BLEND | NF_STAR)) || !fin_p || !fin) { lo = -INFINITY; hi = INFINITY; }
+            // a line, a width or a velocity that is not a number anywhere if it is
+            // not one here (a width of 0: 0 times infinity)
+            if ((fl & (NF_BLEND | NF_STAR)) || !fin_p || !fin || !blk_sane(u_p, gn.u, wl, wl_p)) {
+                lo = -INFINITY;
+                hi = INFINITY;
+            }
         }
         blk_store(lane, k, n, A, B, lo, hi, ovf, blk);
         jd_c = __shfl(v[CR_JD], 63);
@@ -812,8 +816,9 @@ __device__ inline void nodes_ray_line(int ray, int lane, const long long *__rest
             lo = fminf(u_p, u1) - z;
             hi = fmaxf(u_p, u1) + z;
             // never free: the star's intensity, which follows the channel, and
-            // a line that is not a number anywhere if it is not one here
-            if ((fl & (NF_BLEND | NF_STAR)) || !(most < INFINITY)) {
+            // a line, a width or a velocity that is not a number anywhere if it is
+            // not one here
+            if ((fl & (NF_BLEND | NF_STAR)) || !(most < INFINITY) || !blk_sane(u_p, u1, wl, wl_p)) {
                 lo = -INFINITY;
                 hi = INFINITY;
             }

@@ -266,8 +266,9 @@ __device__ __forceinline__ void segment32(Acc32<AFF> &x, const SegHot *hot, cons
     elem_map32(hds, e, q.jcl * h.ng, dcn, sig, nl_adh(q.sig), q.jdh, c, ovf, e0, b);
     x.step(e0, b);
     // maser flag (telescope.F:4295-4297): line alpha * ds < -0.01 at the end;
-    // the line coefficient is negative only where the populations are inverted
-    if (q.dcl < 0.0f && sig * (dcn * e) * ds < -0.01f) maser = 1;
+    // the line coefficient is negative only where the populations are inverted (or
+    // the width negative)
+    if (dcn < 0.0f && sig * (dcn * e) * ds < -0.01f) maser = 1;
 }
 
 // charintline (telescope.F:3889-4312) on split records, one lane: one channel
