@@ -23,10 +23,9 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-FP32_PEAK_TFLOPS = 157.3
-FP64_PEAK_TFLOPS = 78.6
-
-
+# FP32 wave64 instructions issued per second at most: 2 per CU and cycle (157.3
+# TFLOP/s as fused multiply-adds), 256 CUs at 2.4 GHz
+VALU_ISSUE_PEAK = 2 * 256 * 2.4e9
 
 
 def measured_traffic(precision, kernel):
@@ -45,17 +44,18 @@ def measured_traffic(precision, kernel):
     return None
 
 
-def measured_valu_issue(precision):
-    """VALU wave-instructions per CU-cycle of the formal kernel over the FP32
-    wave64 issue peak (2 per CU-cycle), from the committed rocprofv3 SQ
-    counter summary, or None."""
+def measured_valu(precision, kernel):
+    """(VALU wave instructions per launch of the formal kernel, the share of
+    their lanes that are active) from the committed rocprofv3 SQ counter
+    summary, or (None, None)."""
     path = os.path.join(ROOT, "profiles", f"sq_counters_c2_{precision}_forward.txt")
-    if not os.path.exists(path):
-        return None
-    for line in open(path):
-        if "k_formal VALU wave-instructions per CU-cycle" in line:
-            return float(line.split("=")[1].split()[0]) / 2.0
-    return None
+    got = {}
+    if os.path.exists(path):
+        for line in open(path):
+            f = line.split()
+            if len(f) == 4 and f[1] == kernel and f[2] == precision:
+                got[f[0]] = float(f[3])
+    return got.get("valu_instructions_per_launch"), got.get("valu_lanes_active")
 
 
 def bench_adjoint(args):
@@ -561,13 +561,12 @@ def main():
     bytes_per_rc = (32.0 if args.precision == "fp32" else 64.0) * nseg
     nbatch, tile_cw, tile_blocks = rt.batch_info()
     formal_s = float(np.mean(t_formal)) / 1e3     # per step: every batch's formal launch
-    # per launch (one inclination): algorithmic bytes / mean launch duration
-    flops_per_rc = 40.0 * nseg
-    peak_tf = FP32_PEAK_TFLOPS if args.precision == "fp32" else FP64_PEAK_TFLOPS
-    achieved_tf = flops_per_rc * nominal / formal_s / 1e12
     kname = "k_formal"
     traffic = measured_traffic(args.precision, kname) if args.workload == "c2" else None
     hbm_gbs = traffic * nbatch / formal_s / 1e9 if traffic is not None else None
+    insts, lanes = (measured_valu(args.precision, kname)
+                    if args.workload == "c2" and args.skip == "none" else (None, None))
+    issue = insts * nbatch / formal_s if insts is not None else None
 
     out = {
         "metric": "ray*channel integrations/s (forward)",
@@ -594,29 +593,30 @@ def main():
                                            "t_flux_ms", "t_total_ms")},
         "roofline": {
             # the formal kernel is bound by VALU issue and latency, not by HBM:
-            # algorithmic FP32 operations (40 per segment per ray*channel) per
-            # second of the kernel against the MI355X FP32 vector peak
+            # VALU wave instructions (counted per launch by the SQ, committed
+            # summary) over the kernel's time in this run, against the issue peak;
+            # the share of their lanes with work beside it
             "bound": "valu",
-            "achieved": achieved_tf,
-            "peak": peak_tf,
-            "unit": "TFLOP/s",
-            "frac": achieved_tf / peak_tf,
+            "achieved": issue / 1e12 if issue is not None else None,
+            "peak": VALU_ISSUE_PEAK / 1e12,
+            "unit": "T wave64 instructions/s",
+            "frac": issue / VALU_ISSUE_PEAK if issue is not None else None,
+            "lanes_active": lanes,
+            # not a rate of work done: what 40 operations for every segment and
+            # channel would come to, of which the line-free blocks leave most out
+            "nominal_equivalent_tflops": 40.0 * nseg * nominal / formal_s / 1e12,
             "traffic": traffic,
             "kernel": kname,
             "kernel_ms": formal_s * 1e3 / nbatch,        # mean per launch (one batch)
             "launches_per_step": nbatch,
             "items_per_launch": len(items) // nbatch,
-            "flops_per_ray_channel": flops_per_rc,
             "tile_cw": tile_cw, "persistent_blocks": tile_blocks,
-            # HBM, reported apart: the streaming formulation's bytes (28 B per
-            # segment per ray*channel) and the counter-measured bytes per
-            # launch over the kernel time, against the 8 TB/s peak
+            # HBM, reported apart: the bytes of the records if every ray*channel
+            # read them for itself, and the counter-measured bytes per launch over
+            # the kernel time, against the 8 TB/s peak
             "hbm_algorithmic_bytes_per_ray_channel": bytes_per_rc,
             "hbm_measured_gbs": hbm_gbs,
             "hbm_measured_frac": (hbm_gbs / HBM_PEAK_GBS) if hbm_gbs is not None else None,
-            # measured VALU issue rate over the wave64 FP32 issue peak (SQ counters)
-            "valu_issue_frac_measured": (measured_valu_issue(args.precision)
-                                         if args.workload == "c2" else None),
         },
     }
     rt.close()
