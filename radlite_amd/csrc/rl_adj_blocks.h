@@ -17,7 +17,8 @@
 // sub-grid points of the few channels at resonance.
 // 200 x 100 disk, 100 channels, FP32: reverse sweep 13.1 -> 6.9 ms (pairs 5.7,
 // lambda 1.0, bounds 0.2), a fit's step 20.2 -> 11.5 ms with the forward by maps;
-// FP64 9.3 -> 4.6 ms with 32 angles; 40 x 24 disk, 24 channels, FP64, 1.6 -> 0.96.
+// FP64, 32 angles, a step 11.6 -> 5.8 ms; 40 x 24 disk, 24 channels, FP64, a step
+// 1.78 -> 0.90.  Half of the lanes of k_adj_pairs have work (SQ counters).
 // Held to 128 registers it spills, with more than 168 too few waves are left.
 #pragma once
 #include "rl_adjoint.h"

@@ -4,8 +4,10 @@
 // physics in the reference's own evaluation order; the FP64
 // instantiation is the parity mode, the FP32 instantiation the
 // performance mode.  The translation unit is compiled with
-// -ffp-contract=off so that FP64 arithmetic rounds exactly as the
-// reference's (x86-64, no FMA) evaluation does.
+// -ffp-contract=off so that FP64 arithmetic rounds each element exactly as the
+// reference's (x86-64, no FMA) evaluation does.  Where elements are composed to
+// maps of the intensity (rl_blocks.h, rl_walk.h) the sums along a ray associate
+// otherwise: 1e-15 of the intensity.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

@@ -22,8 +22,9 @@
 // What bounds it: instruction issue, then the latency of a batch's steps.
 // Lanes that held one (ray, channel) each and met at every block that one of 16
 // channels saw had work in 38% of their instructions, and a ray of many blocks
-// was one serial chain; packed pairs fill 68%, and their chains are a block
-// long.  One launch, 400 x 200 disk, two inclinations, FP32: 19.3 -> 16.1 ms;
+// was one serial chain; packed pairs fill 65% (SQ counters, 400 x 200 disk, 200
+// channels, FP32; 0.92 VALU instructions a cycle and compute unit), and their chains
+// are a block long.  One launch, 400 x 200 disk, two inclinations, FP32: 19.3 -> 16.1 ms;
 // 200 x 100 disk, FP64: 4.8 -> 3.1 ms; 100 x 60 disk, FP64: 0.96 -> 0.40 ms;
 // 97 x 61 disk, FP32: 0.62 -> 0.27 ms.  (A wave per eighth of a ray, for
 // launches of few rays: 14 of 64 lanes with work, 1.22 ms for the 100 x 60
