@@ -160,9 +160,10 @@ __device__ __forceinline__ void walk(WalkLds<T, G> &S, const BlkRec *__restrict_
         const bool some = cnt > 0, overs = __any(nov != 0);
         // the blocks with pairs that are not in LDS yet, and of these the first
         // `ahead` whose nodes are in registers (slots by rank); none where the
-        // pairs of BATCH_BLOCKS blocks do not fill a batch
+        // pairs of BATCH_BLOCKS blocks do not fill a batch, and there are more
         unsigned long long rest = __ballot(some);
-        const bool sparse = FEW && total * BATCH_BLOCKS < 64 * __popcll(rest);
+        const int seen = __popcll(rest);
+        const bool sparse = FEW && seen > BATCH_BLOCKS && total * BATCH_BLOCKS < 64 * seen;
         if (sparse) rest = 0;
         const int rank = __popcll(rest & (upto >> 1));
         int staged = 0, ahead = 0;
