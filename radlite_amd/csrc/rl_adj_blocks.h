@@ -62,15 +62,12 @@ __device__ inline void adj_bounds(int lane, const FastRecT<T> *__restrict__ rec,
         const int k1 = min(j * BLK + BLK, n);
         int k = max(1, j * BLK);
         FastRecT<T> p = rec[k - 1];
-        double A = 1.0, B = 0.0;
+        RayMap<T> x;
         for (; k < k1; k++) {
             const FastRecT<T> r = rec[k];
             FastCarryT<T> c;
-            T q = T(0);
             int ovs = 0;
-            elem_fast<T>(L, q, r.ds, dust_of<T>(p), dust_of<T>(r), r.inv_aa, r.norm, c, ovs);
-            B = B * (double)c.P + (double)q;
-            A = A * (double)c.P;
+            elem_fast<T>(L, x, r.ds, dust_of<T>(p), dust_of<T>(r), r.inv_aa, r.norm, c, ovs);
             // the widest and narrowest profile at node k-1
             const bool two = k > 1;
             const float ia = (float)(two && p.inv_aa < r.inv_aa ? p.inv_aa : r.inv_aa);
@@ -93,7 +90,7 @@ __device__ inline void adj_bounds(int lane, const FastRecT<T> *__restrict__ rec,
             p = r;
         }
         out[j] = make_float2(lo, hi);
-        dust[j] = make_double2(A, B);
+        dust[j] = make_double2(x.P, x.B);
     }
 }
 
@@ -108,7 +105,6 @@ __device__ inline void block_carry(const FastRecT<T> *__restrict__ rec, int j,
                                    const FastLineT<T> &L, FastCarryT<T> &c) {
     const FastRecT<T> a = rec[max(j * BLK - 1, 0)];
     c.u0 = a.u;
-    c.P = T(1);
     c.init = 1;
     if (j > 0) {
         T jl0, al0, z_, phi_;
@@ -134,14 +130,14 @@ __device__ inline void block_dust_rev(const FastRecT<T> *__restrict__ rec, int j
     for (int k = k0; k < k1; k++) {
         const FastRecT<T> r = rec[k];
         FastCarryT<T> c;
-        T q = T(0);
+        RayMap<T> x;
         int ovs = 0;
         pa[k - k0] = A;
         pb[k - k0] = B;
-        elem_fast<T>(L, q, r.ds, dust_of<T>(rec[k - 1]), dust_of<T>(r), r.inv_aa, r.norm, c, ovs);
-        px[k - k0] = (double)c.P;
-        B = B * (double)c.P + (double)q;
-        A = A * (double)c.P;
+        elem_fast<T>(L, x, r.ds, dust_of<T>(rec[k - 1]), dust_of<T>(r), r.inv_aa, r.norm, c, ovs);
+        px[k - k0] = x.P;
+        B = B * x.P + x.B;
+        A = A * x.P;
     }
     double suf = 1.0;
     PGrad<T> cur, prv;
@@ -324,20 +320,20 @@ __device__ __forceinline__ void adj_ray_maps(const AdjRay<T> &y, T *__restrict__
             const T ist = (T)y.istar[ch];
             FastCarryT<T> c;
             block_carry<T>(y.rec, j, L, c);
-            T B = T(0);
+            RayMap<T> x;
             int ovs = 0;
 #pragma unroll 1
             for (int i = 0; i < BLK; i++) {
                 const int k = kb + i;
                 if (k >= 1 && k < y.n) {
                     const FastRecT<T> r = y.rec[k];
-                    segment_fast<T>(r, y.rec + k - 1, point_of<T>(r), L, B, ist, y.sf, c, ovs);
+                    segment_fast<T>(r, y.rec + k - 1, point_of<T>(r), L, x, ist, y.sf, c, ovs);
                 }
             }
             if (p0 + lane < total) {
                 const long long slot = (long long)j * y.nfr + ch;
-                outP[slot] = c.P;
-                outB[slot] = B;
+                outP[slot] = (T)x.P;
+                outB[slot] = (T)x.B;
             }
         }
     }

@@ -383,8 +383,37 @@ template <typename T> struct FastCarryT {
     T sa0 = T(0), sj0 = T(0), ah0 = T(0), S0 = T(0), al0 = T(0);
     int init = 1;
     T u0 = T(0), tau = T(0), tau_c = T(0);
-    T P = T(1);                 // dI/d(I at the start): the product of the elements' factors
 };
+
+// What the elements of a lane act on: the intensity, a T, or the map of the part
+// of the ray passed, I -> P I + B.  The map in double (the elements' values in T):
+// it is rounded to T once a block, and a spectrum by maps is no further off than
+// one by elements.  e0 = 1 - xp: thin elements keep their digits in single precision.
+template <typename T> struct RayMap { double B = 0.0, P = 1.0; };
+template <typename T> __device__ inline void ray_step(T &I, T xp, T, T q) {
+    I = FOps<T>::fma(I, xp, q);
+}
+__device__ inline void ray_step(RayMap<double> &x, double xp, double, double q) {
+    x.B = FOps<double>::fma(x.B, xp, q);
+    x.P = x.P * xp;
+}
+__device__ inline void ray_step(RayMap<float> &x, float, float e0, float q) {
+    x.B = x.B + __builtin_fma(-x.B, (double)e0, (double)q);
+    x.P = __builtin_fma(-x.P, (double)e0, x.P);
+}
+// the central beam's share of the star, and the star
+template <typename T> __device__ inline void ray_blend(T &I, T sf, T istar) {
+    I = (T(1) - sf) * I + sf * istar;
+}
+template <typename T> __device__ inline void ray_blend(RayMap<T> &x, T sf, T istar) {
+    x.B = (double)(T(1) - sf) * x.B + (double)(sf * istar);
+    x.P = x.P * (double)(T(1) - sf);
+}
+template <typename T> __device__ inline void ray_star(T &I, T istar) { I = istar; }
+template <typename T> __device__ inline void ray_star(RayMap<T> &x, T istar) {
+    x.B = (double)istar;
+    x.P = 0.0;
+}
 
 // the carry of a start point p0 with line values jl0, al0 (/ sig)
 template <typename T>
@@ -399,9 +428,9 @@ __device__ inline void carry_start(const FPtT<T> &p0, T jl0, T al0, FastCarryT<T
 
 // integrate_element_linedust (line.F:4515-4624) on scaled values.  The
 // start point is taken from the carry; start() supplies it (an FPtT) only
-// when init is set.
-template <typename T, typename Start>
-__device__ inline void elem_core(const FastLineT<T> &L, T &I, T ds, const Start &start,
+// when init is set.  I: a T or a RayMap<T>.
+template <typename T, typename X, typename Start>
+__device__ inline void elem_core(const FastLineT<T> &L, X &I, T ds, const Start &start,
                                  const FPtT<T> &p1, T inv_aa, T norm, FastCarryT<T> &c,
                                  int &ovs) {
     using O = FOps<T>;
@@ -425,8 +454,8 @@ __device__ inline void elem_core(const FastLineT<T> &L, T &I, T ds, const Start 
         c.tau_c = (t - c.tau) - y;
         c.tau = t;
     }
-    T wa, wb, xp, ra;
-    qdr_weights_f<T>(dtau, wa, wb, xp, ra);
+    T wa, wb, xp, ra, e0;
+    qdr_weights_f<T>(dtau, wa, wb, xp, ra, e0);
     // source functions (transfer.F:1528-1541) from the scaled values
     T q1 = ah1 > T(0) ? FOps<T>::sdiv(jh1, ah1) : T(0);
     T q0 = c.S0;
@@ -435,8 +464,7 @@ __device__ inline void elem_core(const FastLineT<T> &L, T &I, T ds, const Start 
     T q = dtau > T(1e-9f) ? O::fma(wa, s1, wb * s2) : theomax;
     ovs += q > T(2) * theomax;
     q = O::fmn(q, theomax);
-    I = O::fma(I, xp, q);
-    c.P = c.P * xp;
+    ray_step(I, xp, e0, q);
     c.sa0 = p1.sig * ah1;
     c.sj0 = p1.sig * jh1;
     c.ah0 = ah1;
@@ -445,8 +473,8 @@ __device__ inline void elem_core(const FastLineT<T> &L, T &I, T ds, const Start 
     c.init = 0;
 }
 
-template <typename T>
-__device__ inline void elem_fast(const FastLineT<T> &L, T &I, T ds, const FPtT<T> &p0,
+template <typename T, typename X>
+__device__ inline void elem_fast(const FastLineT<T> &L, X &I, T ds, const FPtT<T> &p0,
                                  const FPtT<T> &p1, T inv_aa, T norm, FastCarryT<T> &c,
                                  int &ovs) {
     elem_core<T>(L, I, ds, [&]() { return p0; }, p1, inv_aa, norm, c, ovs);
@@ -512,9 +540,9 @@ __device__ inline FPtT<T> point_of(const FastRecT<T> &a) {
 // one segment (nodes k-1 -> k) of charintline on FastRecT data; prev is
 // the record of node k-1, read only for a flagged or sub-gridded segment
 // (the carry holds what a whole segment needs of its start)
-template <typename T>
+template <typename T, typename X>
 __device__ inline void segment_fast(const FastRecT<T> &b, const FastRecT<T> *prev,
-                                    const FPtT<T> &p1, const FastLineT<T> &L, T &I, T istar,
+                                    const FPtT<T> &p1, const FastLineT<T> &L, X &I, T istar,
                                     T starfract, FastCarryT<T> &c, int &ovs) {
     T ds = b.ds;
     const int fl = (int)b.flag;
@@ -523,11 +551,10 @@ __device__ inline void segment_fast(const FastRecT<T> &b, const FastRecT<T> *pre
     if (__builtin_amdgcn_ballot_w64(fl != 0)) {
         if (fl & NF_RESET) { ds = T(0); c.init = 1; }
         if (fl & NF_BLEND) {
-            I = (T(1) - starfract) * I + starfract * istar;
-            c.P = c.P * (T(1) - starfract);
+            ray_blend(I, starfract, istar);
             c.init = 1;
         }
-        if (fl & NF_STAR) { I = istar; c.P = T(0); c.init = 1; }
+        if (fl & NF_STAR) { ray_star(I, istar); c.init = 1; }
     }
     // one call for the last (or only) element of every segment: a segment
     // integrated whole has sa = 0 and ds - 0 = ds exactly, and its start
